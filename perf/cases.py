@@ -1,0 +1,302 @@
+"""The attention calls whose speed this repository answers for: prompt and decode steps of a serving loop, long contexts,
+speculative decoding, the int8 latent cache, and plain dense batches, each through the public functions of
+`flash_attn_npu` and `flash_attn_npu_3`.
+
+A case is a dict of sizes and options.  Sequence lengths are spread evenly at random over [min_len, max_len]; the case's
+`shape` number fixes them, so that a case is the same work whatever the seed of its values is.  Values are N(0, 1), as in
+the tests and in bench.py; pages are dealt in random order; the block table is as wide as the longest sequence needs."""
+import math
+import os
+import random
+import sys
+
+import torch
+
+_PACKAGE = os.path.join(os.getcwd(), "flash-attention-npu_amd")
+if _PACKAGE not in sys.path:
+    sys.path.insert(0, _PACKAGE)
+
+from flash_attn_npu import flash_attn_func, flash_attn_varlen_func, flash_attn_with_kvcache  # noqa: E402
+from flash_attn_npu_3 import flash_attn_with_kvcache as flash_attn_with_kvcache_3  # noqa: E402
+
+DEVICE = "cuda:0"
+DTYPES = {"bf16": torch.bfloat16, "fp16": torch.float16}
+LATENT, LATENT_V = 576, 512     # columns of a latent cache row, and those of it that are values
+
+
+def _cache_case(name, batch, q_heads, kv_heads, dim, min_len, max_len, new=1, append=False, rotary="none", window=-1, softcap=0.0,
+                page=256, dtype="bf16", shape=1):
+    """flash_attn_with_kvcache over a paged cache: `new` query tokens per sequence behind min_len .. max_len cached keys
+    (appended by the call, or there already), causal."""
+    return {"name": name, "kind": "cache", "batch": batch, "q_heads": q_heads, "kv_heads": kv_heads, "dim": dim, "min_len": min_len,
+            "max_len": max_len, "new": new, "append": append, "rotary": rotary, "window": window, "softcap": softcap, "page": page,
+            "dtype": dtype, "shape": shape}
+
+
+def _latent_case(name, batch, q_heads, min_len, max_len, new=1, append=False, page=256, dtype="bf16", shape=1):
+    """flash_attn_with_kvcache over an int8 latent cache (one latent head, per-token scales), causal."""
+    return {"name": name, "kind": "latent", "batch": batch, "q_heads": q_heads, "min_len": min_len, "max_len": max_len, "new": new,
+            "append": append, "page": page, "dtype": dtype, "shape": shape}
+
+
+def _packed_case(name, batch, q_heads, kv_heads, dim, min_len, max_len, total=0, causal=True, window=-1, softcap=0.0, dtype="bf16", shape=1):
+    """flash_attn_varlen_func over prompts packed back to back (total > 0: the lengths are scaled to that sum)."""
+    return {"name": name, "kind": "packed", "batch": batch, "q_heads": q_heads, "kv_heads": kv_heads, "dim": dim, "min_len": min_len,
+            "max_len": max_len, "total": total, "causal": causal, "window": window, "softcap": softcap, "dtype": dtype, "shape": shape}
+
+
+def _dense_case(name, batch, q_heads, kv_heads, dim, seqlen, causal=False, dtype="fp16"):
+    """flash_attn_func over a batch of equally long sequences."""
+    return {"name": name, "kind": "dense", "batch": batch, "q_heads": q_heads, "kv_heads": kv_heads, "dim": dim, "seqlen": seqlen,
+            "causal": causal, "dtype": dtype}
+
+
+def _step_case(name, rows, q_heads, kv_heads, dim, min_len, max_len, chunk, chunk_len, page=256, dtype="bf16", shape=1):
+    """One token-major step of a serving loop over a paged cache: `rows` sequences that decode one token each behind
+    min_len .. max_len keys, and one prompt chunk of `chunk` tokens that ends a context of chunk_len keys."""
+    return {"name": name, "kind": "step", "rows": rows, "q_heads": q_heads, "kv_heads": kv_heads, "dim": dim, "min_len": min_len,
+            "max_len": max_len, "chunk": chunk, "chunk_len": chunk_len, "page": page, "dtype": dtype, "shape": shape}
+
+
+def listed():
+    return [
+        # one user, the start of a conversation: the smallest call, all latency and launches
+        _cache_case("decode_one", 1, 32, 8, 128, 700, 700, append=True, rotary="half"),
+        # a serving batch of an 8-billion-parameter GQA decoder: bench.py's headline workload
+        _cache_case("decode_many", 64, 32, 8, 128, 1024, 8191, append=True, rotary="half"),
+        # a small decoder without grouped heads, short ragged contexts, small pages
+        _cache_case("decode_mha64", 40, 16, 16, 64, 33, 900, append=True, rotary="interleaved", page=64, dtype="fp16"),
+        # few very long contexts: every sequence is cut over the whole device
+        _cache_case("decode_long", 4, 64, 8, 128, 131072, 131072),
+        # the same cache under a sliding window: only the last 4096 keys of each sequence are visible
+        _cache_case("decode_window", 4, 64, 8, 128, 131072, 131072, window=4095),
+        # speculative decoding: five tokens per sequence are appended and verified at once
+        _cache_case("decode_draft", 24, 32, 8, 128, 200, 6000, new=5, append=True, rotary="half"),
+        # latent attention over an int8 cache, a full batch (bench.py's latent workload) ...
+        _latent_case("latent_many", 32, 128, 2048, 16384),
+        # ... and a few users, each step quantising and appending its token
+        _latent_case("latent_few", 3, 128, 400, 5000, append=True),
+        # prompts of a serving batch, packed: bench.py's prefill workload
+        _packed_case("prompts", 16, 32, 8, 128, 512, 4096, total=32768),
+        # many short prompts of odd lengths under an odd number of heads per group
+        _packed_case("prompts_short", 80, 28, 4, 128, 3, 350),
+        # an encoder or image transformer: dense, bidirectional, half precision
+        _dense_case("dense_encoder", 8, 16, 16, 64, 2050),
+        # chunked prefill: one prompt chunk among decoding sequences
+        _step_case("serving_step", 63, 32, 8, 128, 1024, 8191, 1024, 16384),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+MOST_BYTES, MOST_FLOPS = 2.0e9, 6.0e11    # a drawn case costs no more than the largest listed one,
+MOST_KEY_BYTES = 4.0e9                    # and its pool no more memory (a window sees little of it)
+
+
+def _affordable(case):
+    w = work(case)
+    row = LATENT if case["kind"] == "latent" else 4 * case["kv_heads"] * case["dim"]
+    return w["bytes"] <= MOST_BYTES and w["flops"] <= MOST_FLOPS and sum(keys for _, keys in _blocks(case)) * row <= MOST_KEY_BYTES
+
+
+def _draw_once(rng):
+    kind = rng.choice(["cache", "cache", "cache", "chunk", "latent", "packed", "packed", "dense", "step"])
+    shape = rng.randrange(1 << 20)
+    dtype = rng.choice(["bf16", "bf16", "fp16"])
+    q_heads, kv_heads = rng.choice([(32, 8), (32, 8), (64, 8), (28, 4), (16, 16), (32, 32), (8, 1), (32, 4), (12, 2), (40, 8)])
+    dim = rng.choice([128, 128, 128, 64, 64, 256, 96, 80])
+    page = rng.choice([32, 64, 128, 256, 256])
+    longest = _log_int(rng, 40, 65536)
+    shortest = max(1, int(longest * rng.choice([1.0, 0.5, 0.1])))
+    if kind in ("cache", "chunk"):
+        new = rng.choice([1, 1, 1, 2, 3, 4, 6, 8]) if kind == "cache" else _log_int(rng, 16, 1024)
+        append = rng.random() < 0.6
+        return _cache_case("", _log_int(rng, 1, 200 if kind == "cache" else 16), q_heads, kv_heads, dim, shortest, longest, new, append,
+                           rng.choice(["none", "half", "interleaved"]) if append and dim in (64, 128) else "none",
+                           rng.choice([-1, -1, -1, 1023, 4095]), rng.choice([0.0, 0.0, 0.0, 0.0, 30.0]), page, dtype, shape)
+    if kind == "latent":
+        return _latent_case("", _log_int(rng, 1, 64), rng.choice([128, 128, 64, 16]), shortest, min(longest, 32768), rng.choice([1, 1, 1, 2]),
+                            rng.random() < 0.5, page, dtype, shape)
+    if kind == "packed":
+        return _packed_case("", _log_int(rng, 1, 64), q_heads, kv_heads, dim, shortest, min(longest, 16384), 0, rng.random() < 0.8,
+                            rng.choice([-1, -1, -1, 1023]), rng.choice([0.0, 0.0, 0.0, 0.0, 30.0]), dtype, shape)
+    if kind == "dense":
+        return _dense_case("", _log_int(rng, 1, 32), q_heads, kv_heads, dim, min(longest, 16384), rng.random() < 0.5, dtype)
+    chunk = _log_int(rng, 32, 2048)
+    return _step_case("", _log_int(rng, 2, 100), q_heads, kv_heads, dim, shortest, longest, chunk, chunk + _log_int(rng, 1, 32768), page, dtype, shape)
+
+
+def draw(rng):
+    """One more case: head counts, head dimensions, page sizes and types as the tests use them, batch and lengths spread over
+    their ranges on a logarithmic scale."""
+    while True:
+        case = _draw_once(rng)
+        if "min_len" in case:
+            case["min_len"] = min(case["min_len"], case["max_len"])     # (some kinds take shorter sequences than were drawn)
+        if _affordable(case):
+            del case["name"]
+            return case
+
+
+def _lengths(case):
+    """Cached keys of each sequence (cache, latent, step), or its tokens (packed, dense)."""
+    if case["kind"] == "dense":
+        return [case["seqlen"]] * case["batch"]
+    rng = random.Random(case["shape"])
+    lens = [rng.randint(case["min_len"], case["max_len"]) for _ in range(case["rows"] if case["kind"] == "step" else case["batch"])]
+    if case.get("total"):
+        whole = sum(lens)
+        ends = [round(sum(lens[:i + 1]) * case["total"] / whole) for i in range(len(lens))]
+        lens = [e - b for b, e in zip([0] + ends, ends)]
+    return lens
+
+
+def _blocks(case):
+    """(query tokens, keys they are aligned to the end of) of each sequence."""
+    lens = _lengths(case)
+    if case["kind"] in ("packed", "dense"):
+        return [(n, n) for n in lens]
+    if case["kind"] == "step":
+        return [(1, n) for n in lens] + [(case["chunk"], case["chunk_len"])]
+    return [(case["new"], n + case["new"] * case["append"]) for n in lens]
+
+
+def _paged(lens, page, generator):
+    """Block table (sequence, page) over a pool dealt in random order, and the pool's size."""
+    pages = [-(-n // page) for n in lens]
+    order = torch.randperm(sum(pages), generator=generator, device=DEVICE, dtype=torch.int64).to(torch.int32)
+    table = torch.zeros(len(lens), max(pages), dtype=torch.int32, device=DEVICE)
+    at = 0
+    for b, n in enumerate(pages):
+        table[b, :n] = order[at:at + n]
+        at += n
+    return table, sum(pages)
+
+
+def _ints(values):
+    return torch.tensor(values, dtype=torch.int32).to(DEVICE)
+
+
+def _ends(counts):
+    return _ints([sum(counts[:i]) for i in range(len(counts) + 1)])
+
+
+def prepare(case, seed):
+    generator = torch.Generator(device=DEVICE).manual_seed(seed)
+    dtype = DTYPES[case["dtype"]]
+
+    def normal(*size):
+        return torch.randn(*size, generator=generator, device=DEVICE, dtype=dtype)
+
+    lens, kind = _lengths(case), case["kind"]
+    state = {"case": case}
+    if kind == "dense":
+        b, n, d = case["batch"], case["seqlen"], case["dim"]
+        state.update(q=normal(b, n, case["q_heads"], d), k=normal(b, n, case["kv_heads"], d), v=normal(b, n, case["kv_heads"], d))
+    elif kind == "packed":
+        n, d = sum(lens), case["dim"]
+        state.update(q=normal(n, case["q_heads"], d), k=normal(n, case["kv_heads"], d), v=normal(n, case["kv_heads"], d), ends=_ends(lens),
+                     longest=max(lens))
+    elif kind == "step":
+        blocks, d = _blocks(case), case["dim"]
+        used = [k for _, k in blocks]
+        table, pool = _paged(used, case["page"], generator)
+        state.update(q=normal(sum(q for q, _ in blocks), case["q_heads"], d), k_cache=normal(pool, case["page"], case["kv_heads"], d),
+                     v_cache=normal(pool, case["page"], case["kv_heads"], d), table=table, used=_ints(used), ends=_ends([q for q, _ in blocks]),
+                     tallest=case["chunk"])
+    else:
+        new, batch, append = case["new"], case["batch"], case["append"]
+        table, pool = _paged([n + new * append for n in lens], case["page"], generator)
+        state.update(table=table, used=_ints(lens), k=None, v=None, cos=None, sin=None)
+        if kind == "cache":
+            hk, d = case["kv_heads"], case["dim"]
+            state.update(q=normal(batch, new, case["q_heads"], d), k_cache=normal(pool, case["page"], hk, d), v_cache=normal(pool, case["page"], hk, d))
+            if append:
+                state.update(k=normal(batch, new, hk, d), v=normal(batch, new, hk, d))
+            if case["rotary"] != "none":
+                # rotary tables over the whole head dimension, base 500000
+                rate = 500000.0 ** (-torch.arange(0, d, 2, dtype=torch.float64, device=DEVICE) / d)
+                angle = torch.arange(max(lens) + new, dtype=torch.float64, device=DEVICE)[:, None] * rate[None, :]
+                state.update(cos=torch.cos(angle).to(dtype), sin=torch.sin(angle).to(dtype))
+        else:
+            # symmetric per-token quantisation of N(0, 1) latents: scale = absmax / 127
+            latent = normal(pool, case["page"], 1, LATENT).float()
+            scale = latent.abs().amax(dim=-1) / 127.0
+            codes = torch.clamp(torch.round(latent / scale[..., None]), -127, 127).to(torch.int8)
+            state.update(q=normal(batch, new, case["q_heads"], LATENT), k_cache=codes, v_cache=codes[..., :LATENT_V], scale=scale)
+            if append:
+                fresh = normal(batch, new, 1, LATENT)
+                state.update(k=fresh, v=fresh[..., :LATENT_V])
+    return state
+
+
+def run(state):
+    case = state["case"]
+    kind = case["kind"]
+    if kind == "dense":
+        return flash_attn_func(state["q"], state["k"], state["v"], causal=case["causal"])
+    if kind == "packed":
+        out, lse, _ = flash_attn_varlen_func(state["q"], state["k"], state["v"], state["ends"], state["ends"], state["longest"], state["longest"],
+                                             causal=case["causal"], window_size=(case["window"], 0 if case["causal"] else case["window"]),
+                                             softcap=case["softcap"], return_attn_probs=True)
+        return out, lse
+    if kind == "step":
+        out, lse, _, _ = flash_attn_with_kvcache_3(state["q"], state["k_cache"], state["v_cache"], cache_seqlens=state["used"], page_table=state["table"],
+                                                   cu_seqlens_q=state["ends"], max_seqlen_q=state["tallest"], causal=True, return_softmax_lse=True)
+        return out, lse
+    if kind == "latent":
+        out, lse = flash_attn_with_kvcache(state["q"], state["k_cache"], state["v_cache"], state["k"], state["v"], cache_seqlens=state["used"],
+                                           block_table=state["table"], softmax_scale=192 ** -0.5, causal=True, return_softmax_lse=True,
+                                           k_scale_cache=state["scale"])
+        return (out, lse, state["k_cache"], state["scale"]) if case["append"] else (out, lse)
+    out, lse = flash_attn_with_kvcache(state["q"], state["k_cache"], state["v_cache"], state["k"], state["v"], state["cos"], state["sin"],
+                                       cache_seqlens=state["used"], block_table=state["table"], causal=True, window_size=(case["window"], 0) if
+                                       case["window"] >= 0 else (-1, -1), softcap=case["softcap"], rotary_interleaved=case["rotary"] == "interleaved",
+                                       return_softmax_lse=True)
+    return (out, lse, state["k_cache"], state["v_cache"]) if case["append"] else (out, lse)
+
+
+def _visible(case, n_q, n_k):
+    """((query, key) pairs that the masks leave of a block, keys that at least one query sees)."""
+    causal = case.get("causal", True)
+    left = case.get("window", -1)
+    right = 0 if causal else left
+    if left < 0 and right < 0:
+        return n_q * n_k, n_k
+    pairs, lowest, highest = 0, n_k, -1
+    for i in range(n_q):
+        at = i + n_k - n_q
+        lo = max(0, at - left) if left >= 0 else 0
+        hi = min(n_k - 1, at + right) if right >= 0 else n_k - 1
+        if hi >= lo:
+            pairs += hi - lo + 1
+            lowest, highest = min(lowest, lo), max(highest, hi)
+    return pairs, max(0, highest - lowest + 1)
+
+
+def work(case):
+    latent = case["kind"] == "latent"
+    d, dv = (LATENT, LATENT_V) if latent else (case["dim"], case["dim"])
+    hq, hk = case["q_heads"], 1 if latent else case["kv_heads"]
+    key_bytes = LATENT + 4 if latent else hk * 2 * (d + dv)
+    total_bytes = flops = 0
+    seen = {}
+    for block in _blocks(case):
+        if block not in seen:
+            seen[block] = _visible(case, *block)
+        pairs, keys = seen[block]
+        flops += 2 * (d + dv) * hq * pairs
+        total_bytes += keys * key_bytes + block[0] * hq * (2 * (d + dv) + 4)
+        if case.get("append"):
+            # the new rows are read; the rows written into the cache are then read as keys
+            total_bytes += block[0] * (hk * 2 * (d + (0 if latent else dv)) + key_bytes)
+    return {"bytes": total_bytes, "flops": flops}
+
+
+def tolerance(case):
+    # Against the same attention in 64 bits (rotated queries unrounded), the outputs of the listed kinds are off by at most
+    # rel 2.7e-3, max 2.1e-2 in bf16 and rel 3.3e-4, max 2.3e-3 in fp16: the weights are rounded to the 16-bit type in front of
+    # the second product, the outputs behind it.  Four times that; appended rows, codes and scales are the same to the bit.
+    return {"rel": 1.0e-2, "max": 0.08} if case["dtype"] == "bf16" else {"rel": 1.3e-3, "max": 0.01}
