@@ -295,6 +295,98 @@ def work(case):
     return {"bytes": total_bytes, "flops": flops}
 
 
+EXACT_FLOPS = 2.0e12      # (a few seconds in 64 bits)
+EXACT_SCORES = 1 << 27    # scores held at a time
+
+
+def _rotate(x, cos, sin, first, interleaved):
+    """(tokens, heads, dim) in 64 bits, token i turned by row first + i of the tables."""
+    c, s = (t[first:first + x.shape[0], None, :].double() for t in (cos, sin))
+    a, b = (x[..., 0::2], x[..., 1::2]) if interleaved else x.chunk(2, dim=-1)
+    turned = (a * c - b * s, a * s + b * c)
+    return torch.stack(turned, dim=-1).flatten(-2) if interleaved else torch.cat(turned, dim=-1)
+
+
+def _attend(case, q, k, v, scale):
+    """out (queries, heads, dim of v) and log-sum-exp (heads, queries) of one sequence, all in 64 bits."""
+    n_q, hq, d = q.shape
+    n_k, hk, dv = v.shape
+    left, causal, softcap = case.get("window", -1), case.get("causal", True), case.get("softcap", 0.0)
+    kt, vt = k.permute(1, 2, 0).contiguous(), v.transpose(0, 1).contiguous()
+    out, lse = torch.empty(n_q, hq, dv, dtype=torch.float64, device=DEVICE), torch.empty(hq, n_q, dtype=torch.float64, device=DEVICE)
+    step = max(1, EXACT_SCORES // (hq * n_k))
+    for i in range(0, n_q, step):
+        n = min(step, n_q - i)
+        scores = torch.bmm(q[i:i + n].reshape(n, hk, hq // hk, d).permute(1, 2, 0, 3).reshape(hk, -1, d), kt).view(hq, n, n_k) * scale
+        if softcap:
+            scores = softcap * torch.tanh(scores / softcap)
+        behind = torch.arange(n_k, device=DEVICE) - (torch.arange(i, i + n, device=DEVICE) + n_k - n_q)[:, None]
+        hidden = torch.zeros_like(behind, dtype=torch.bool)
+        if causal or left >= 0:
+            hidden |= behind > (0 if causal else left)
+        if left >= 0:
+            hidden |= behind < -left
+        scores.masked_fill_(hidden, -math.inf)
+        total = torch.logsumexp(scores, dim=-1)
+        weights = torch.exp(scores - total[..., None]).nan_to_num_(0.0)
+        out[i:i + n] = torch.bmm(weights.view(hk, -1, n_k), vt).view(hq, n, dv).transpose(0, 1)
+        lse[:, i:i + n] = torch.where(torch.isinf(total), math.inf, total)     # (a query that sees nothing)
+    return out, lse
+
+
+def _append_exactly(case, state, b, at, rows):
+    """The new rows of sequence b into the pages and slots `rows` of the caches, in the caches' types."""
+    where = (rows[0][at:at + case["new"]], rows[1][at:at + case["new"]])
+    if case["kind"] == "latent":
+        fresh = state["k"][b].float()
+        scale = fresh.abs().amax(dim=-1) / 127.0
+        state["k_cache"][where] = torch.clamp(torch.round(fresh / scale[..., None]), -127, 127).to(torch.int8)
+        state["scale"][where] = scale
+        return
+    k = state["k"][b].double()
+    if case["rotary"] != "none":
+        k = _rotate(k, state["cos"], state["sin"], at, case["rotary"] == "interleaved")
+    state["k_cache"][where] = k.to(state["k_cache"].dtype)
+    state["v_cache"][where] = state["v"][b]
+
+
+def exact(case, seed):
+    """What run() returns, in 64 bits (appended rows in the caches' types, as the attention reads them)."""
+    if work(case)["flops"] > EXACT_FLOPS:
+        return None
+    state, kind = prepare(case, seed), case["kind"]
+    lens, blocks = _lengths(case), _blocks(case)
+    if kind == "dense":
+        return torch.stack([_attend(case, q.double(), k.double(), v.double(), case["dim"] ** -0.5)[0]
+                            for q, k, v in zip(state["q"], state["k"], state["v"])])
+    done, first = [], 0
+    for b, (n_q, n_k) in enumerate(blocks):
+        q = state["q"][b].double() if kind in ("cache", "latent") else state["q"][first:first + n_q].double()
+        if kind == "packed":
+            k, v = (state[name][first:first + n_k].double() for name in ("k", "v"))
+        else:
+            at = torch.arange(n_k, device=DEVICE)
+            rows = (state["table"][b].long()[at // case["page"]], at % case["page"])
+            if case.get("append"):
+                _append_exactly(case, state, b, lens[b], rows)
+            k = state["k_cache"][rows].double()
+            if kind == "latent":
+                k *= state["scale"][rows].double()[..., None]
+                v = k[..., :LATENT_V]
+            else:
+                v = state["v_cache"][rows].double()
+                if case.get("rotary", "none") != "none":
+                    q = _rotate(q, state["cos"], state["sin"], lens[b], case["rotary"] == "interleaved")
+        done.append(_attend(case, q, k, v, 192 ** -0.5 if kind == "latent" else case["dim"] ** -0.5))
+        first += n_q
+    if kind in ("packed", "step"):
+        return torch.cat([out for out, _ in done]), torch.cat([lse for _, lse in done], dim=1)
+    out, lse = torch.stack([out for out, _ in done]), torch.stack([lse for _, lse in done])
+    if not case["append"]:
+        return out, lse
+    return out, lse, state["k_cache"], state["scale" if kind == "latent" else "v_cache"]
+
+
 def tolerance(case):
     # Against the same attention in 64 bits (rotated queries unrounded), the outputs of the listed kinds are off by at most
     # rel 2.7e-3, max 2.1e-2 in bf16 and rel 3.3e-4, max 2.3e-3 in fp16: the weights are rounded to the 16-bit type in front of
