@@ -170,10 +170,15 @@ __device__ __forceinline__ void append_rows_wave(const DecodeParams &p, int b, i
 // l's 16 bytes land at the instruction's LDS base + 16 l, so the lane that fills a place of the swizzled tile fetches
 // the piece that belongs there), into the one of the wave's two tiles that is not being read; `ktile` then points at
 // both (2 * kTileBytes), and the second doubles as the staging area of the q rows before the first chunk uses it.
-template <typename T, int D, bool SOFTCAP, bool PART, int RT>
+// UNIT: the piece is one of several that the waves of a workgroup hold of the same unit; instead of writing anything to
+// memory the wave leaves its rows in its own LDS tiles (fp32, normalised by the piece's own sum; 16-byte pieces of a row
+// swizzled by the row: unit_piece_at()) and their base-2 log-sum-exps in s_lse, for merge_unit().
+template <int D> __device__ __forceinline__ int unit_piece_at(int row, int piece) { return row * (D * 4) + ((piece ^ (row & 15)) << 4); }
+
+template <typename T, int D, bool SOFTCAP, bool PART, int RT, bool UNIT>
 __device__ __forceinline__ void wave_piece(const DecodeParams &p, const int b, const int kvh, const int row0, const int n_rows,
                                            const UnitRange &ur, const int range_lo, const int range_hi, const bool write_final,
-                                           const int64_t slot, uint8_t *ktile) {
+                                           const int64_t slot, uint8_t *ktile, float *s_lse = nullptr) {
     using Cfg = WaveCfg<D>;
     const int lane = threadIdx.x & 63;
     const int lq = lane >> 4;
@@ -461,6 +466,22 @@ __device__ __forceinline__ void wave_piece(const DecodeParams &p, const int b, c
     for (int r = 0; r < RT; ++r) {
         const float lr = quad_rows_sum(l_run[r]);
         const int trow = 16 * r + ln;                 // row of the unit
+        if constexpr (UNIT) {
+            // (every lane reads its own LDS operands of the last chunk before it writes here: the products above have taken them)
+            const float inv = (lr > 0.f) ? 1.f / lr : 0.f;
+#pragma unroll
+            for (int hh = 0; hh < Cfg::kVH; ++hh)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int w = 0; w < Cfg::kVW; w += 4) {
+                        const int t0 = hh * Cfg::kVW + w;
+                        *reinterpret_cast<float4 *>(ktile + unit_piece_at<D>(trow, (hh * 128 + (lq * 4 + i) * Cfg::kVW + w) / 4)) =
+                            make_float4(o_acc[r][t0][i] * inv, o_acc[r][t0 + 1][i] * inv, o_acc[r][t0 + 2][i] * inv, o_acc[r][t0 + 3][i] * inv);
+                    }
+            if (lq == 0) s_lse[trow] = (lr > 0.f) ? m_run[r] + fast_log2(lr) : lr == lr ? -INFINITY : lr;   // (a NaN stays one)
+            continue;
+        }
         if (row0 + trow < n_rows && trow >= dead_rows(p, b)) {
             const float inv = (lr > 0.f) ? 1.f / lr : 0.f;
             const int qi = (row0 + trow) / p.group;
@@ -518,9 +539,107 @@ __global__ void __launch_bounds__(256, (D <= 128) ? 2 : 1) decode_wave_kernel(co
                        row0 = (unit - kvh * p.row_tiles) * 16;
                        n_rows = p.rows_total;
                    }
-                   wave_piece<T, D, SOFTCAP, PART, RT>(p, b, kvh, row0, n_rows, ur, range_lo, range_hi, whole, slot, s_k[wave]);
+                   wave_piece<T, D, SOFTCAP, PART, RT, false>(p, b, kvh, row0, n_rows, ur, range_lo, range_hi, whole, slot, s_k[wave]);
                });
     init_empty_units<D>(p, pt);
+}
+
+// Merge of the pieces that the NW waves of a workgroup left of unit (b, kvh): every thread takes 16-byte pieces of rows.
+template <typename T, int D, int NW, int RT>
+__device__ __forceinline__ void merge_unit(const DecodeParams &p, int b, int kvh, const uint8_t *tiles, int wave_bytes, const float (*s_lse)[RT * 16]) {
+    constexpr int kPieces = D / 4;
+    for (int idx = threadIdx.x; idx < p.rows * kPieces; idx += NW * 64) {
+        const int row = idx / kPieces;
+        const int piece = idx - row * kPieces;
+        if (row < dead_rows(p, b) || piece * 4 >= p.headdim) continue;
+        float lw[NW];
+        float mx = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            lw[w] = s_lse[w][row];
+            mx = fmaxf(mx, lw[w]);
+        }
+        const float mx_use = (mx == -INFINITY) ? 0.f : mx;
+        float tot = 0.f;
+        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            if (lw[w] == -INFINITY) continue;   // nothing visible, or no piece at all: its tile holds no rows
+            const float e = fast_exp2(lw[w] - mx_use);
+            const float4 o = *reinterpret_cast<const float4 *>(tiles + w * wave_bytes + unit_piece_at<D>(row, piece));
+            tot += e;
+            acc[0] += e * o.x;
+            acc[1] += e * o.y;
+            acc[2] += e * o.z;
+            acc[3] += e * o.w;
+        }
+        const float inv = (tot > 0.f) ? 1.f / tot : 0.f;
+        const RowId rid = row_id(p, kvh, row);
+        uint16_t *dst = reinterpret_cast<uint16_t *>(p.out) + (int64_t)b * p.o_stride_b + (int64_t)rid.qi * p.o_stride_s +
+                        (int64_t)rid.head * p.o_stride_h + piece * 4;
+        uint2 o2;
+        o2.x = pack2<T>(acc[0] * inv, acc[1] * inv);
+        o2.y = pack2<T>(acc[2] * inv, acc[3] * inv);
+        *reinterpret_cast<uint2 *>(dst) = o2;
+        if (piece == 0)
+            p.lse[((int64_t)b * p.nheads + rid.head) * p.seqlen_q + rid.qi] = (tot > 0.f) ? (mx + fast_log2(tot)) * kLn2 : INFINITY;
+    }
+}
+
+// Short units: one workgroup per (batch row, kv head), its chunks cut evenly over the workgroup's NW waves, and the waves'
+// pieces merged through LDS.  One launch, no partials in memory, no partition to work out: what is left in front of the
+// first keys are the length and the table entry.
+// Bound by latency: ~6 us of launch, lengths, table entry, q rows and merge, and one trip to memory (~2.6 us) per chunk of a
+// wave, which is why the chunks go to as many waves as a compute unit holds.  1 sequence x 8 kv heads x 700 keys, D = 128:
+// 16.7 us as a partition over the device with its merge launch, 10.0 us here; 40 x 16 kv heads x 33..900 keys, D = 64 (80 MB):
+// 31.1 and 20.8 us.  Which calls come here is the host's rule (unit_waves() in fa_rocm_api.cpp).
+template <typename T, int D, bool SOFTCAP, bool PART, int RT, int NW>
+__global__ void __launch_bounds__(NW * 64, (D <= 128) ? 2 : 1) decode_unit_kernel(const DecodeParams p) {
+    using Cfg = WaveCfg<D>;
+    __shared__ __attribute__((aligned(16))) uint8_t s_k[NW][2 * Cfg::kTileBytes];
+    __shared__ float s_lse[NW][RT * 16];
+    static_assert(RT * 16 * D * 4 <= 2 * Cfg::kTileBytes, "a wave's rows fit its tiles");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b = blockIdx.x / p.nheads_k;
+    const int kvh = blockIdx.x - b * p.nheads_k;
+    const UnitRange ur = unit_range(p, b, window_norm_m(p));
+    const int per = (ur.nchunks + NW - 1) / NW;
+    const int lo = wave * per, hi = min(ur.nchunks, lo + per);
+    if (lo < hi) {
+        const int range_lo = max(ur.lo, (ur.c0 + lo) * kChunk), range_hi = min(ur.hi, (ur.c0 + hi) * kChunk);
+        wave_piece<T, D, SOFTCAP, PART, RT, true>(p, b, kvh, 0, p.rows, ur, range_lo, range_hi, false, 0, s_k[wave], s_lse[wave]);
+    } else if ((threadIdx.x & 63) < RT * 16) {
+        s_lse[wave][threadIdx.x & 63] = -INFINITY;
+    }
+    __syncthreads();
+    merge_unit<T, D, NW, RT>(p, b, kvh, &s_k[0][0], 2 * Cfg::kTileBytes, s_lse);
+}
+
+template <typename T, int D, int RT, int NW> static hipError_t launch_unit_nw(const DecodeParams &p, hipStream_t stream) {
+    const dim3 grid((unsigned)(p.batch * p.nheads_k)), block(NW * 64);
+    const bool part = p.headdim < D;
+    if (p.softcap_post != 0.f) {
+        if (part)
+            hipLaunchKernelGGL((decode_unit_kernel<T, D, true, true, RT, NW>), grid, block, 0, stream, p);
+        else
+            hipLaunchKernelGGL((decode_unit_kernel<T, D, true, false, RT, NW>), grid, block, 0, stream, p);
+    } else {
+        if (part)
+            hipLaunchKernelGGL((decode_unit_kernel<T, D, false, true, RT, NW>), grid, block, 0, stream, p);
+        else
+            hipLaunchKernelGGL((decode_unit_kernel<T, D, false, false, RT, NW>), grid, block, 0, stream, p);
+    }
+    return hipGetLastError();
+}
+
+template <typename T, int D> static hipError_t launch_unit_d(const DecodeParams &p, hipStream_t stream) {
+    if (p.headdim > D || p.headdim < 8 || p.headdim % 8 != 0) return hipErrorInvalidValue;
+    if constexpr (D <= 128) {
+        if (p.unit_waves == 8) return p.rows > 16 ? launch_unit_nw<T, D, 2, 8>(p, stream) : launch_unit_nw<T, D, 1, 8>(p, stream);
+        return p.rows > 16 ? launch_unit_nw<T, D, 2, 4>(p, stream) : launch_unit_nw<T, D, 1, 4>(p, stream);
+    } else {
+        return launch_unit_nw<T, D, 1, 4>(p, stream);
+    }
 }
 
 template <typename T, int D, int RT> static hipError_t launch_wave_rt(const DecodeParams &p, hipStream_t stream) {
@@ -560,6 +679,22 @@ template <typename T> static hipError_t launch_wave_t(const DecodeParams &p, int
         case 256: return launch_wave_d<T, 256>(p, stream);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_decode_unit(const DecodeParams &p, int dtype, int headdim, hipStream_t stream) {
+    if (p.rows > wave_rows_per_unit(headdim) || p.row_tiles > 1 || p.units_per_token > 0 || (p.unit_waves != 4 && p.unit_waves != 8) ||
+        (int64_t)p.batch * p.nheads_k >= (1ll << 31))
+        return hipErrorInvalidValue;
+    auto pick = [&](auto t) -> hipError_t {
+        using T = decltype(t);
+        switch (headdim) {
+            case 64: return launch_unit_d<T, 64>(p, stream);
+            case 128: return launch_unit_d<T, 128>(p, stream);
+            case 256: return launch_unit_d<T, 256>(p, stream);
+            default: return hipErrorInvalidValue;
+        }
+    };
+    return dtype == 0 ? pick(BF16{}) : pick(FP16{});
 }
 
 hipError_t launch_decode_wave(const DecodeParams &p, int dtype, int headdim, hipStream_t stream) {

@@ -59,6 +59,7 @@ struct DecodeParams {
                                    // its own for the wave-level kernel: nheads_k = kv heads * row_tiles units per batch row (unit =
                                    // kv head * row_tiles + tile), rows = 16 per unit, rows_total = seqlen_q * group; else 0 or 1
     int32_t rows_total;            // seqlen_q * group when row_tiles > 1
+    int32_t unit_waves;            // short units (launch_decode_unit): waves of the workgroup that takes a unit, 4 or 8
 };
 
 struct AppendParams {
@@ -213,6 +214,8 @@ hipError_t launch_append_quant_i8(const AppendParams &p, int dtype, hipStream_t 
 hipError_t launch_rotate_q(const RotateQParams &p, int dtype, hipStream_t stream);
 hipError_t launch_decode_paged(const DecodeParams &p, int dtype, int headdim, hipStream_t stream);
 hipError_t launch_decode_wave(const DecodeParams &p, int dtype, int headdim, hipStream_t stream);
+// one workgroup of unit_waves waves per (batch row, kv head): no workspace, no merge launch
+hipError_t launch_decode_unit(const DecodeParams &p, int dtype, int headdim, hipStream_t stream);
 hipError_t launch_splitkv_combine(const DecodeParams &p, int dtype, int headdim_v, hipStream_t stream);
 hipError_t launch_decode_mla_i8(const DecodeParams &p, int dtype, hipStream_t stream);
 hipError_t launch_prefill(const PrefillParams &p, int dtype, int headdim, hipStream_t stream);

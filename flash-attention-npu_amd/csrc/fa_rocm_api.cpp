@@ -71,6 +71,7 @@ struct EnvKnobs {
     bool block_workers = false;    // FA_ROCM_DECODE_BLOCK_WORKERS
     int min_share = 0;             // FA_ROCM_MIN_SHARE
     int piece_cost = -1;           // FA_ROCM_PIECE_COST
+    int unit_waves = -1;           // FA_ROCM_UNIT_WAVES: 0 = no workgroup per unit; 4 or 8 = always, with that many waves
     bool no_head_interleave = false, separate_append = false, no_short_blocks = false;
     bool validate = false;         // FA_ROCM_VALIDATE: check tables, capacities and positions on the device (slow)
 };
@@ -94,6 +95,7 @@ void load_env() {
     e.block_workers = flag("FA_ROCM_DECODE_BLOCK_WORKERS");
     e.min_share = num("FA_ROCM_MIN_SHARE", 0);
     e.piece_cost = std::getenv("FA_ROCM_PIECE_COST") ? std::max(0, num("FA_ROCM_PIECE_COST", 0)) : -1;
+    e.unit_waves = num("FA_ROCM_UNIT_WAVES", -1);
     e.no_head_interleave = flag("FA_ROCM_NO_HEAD_INTERLEAVE");
     e.separate_append = flag("FA_ROCM_SEPARATE_APPEND");
     e.no_short_blocks = flag("FA_ROCM_NO_SHORT_BLOCKS");
@@ -223,6 +225,45 @@ int64_t live_keys_bound(const fa_kvcache_args *a) {
         if (span < cap) cap = span;
     }
     return cap > 0 ? cap : 1;
+}
+
+// Waves of the workgroup that takes a whole unit (batch row, kv head) of this call (fa::launch_decode_unit), 0 when the
+// units are cut over the device instead.
+// The partition over the device costs ~10 us whatever the work: the lengths' prefix pass, partials of every wave, a merge
+// launch.  A workgroup per unit costs ~6 us and ~2.6 us per chunk of its longest wave (one chunk of a wave is in flight, a
+// trip to memory each), so it is ahead while the longest unit is short, and for longer ones where there are units enough to
+// keep every compute unit busy; the host knows the longest unit's bound, the keys that the table or the window allows.
+// Whole call in us, partition / workgroup per unit, 4 q heads per kv head, all units of the stated keys unless a range:
+//   D = 128:  8 units x 512 keys 16.5 / 10.1, x 1024 16.6 / 16.1, x 2048 20.7 / 27.4;  64 x 1024 21.5 / 18.1, x 2048 27.9 / 30.1
+//             128 x 1500 34.2 / 26.2, x 200..2000 31.3 / 28.8, x 400..4000 41.4 / 50.9;  320 x 200..2000 45.9 / 45.5, x 400..4000 70.9 / 83.8
+//             1024 x 128 33.1 / 20.3, x 200..2048 115.9 / 111.0;  2048 x 128 36.8 / 37.2, x 512 96.6 / 91.9;  4096 x 128 63.2 / 70.2
+//   D = 64:   256 x 1024 30.9 / 16.8;  2048 x 512 55.2 / 52.4;  6400 x 40 49.6 / 45.1, x 512 154.1 / 151.2
+//   D = 256:  8 x 512 21.2 / 19.1, x 1024 21.1 / 29.4;  256 x 2048 99.9 / 81.1;  512 x 2048 180.1 / 162.1;  1024 x 128 38.8 / 48.8
+//   17-32 rows, D = 128, against the tiled kernel or two tiles per wave:  16 units x 700 22.1 / 18.7, x 1000 24.3 / 26.4
+//             128 x 300..3000 52.9 / 47.9;  192 x 1000 47.2 / 31.8;  1024 x 2048 227 / 191;  2048 x 128 52.9 / 67.0
+// Workgroups of 8 waves up to one per compute unit, of 4 beyond (512 units x 512 keys 29.6 with 8, 26.0 with 4).
+int unit_waves(const fa_kvcache_args *a, size_t rows, int num_cus) {
+    const EnvKnobs &e = env();
+    const int width = fa::tile_headdim(a->headdim_qk);
+    if (is_mla_i8(a) || a->num_splits != 0 || rows > (size_t)fa::wave_rows_per_unit(width)) return 0;
+    if (e.unit_waves >= 0) return e.unit_waves == 8 && width <= 128 ? 8 : e.unit_waves > 0 ? 4 : 0;
+    // (the other knobs ask for the partition over the device)
+    if (e.decode_max_rows || e.wave_max_rows || e.wave_two_tiles || e.decode_wgs || e.block_workers || e.min_share || e.piece_cost >= 0 ||
+        e.no_head_interleave || e.separate_append)
+        return 0;
+    const int64_t units = (int64_t)a->batch * a->nheads_k, keys = live_keys_bound(a), cus = num_cus;
+    const bool few = units < cus / 2;
+    int64_t most;   // keys of the longest unit
+    if (width > 128)
+        most = units < cus ? 512 : units <= 2 * cus ? 2048 : 0;
+    else if (rows > 16)
+        most = few ? 768 : units <= 4 * cus ? 3072 : 0;
+    else if (units > 6 * cus)
+        most = (width == 64 ? units <= 32 * cus : units <= 8 * cus) ? 512 : 0;
+    else
+        most = few ? 1024 : 2048;
+    if (keys > most) return 0;
+    return width <= 128 && units <= cus && (rows <= 16 || keys > 512) ? 8 : 4;
 }
 
 }  // namespace
@@ -499,7 +540,8 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
 
     int cus_t = device_cus();
     if (cus_t <= 0) cus_t = 256;
-    if (!is_mla_i8(a) && rows > decode_max_rows(a, cus_t)) {
+    const int waves_of_unit = unit_waves(a, (size_t)rows, cus_t);
+    if (!is_mla_i8(a) && waves_of_unit == 0 && rows > decode_max_rows(a, cus_t)) {
         // query block too tall for the decode kernel: tiled forward over the paged cache
         fa_split_plan tplan;
         rc = fa_rocm_plan_kvcache(a, cus_t, &tplan);
@@ -696,7 +738,8 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
     p.num_wgs = plan.num_wgs;
     p.num_workers = plan.num_workers;
     p.min_share = plan.min_share;
-    p.wave_workers = plan.num_workers != plan.num_wgs;
+    p.wave_workers = waves_of_unit > 0 || plan.num_workers != plan.num_wgs;
+    p.unit_waves = waves_of_unit;
     p.min_share_long = (p.wave_workers && env().min_share <= 0) ? 4 : 0;
     // wave workers of neighbouring kv heads walk the same token range together
     // Fixed cost of starting on a unit, in chunk times.  Latent kernel: ~15 us of q staging and pipeline
@@ -705,7 +748,7 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
     // charging 1-3 chunks measured within +-1 %, so it is not charged.
     p.piece_cost = is_mla_i8(a) ? 7 : 0;
     if (env().piece_cost >= 0) p.piece_cost = env().piece_cost;
-    const int row_tiles = p.wave_workers ? wave_row_tiles(a, rows, cus) : 0;
+    const int row_tiles = (p.wave_workers && p.unit_waves == 0) ? wave_row_tiles(a, rows, cus) : 0;
     if (row_tiles > 1) {
         // (kv head, 16-row tile) units: the tiles of a kv head are neighbouring units
         p.row_tiles = row_tiles;
@@ -715,7 +758,7 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
     }
     p.head_interleave = p.wave_workers && p.nheads_k > 1 && plan.num_workers % p.nheads_k == 0 &&
                         !env().no_head_interleave;
-    const bool needs_combine = need > 0;
+    const bool needs_combine = need > 0 && p.unit_waves == 0;
     if (needs_combine) {
         const size_t hdr = p.balanced ? fa::kPartitionHeaderBytes : 0;
         const size_t slot_rows = (need - hdr) / partial_row_bytes(a);
@@ -728,7 +771,7 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
     // (and so owned by exactly one wave): causal or no right bound, and no left bound that could
     // exclude the oldest new key.  Otherwise the rows are written by their own kernel first.
     // With row tiles several waves read every chunk and only one of them would write the row: no fusion.
-    const bool fuse_append = a->k_new && p.balanced && p.wave_workers && row_tiles <= 1 && (a->causal || a->window_right < 0) &&
+    const bool fuse_append = a->k_new && (p.balanced || p.unit_waves > 0) && p.wave_workers && row_tiles <= 1 && (a->causal || a->window_right < 0) &&
                              (a->window_left < 0 || (int64_t)a->seqlen_q + a->window_left >= a->seqlen_new) &&
                              !env().separate_append;
     if (fuse_append) {
@@ -754,7 +797,9 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
         p.rows = 128;
         e = fa::launch_decode_mla_i8(p, a->io_dtype, stream);
     }
-    else {
+    else if (p.unit_waves > 0) {
+        e = fa::launch_decode_unit(p, a->io_dtype, fa::tile_headdim(a->headdim_qk), stream);
+    } else {
         e = fa::launch_decode_paged(p, a->io_dtype, fa::tile_headdim(a->headdim_qk), stream);
     }
     if (e != hipSuccess) return fail(FA_ERR_LAUNCH, "decode launch failed: %s", hipGetErrorString(e));
