@@ -240,7 +240,8 @@ int64_t live_keys_bound(const fa_kvcache_args *a) {
 //   D = 64:   256 x 1024 30.9 / 16.8;  2048 x 512 55.2 / 52.4;  6400 x 40 49.6 / 45.1, x 512 154.1 / 151.2
 //   D = 256:  8 x 512 21.2 / 19.1, x 1024 21.1 / 29.4;  256 x 2048 99.9 / 81.1;  512 x 2048 180.1 / 162.1;  1024 x 128 38.8 / 48.8
 //   17-32 rows, D = 128, against the tiled kernel or two tiles per wave:  16 units x 700 22.1 / 18.7, x 1000 24.3 / 26.4
-//             128 x 300..3000 52.9 / 47.9;  192 x 1000 47.2 / 31.8;  1024 x 2048 227 / 191;  2048 x 128 52.9 / 67.0
+//             64 x 8000 68.7 / 101.7;  128 x 300..3000 52.9 / 47.9;  192 x 1000 47.2 / 31.8, x 400..4000 84.8 / 65.2, x 8000 240 / 136
+//             256 x 800..8000 152 / 133;  512 x 400..4000 140 / 132;  1024 x 2048 227 / 191;  2048 x 128 52.9 / 67.0
 // Workgroups of 8 waves up to one per compute unit, of 4 beyond (512 units x 512 keys 29.6 with 8, 26.0 with 4).
 int unit_waves(const fa_kvcache_args *a, size_t rows, int num_cus) {
     const EnvKnobs &e = env();
@@ -257,7 +258,7 @@ int unit_waves(const fa_kvcache_args *a, size_t rows, int num_cus) {
     if (width > 128)
         most = units < cus ? 512 : units <= 2 * cus ? 2048 : 0;
     else if (rows > 16)
-        most = few ? 768 : units <= 4 * cus ? 3072 : 0;
+        most = few ? 768 : units <= 4 * cus ? (4 * units >= 3 * cus && units <= cus ? 8192 : 3072) : 0;
     else if (units > 6 * cus)
         most = (width == 64 ? units <= 32 * cus : units <= 8 * cus) ? 512 : 0;
     else
