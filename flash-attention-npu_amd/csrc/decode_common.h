@@ -65,7 +65,11 @@ __device__ __forceinline__ UnitRange unit_range(const DecodeParams &p, int b, in
 // share holds the start of a further unit gets that many fewer chunks.  Partition::cost is
 // p.piece_cost when the shares are long against it and 0 otherwise: every worker pays for its first
 // piece anyway, and with shares of a few chunks charging the unit starts would unbalance them.
-__device__ __forceinline__ int unit_cost(int nchunks, int cost) { return nchunks > 0 ? nchunks + cost : 0; }
+// align > 1: the lengths are rounded up to multiples of the share, so that no share crosses into a second unit.
+__device__ __forceinline__ int unit_cost(int nchunks, int cost, int align) {
+    const int n = nchunks > 0 ? nchunks + cost : 0;
+    return align > 1 ? (n + align - 1) / align * align : n;
+}
 
 // exclusive prefixes over 256 equal segments of the batch: s_pref[t] = chunks of rows [0, t*seg),
 // s_cnt[t] = rows among them with a visible key; [256] = totals.  All threads of the block must call
@@ -140,7 +144,7 @@ struct UnitPos {
 
 // batch row whose units contain list position `pos` (0 <= pos < Hk * total)
 __device__ __forceinline__ UnitPos locate_row(const DecodeParams &p, const int *s_pref, int seg, int64_t pos, int M,
-                                              int list_heads, int cost) {
+                                              int list_heads, int cost, int align) {
     const int target = (int)(pos / list_heads);  // rows with pref <= target < pref + n
     int lo = 0, hi = 256;                        // segment t with s_pref[t] <= target < s_pref[t+1]
     while (hi - lo > 1) {
@@ -151,7 +155,7 @@ __device__ __forceinline__ UnitPos locate_row(const DecodeParams &p, const int *
     u.b = lo * seg;
     u.pref = s_pref[lo];
     for (;;) {
-        const int n = unit_cost(unit_range(p, u.b, M).nchunks, cost);
+        const int n = unit_cost(unit_range(p, u.b, M).nchunks, cost, align);
         if (target < u.pref + n || u.b + 1 >= p.batch) break;
         u.pref += n;
         ++u.b;
@@ -290,6 +294,7 @@ struct Partition {
     int seg;        // batch rows per prefix segment
     int list_heads; // kv heads inside the list: nheads_k (plain) or 1 (head-interleaved)
     int cost;       // list length charged per unit on top of its chunks (unit_cost)
+    int align;      // > 1: units are padded to multiples of this many chunks, which is S
     int64_t W, S;
     bool any_empty; // some batch row has no visible key
     __device__ __forceinline__ int64_t worker_of(int64_t share, int kvh, int hk) const {
@@ -297,9 +302,59 @@ struct Partition {
     }
 };
 
+// A share that holds the end of one unit and the start of the next pays the fixed cost of a piece (lengths -> table ->
+// keys, q rows, stores: ~12 us of a workgroup of the latent kernel) twice, and the launch lasts as long as its slowest
+// worker.  With shares of a few chunks (~2 us each) that is most of the launch, so the units are padded to multiples of
+// the share there, if the device has workers enough for it at the same share or one up to p.align_slack chunks longer;
+// long shares are left as they are (a longer one would cost more than the second start).
+// Latent kernel, whole call, shares that cross units / aligned: 3 sequences of 916..2489 keys 47.1 / 39.1 us, 8 of
+// 1000..10000 52.4 / 44.5, 64 of 300..3000 83.5 / 62.9 (85.0 without a longer share); one sequence 24.9 / 27.1 (nothing to
+// cross: the host leaves it off).  The wave-level kernel, whose pieces start in ~6 us, gains nothing: 4 sequences x 8 kv
+// heads x 4096 visible keys 27.1 / 29.1, 8 x 4 heads x 2000..20000 keys 44.9 / 45.8.
+constexpr int kAlignTries = 4, kAlignMaxShare = 16;
+__device__ __forceinline__ void align_partition(const DecodeParams &p, Partition &pt, int *s_pref, int64_t shares) {
+    __shared__ int s_need[4][kAlignTries], s_sum[4];
+    if (pt.seg != 1 || pt.cost != 0 || p.align_slack < 0 || pt.S > kAlignMaxShare) return;   // the same in every thread
+    const int tid = threadIdx.x, S0 = (int)pt.S;
+    const int n = tid < 256 ? s_pref[tid + 1] - s_pref[tid] : 0;   // this batch row's chunks
+    int need[kAlignTries];
+#pragma unroll
+    for (int i = 0; i < kAlignTries; ++i) {
+        need[i] = (n + S0 + i - 1) / (S0 + i);
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) need[i] += __shfl_xor(need[i], d, 64);
+        if ((tid & 63) == 0 && tid < 256) s_need[tid >> 6][i] = need[i];
+    }
+    __syncthreads();
+    int S = 0;
+#pragma unroll
+    for (int i = kAlignTries - 1; i >= 0; --i) {
+        const int64_t all = (int64_t)(s_need[0][i] + s_need[1][i] + s_need[2][i] + s_need[3][i]) * pt.list_heads;
+        if (i <= p.align_slack && all <= shares) S = S0 + i;
+    }
+    if (S == 0) return;
+    int inc = unit_cost(n, 0, S);
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int v = __shfl_up(inc, d, 64);
+        if ((tid & 63) >= d) inc += v;
+    }
+    if ((tid & 63) == 63 && tid < 256) s_sum[tid >> 6] = inc;
+    __syncthreads();   // (everyone has read the old prefixes)
+    if (tid < 256) {
+        for (int w = 0; w < (tid >> 6); ++w) inc += s_sum[w];
+        s_pref[tid + 1] = inc;
+    }
+    __syncthreads();
+    pt.align = S;
+    pt.S = S;
+    pt.W = (int64_t)s_pref[256] * pt.list_heads;
+}
+
 // Block-level (256 threads, contains barriers): prefix sums into s_pref[257], share size for
 // p.num_workers workers (never below p.min_share chunks).
-__device__ __forceinline__ Partition make_partition(const DecodeParams &p, int *s_pref) {
+// ALIGN: shares of a few chunks may be aligned to the units (align_partition); batches of more than 256 rows never are.
+template <bool ALIGN = false> __device__ __forceinline__ Partition make_partition(const DecodeParams &p, int *s_pref) {
     Partition pt;
     pt.seg = (p.batch + 255) / 256;
     pt.M = window_norm_m(p);
@@ -315,8 +370,10 @@ __device__ __forceinline__ Partition make_partition(const DecodeParams &p, int *
         __syncthreads();
     }
     pt.W = (int64_t)s_pref[256] * pt.list_heads;
-    const bool long_units = p.min_share_long > 0 && (int64_t)s_pref[256] >= (int64_t)kLongUnitChunks * max(s_cnt[256], 1) + (int64_t)pt.cost * s_cnt[256];
+    const bool long_units = p.min_share_long > 0 && (int64_t)s_pref[256] >= (int64_t)p.long_unit_chunks * max(s_cnt[256], 1) + (int64_t)pt.cost * s_cnt[256];
     pt.S = max((pt.W + shares - 1) / shares, (int64_t)max(long_units ? p.min_share_long : p.min_share, 1));
+    pt.align = 1;
+    if constexpr (ALIGN) align_partition(p, pt, s_pref, shares);
     return pt;
 }
 
@@ -329,6 +386,7 @@ __device__ __forceinline__ void publish_partition(const DecodeParams &p, const P
     if (threadIdx.x == 0) {
         p.part_hdr[0] = pt.M;
         p.part_hdr[1] = pt.cost;
+        p.part_hdr[6] = pt.align;
         p.part_hdr[2] = (int32_t)(uint32_t)pt.W;
         p.part_hdr[3] = (int32_t)((uint64_t)pt.W >> 32);
         p.part_hdr[4] = (int32_t)(uint32_t)pt.S;
@@ -343,6 +401,7 @@ __device__ __forceinline__ Partition read_partition(const DecodeParams &p, int b
     pt.seg = 1;
     pt.M = h[0];
     pt.cost = h[1];
+    pt.align = h[6];
     pt.W = (int64_t)(((uint64_t)(uint32_t)h[3] << 32) | (uint32_t)h[2]);
     pt.S = (int64_t)(((uint64_t)(uint32_t)h[5] << 32) | (uint32_t)h[4]);
     pt.list_heads = p.head_interleave ? 1 : p.nheads_k;
@@ -355,7 +414,7 @@ __device__ __forceinline__ Partition read_partition(const DecodeParams &p, int b
 __device__ __forceinline__ int chunks_before(const DecodeParams &p, const Partition &pt, const int *s_pref, int b) {
     const int t = b / pt.seg;
     int pref = s_pref[t];
-    for (int bb = t * pt.seg; bb < b; ++bb) pref += unit_cost(unit_range(p, bb, pt.M).nchunks, pt.cost);
+    for (int bb = t * pt.seg; bb < b; ++bb) pref += unit_cost(unit_range(p, bb, pt.M).nchunks, pt.cost, pt.align);
     return pref;
 }
 
@@ -386,10 +445,10 @@ __device__ __forceinline__ void walk_share(const DecodeParams &p, const Partitio
     int64_t pos = share * pt.S;
     const int64_t end = min(pt.W, pos + pt.S);
     if (pos >= end) return;
-    UnitPos up = locate_row(p, s_pref, pt.seg, pos, pt.M, pt.list_heads, pt.cost);
+    UnitPos up = locate_row(p, s_pref, pt.seg, pos, pt.M, pt.list_heads, pt.cost, pt.align);
     UnitRange ur = unit_range(p, up.b, pt.M);
     const int64_t row_start = (int64_t)up.pref * pt.list_heads;   // list position of unit (b, 0)
-    int ucost = unit_cost(ur.nchunks, pt.cost);
+    int ucost = unit_cost(ur.nchunks, pt.cost, pt.align);
     int kvh = (int)((pos - row_start) / ucost);
     int cost_off = (int)((pos - row_start) - (int64_t)kvh * ucost);  // offset into the unit's interval
     bool first = true;
@@ -397,7 +456,7 @@ __device__ __forceinline__ void walk_share(const DecodeParams &p, const Partitio
         const int take_cost = (int)min((int64_t)(ucost - cost_off), end - pos);
         // the chunks of the unit that this stretch of its interval holds
         const int off_lo = max(0, cost_off - pt.cost);
-        const int off_hi = max(0, cost_off + take_cost - pt.cost);
+        const int off_hi = min(ur.nchunks, max(0, cost_off + take_cost - pt.cost));   // (the padding holds none)
         if (off_hi > off_lo) {
             const bool whole = (off_lo == 0) && (off_hi == ur.nchunks);
             const int c_lo = ur.c0 + off_lo;
@@ -415,7 +474,7 @@ __device__ __forceinline__ void walk_share(const DecodeParams &p, const Partitio
                 if (up.b < p.batch) ur = unit_range(p, up.b, pt.M);
             } while (up.b < p.batch && ur.nchunks == 0);
             if (up.b >= p.batch) break;
-            ucost = unit_cost(ur.nchunks, pt.cost);
+            ucost = unit_cost(ur.nchunks, pt.cost, pt.align);
         }
     }
 }
@@ -431,10 +490,10 @@ template <int DV> __device__ __forceinline__ void init_empty_units(const DecodeP
 }
 
 // Workgroup-level worker: the share `worker` (a permutation of the workgroup numbers), then the empty-unit duty.
-template <int DV, typename PieceFn>
+template <int DV, bool ALIGN = false, typename PieceFn>
 __device__ __forceinline__ void balanced_driver(const DecodeParams &p, int worker, PieceFn piece) {
     __shared__ int s_pref[257];
-    const Partition pt = make_partition(p, s_pref);
+    const Partition pt = make_partition<ALIGN>(p, s_pref);
     publish_partition(p, pt, s_pref);
     walk_share(p, pt, s_pref, worker, piece);
     init_empty_units<DV>(p, pt);

@@ -1,0 +1,22 @@
+"""Latent decode of ragged batches whose units are padded to whole shares, and of batches with too many units for that:
+lengths around the 32-key chunk, empty rows, one to many units, against the oracle."""
+import pytest
+import torch
+
+import fa_oracle as O
+from helpers import check_out, library_env
+from test_gpu_mla import mla_case, run
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [0, 1, 31, 32, 33, 63, 64, 65, 96, 500, 2049]
+
+
+@pytest.mark.parametrize("wgs", [0, 13, 40])          # 0: the device's; 13: a worker takes several units; 40: barely enough to align
+@pytest.mark.parametrize("lens", [[700, 33], EDGES, [1500, 916, 2489], [40 + 37 * i for i in range(30)]])
+def test_ragged_shares(lens, wgs):
+    case = mla_case(len(lens), 128, lens, page=64, seed=len(lens) + wgs)
+    with library_env(**({"FA_ROCM_DECODE_WGS": wgs} if wgs else {})):
+        got, ref, _ = run(case)
+    check_out(got[0], ref[0], got[1], ref[1], f"shares {len(lens)} units, {wgs} workers")
+
