@@ -142,6 +142,7 @@ struct PrefillParams {
     int32_t *list_state;
     int32_t list_wgs;
     int32_t num_mb, units8;        // set by the launcher: 128-row blocks per unit, units rounded up to 8
+    int32_t mb_run;                // set by the launcher: blocks of a unit that are neighbours in the launch order
     int32_t seqlen_q_fixed, seqlen_k_add;   // kvcache layout: Sq per row, keys appended this call
     int32_t max_seqlen_q, total_q;
     int32_t page_size, max_blocks, num_blocks;
