@@ -92,7 +92,16 @@ __global__ void __launch_bounds__(64) append_quant_i8_kernel(const AppendParams 
     const uint16_t *src = reinterpret_cast<const uint16_t *>(p.k_new) + (int64_t)b * p.kn_stride_b + (int64_t)t * p.kn_stride_s;
     int8_t *dst = reinterpret_cast<int8_t *>(p.k_cache) + (int64_t)blk * p.k_stride_block + (int64_t)inpage * p.k_stride_row;
 
-    const float scale = quantise_row<T>(src, dst, d);
+    float absmax = 0.f;
+    for (int e = lane; e < d; e += 64) absmax = fmaxf(absmax, fabsf(to_float<T>(src[e])));
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) absmax = fmaxf(absmax, __shfl_xor(absmax, m, 64));
+    const float scale = __fdiv_rn(absmax, 127.0f);
+    for (int e = lane; e < d; e += 64) {
+        float c = 0.f;
+        if (scale > 0.f) c = fminf(fmaxf(rintf(__fdiv_rn(to_float<T>(src[e]), scale)), -127.f), 127.f);
+        dst[e] = (int8_t)(int)c;
+    }
     if (lane == 0) {
         const int64_t so = (int64_t)blk * p.ks_stride_block + (int64_t)inpage * p.ks_stride_row;
         p.k_scale[so] = scale;

@@ -832,35 +832,7 @@ __device__ __forceinline__ void mla_piece(const DecodeParams &p, const int b, co
     __syncthreads();   // the LDS tiles and sums are reused by the next piece
 }
 
-// The new rows whose positions fall into [range_lo, range_hi), quantised into the cache by the workgroup that is about to
-// read that range (the host asks for it only where every chunk has one reader), a wave a row: the append kernel's launch
-// in front of the decode was 5 us of a call (3 sequences of 916..2489 keys: 38.2 -> 35.8 us).
-template <typename T>
-__device__ __forceinline__ void append_latent_rows(const DecodeParams &p, int b, int len_cache, int range_lo, int range_hi) {
-    const int wave = threadIdx.x >> 6;
-    for (int t = max(0, range_lo - len_cache) + wave; t < min(p.seqlen_new, range_hi - len_cache); t += kMlaThreads / 64) {
-        const int pos = len_cache + t;
-        const int page = pos / p.page_size;
-        if (page >= p.max_blocks) continue;
-        const int blk = p.block_table[(int64_t)b * p.bt_stride_b + page];
-        if (blk < 0 || blk >= p.num_blocks) continue;
-        const int inpage = pos - page * p.page_size;
-        const uint16_t *src = reinterpret_cast<const uint16_t *>(p.k_new) + (int64_t)b * p.kn_stride_b + (int64_t)t * p.kn_stride_s;
-        int8_t *dst = const_cast<int8_t *>(reinterpret_cast<const int8_t *>(p.k_cache)) + (int64_t)blk * p.k_stride_block +
-                      (int64_t)inpage * p.k_stride_row;
-        const float scale = quantise_row<T>(src, dst, kMlaDqk);
-        if ((threadIdx.x & 63) == 0) {
-            const int64_t so = (int64_t)blk * p.ks_stride_block + (int64_t)inpage * p.ks_stride_row;
-            const_cast<float *>(p.k_scale)[so] = scale;
-            if (p.v_scale != p.k_scale) const_cast<float *>(p.v_scale)[so] = scale;
-        }
-    }
-    __threadfence_block();
-    __syncthreads();   // every wave of the workgroup loads these rows next
-}
-
-// APPEND is a kernel of its own: the code costs the main loop 2 % where it never runs (registers).
-template <typename T, bool SOFTCAP, bool APPEND>
+template <typename T, bool SOFTCAP>
 __global__ void __launch_bounds__(kMlaThreads) decode_mla_i8_kernel(const DecodeParams p) {
     __shared__ MlaShared sh;
     // Neighbouring shares are mostly pieces of one batch row and read the same 147 KB of Q.  Workgroup x runs on XCD
@@ -868,9 +840,6 @@ __global__ void __launch_bounds__(kMlaThreads) decode_mla_i8_kernel(const Decode
     const int G = gridDim.x;
     const int worker = (G & 7) ? (int)blockIdx.x : (int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3);
     balanced_driver<kMlaDv, true>(p, worker, [&](int b, int unit, const UnitRange &ur, int range_lo, int range_hi, bool whole, int64_t slot) {
-        if constexpr (APPEND) {
-            if (range_hi > ur.len_cache) append_latent_rows<T>(p, b, ur.len_cache, range_lo, range_hi);   // workgroup-uniform
-        }
         mla_piece<T, SOFTCAP>(p, b, unit, ur, range_lo, range_hi, whole, slot, sh);
     });
 }
@@ -880,18 +849,18 @@ hipError_t launch_decode_mla_i8(const DecodeParams &p, int dtype, hipStream_t st
     if (p.units_per_token <= 0 || p.rows != kMlaUnitHeads || p.group != kMlaUnitHeads || !p.balanced)
         return hipErrorInvalidValue;
     dim3 grid(p.num_wgs), block(kMlaThreads);
-    auto go = [&](auto t, auto softcap_c) {
-        using T = decltype(t);
-        constexpr bool kCap = decltype(softcap_c)::value;
-        if (p.k_new)
-            hipLaunchKernelGGL((decode_mla_i8_kernel<T, kCap, true>), grid, block, 0, stream, p);
+    const bool softcap = p.softcap_post != 0.f;
+    if (dtype == 0) {
+        if (softcap)
+            hipLaunchKernelGGL((decode_mla_i8_kernel<BF16, true>), grid, block, 0, stream, p);
         else
-            hipLaunchKernelGGL((decode_mla_i8_kernel<T, kCap, false>), grid, block, 0, stream, p);
-    };
-    auto pick = [&](auto t) {
-        if (p.softcap_post != 0.f) go(t, std::true_type{}); else go(t, std::false_type{});
-    };
-    if (dtype == 0) pick(BF16{}); else pick(FP16{});
+            hipLaunchKernelGGL((decode_mla_i8_kernel<BF16, false>), grid, block, 0, stream, p);
+    } else {
+        if (softcap)
+            hipLaunchKernelGGL((decode_mla_i8_kernel<FP16, true>), grid, block, 0, stream, p);
+        else
+            hipLaunchKernelGGL((decode_mla_i8_kernel<FP16, false>), grid, block, 0, stream, p);
+    }
     return hipGetLastError();
 }
 

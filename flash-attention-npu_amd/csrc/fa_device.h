@@ -129,23 +129,6 @@ __device__ __forceinline__ void rotate_pair(float x1, float x2, float c, float s
     r2 = e + f;
 }
 
-// One row of the int8 latent cache by one wave: symmetric codes of d columns, scale = absmax / 127 (the return value, the
-// same in every lane).  Each step is a single correctly rounded fp32 operation, so codes and scale are defined to the bit.
-template <typename T> __device__ __forceinline__ float quantise_row(const uint16_t *src, int8_t *dst, int d) {
-    const int lane = threadIdx.x & 63;
-    float absmax = 0.f;
-    for (int e = lane; e < d; e += 64) absmax = fmaxf(absmax, fabsf(to_float<T>(src[e])));
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) absmax = fmaxf(absmax, __shfl_xor(absmax, m, 64));
-    const float scale = __fdiv_rn(absmax, 127.0f);
-    for (int e = lane; e < d; e += 64) {
-        float c = 0.f;
-        if (scale > 0.f) c = fminf(fmaxf(rintf(__fdiv_rn(to_float<T>(src[e]), scale)), -127.f), 127.f);
-        dst[e] = (int8_t)(int)c;
-    }
-    return scale;
-}
-
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 

@@ -774,10 +774,7 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
     // (and so owned by exactly one wave): causal or no right bound, and no left bound that could
     // exclude the oldest new key.  Otherwise the rows are written by their own kernel first.
     // With row tiles several waves read every chunk and only one of them would write the row: no fusion.
-    // The latent kernel does the same for its quantised rows where a batch row is one unit, i.e. one reader of every chunk.
-    const bool fuse_append = is_mla_i8(a) ? a->k_new && a->seqlen_q == 1 && a->nheads <= 128 && (a->causal || a->window_right < 0) &&
-                                                (a->window_left < 0 || (int64_t)1 + a->window_left >= a->seqlen_new) && !env().separate_append
-                                          : a->k_new && (p.balanced || p.unit_waves > 0) && p.wave_workers && row_tiles <= 1 && (a->causal || a->window_right < 0) &&
+    const bool fuse_append = a->k_new && (p.balanced || p.unit_waves > 0) && p.wave_workers && row_tiles <= 1 && (a->causal || a->window_right < 0) &&
                              (a->window_left < 0 || (int64_t)a->seqlen_q + a->window_left >= a->seqlen_new) &&
                              !env().separate_append;
     if (fuse_append) {
