@@ -18,6 +18,7 @@ hipError_t launch_append_quant_i8(const AppendParams &, int, hipStream_t) { retu
 hipError_t launch_rotate_q(const RotateQParams &, int, hipStream_t) { return hipErrorNotSupported; }
 hipError_t launch_decode_paged(const DecodeParams &, int, int, hipStream_t) { return hipErrorNotSupported; }
 hipError_t launch_decode_wave(const DecodeParams &, int, int, hipStream_t) { return hipErrorNotSupported; }
+hipError_t launch_decode_unit(const DecodeParams &, int, int, hipStream_t) { return hipErrorNotSupported; }
 hipError_t launch_splitkv_combine(const DecodeParams &, int, int, hipStream_t) { return hipErrorNotSupported; }
 hipError_t launch_decode_mla_i8(const DecodeParams &, int, hipStream_t) { return hipErrorNotSupported; }
 hipError_t launch_prefill(const PrefillParams &, int, int, hipStream_t) { return hipErrorNotSupported; }
