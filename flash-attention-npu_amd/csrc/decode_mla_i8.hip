@@ -183,13 +183,14 @@ struct MlaShared {
     struct __attribute__((aligned(16))) Scales {                 // per-token scales of a tile, side by side: one LDS base address
         float ksl[kChunk];                                       // key-side scale x softmax scale (log2 units)
         float vs[kChunk];                                        // V-side scale
-        float vsi[kChunk];                                       // its inverse (0 for a zero scale)
+        float vsi[kChunk];                                       // its inverse (0: weightless, see stash_scales)
         uint16_t vsi_hi[kChunk];                                 // the inverse as two bf16 terms (hi + lo), for v_dot2_f32_bf16
         uint16_t vsi_lo[kChunk];
     } sc[3];
     __attribute__((aligned(16))) u32x4_t pk[2][4][2][64];        // P^T operands: [chunk parity][head group][k-step][lane]
     float alpha[2][kMlaUnitHeads];                               // accumulator rescale per head (slow path only)
     __attribute__((aligned(16))) int32_t moved[2][4];                                         // head group moved its reference in this chunk
+    float xmax0[4];                                              // what the maximum over a tile's scores starts from: +inf if it holds a weightless key
     float l[kMlaUnitHeads];                                      // final normaliser per head
     __attribute__((aligned(16))) u32x4_t q[4][kMlaQLds][64];     // Q^T operands of the last k-steps: [wave][k-step][lane]
     __attribute__((aligned(16))) uint8_t k[3][kMlaTileBytes];   // widened key tiles
@@ -362,11 +363,17 @@ __device__ __forceinline__ void mla_piece(const DecodeParams &p, const int b, co
             if (q == 3) *reinterpret_cast<u32x4_t *>(&sh.k[tile][st_off + i * 128]) = wide;
         }
     };
+    // A key whose V-side scale is zero (an all-zero token: the append writes it so), or below what the I/O type holds of a
+    // weight times it, is weightless: its products with P vanish, and so would its share of the normaliser, which sums the
+    // rounded products times the inverse scale.  softmax_check adds the exponential itself there.
+    constexpr float kLeastScale = __is_same(T, BF16) ? 1.17549435e-38f : 5.9604645e-8f;   // 2^-126, 2^-24
     auto stash_scales = [&](int tile) {
         if (tid < kChunk) {
             sh.sc[tile].ksl[tid] = st_ks * (SOFTCAP ? p.softcap_pre : p.scale_log2);
             sh.sc[tile].vs[tid] = st_vs;
-            const float inv = (st_vs > 0.f) ? __builtin_amdgcn_rcpf(st_vs) : 0.f;
+            const bool weightless = !(st_vs >= kLeastScale);
+            const float inv = weightless ? 0.f : __builtin_amdgcn_rcpf(st_vs);
+            sh.xmax0[tile] = __any(weightless) ? INFINITY : -INFINITY;   // (the same from every lane)
             sh.sc[tile].vsi[tid] = inv;
             const uint16_t hi = from_float<BF16>(inv);
             sh.sc[tile].vsi_hi[tid] = hi;
@@ -439,7 +446,7 @@ __device__ __forceinline__ void mla_piece(const DecodeParams &p, const int b, co
     auto load_vsi_lo = [&](int tile, int g) { return *reinterpret_cast<const uint2 *>(&sh.sc[tile].vsi_lo[4 * lh + 8 * g]); };
     // scores in log2 units RELATIVE TO THE STANDING REFERENCE, in place, and their maximum (registers 4g .. 4g+3): the
     // subtraction rides in the scaling's fused multiply-add, and the common chunk exponentiates what it finds here
-    float xmax = -INFINITY;
+    float xmax;   // starts from sh.xmax0[tile]
     auto softmax_scale4 = [&](int g, const float4 &kq) {
         const float kv[4] = {kq.x, kq.y, kq.z, kq.w};
         const float m_std = (m_ref == -INFINITY) ? 0.f : m_ref;
@@ -461,9 +468,9 @@ __device__ __forceinline__ void mla_piece(const DecodeParams &p, const int b, co
         }
     };
     // The common chunk keeps the standing reference.  Anything else (the first chunk: the reference is -inf; a maximum
-    // beyond the lazy bound; a chunk with masked keys) goes through here: masks, a moved reference, the rescale
+    // beyond the lazy bound; a chunk with masked or weightless keys) goes through here: masks, a moved reference, the rescale
     // factors for the column owners; the scores are then re-expressed relative to the reference the exponentials use.
-    auto softmax_check = [&](int j) {
+    auto softmax_check = [&](int j, int tile) {
         const int pb = j & 1;
         const int key0 = (c_begin + j) * kChunk;
         const bool edge = key0 < mask_lo || key0 + kChunk > mask_hi;   // wave-uniform
@@ -491,9 +498,13 @@ __device__ __forceinline__ void mla_piece(const DecodeParams &p, const int b, co
             const float m_use = (m_ref == -INFINITY) ? 0.f : m_ref;
 #pragma unroll
             for (int r = 0; r < 16; ++r) s_acc[r] -= m_use;
+            if (__any(xmax == INFINITY)) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    if (sh.sc[tile].vsi[8 * (r >> 2) + 4 * lh + (r & 3)] == 0.f) l_norm += fast_exp2(s_acc[r]);
+            }
         }
         if (lane == 0) sh.moved[pb][wave] = moved;
-        xmax = -INFINITY;
     };
     // exponentials (registers 4g .. 4g+3)
     auto softmax_exp4 = [&](int g) {
@@ -625,7 +636,10 @@ __device__ __forceinline__ void mla_piece(const DecodeParams &p, const int b, co
             va[0] = read_va(tb0, 0);
             va[1] = read_va(tb0, 1);
         }
-        if constexpr (SM) sc0 = load_ksl(tile_sm, 0);
+        if constexpr (SM) {
+            xmax = sh.xmax0[tile_sm];
+            sc0 = load_ksl(tile_sm, 0);
+        }
         // quarter 0: half 0, column tiles 0 and 1; scaled scores and their maximum
         static_for<0, 8>([&](auto slot_) {
             constexpr int slot = decltype(slot_)::value;
@@ -644,7 +658,7 @@ __device__ __forceinline__ void mla_piece(const DecodeParams &p, const int b, co
             __builtin_amdgcn_sched_barrier(0);
         });
         if constexpr (SM) {
-            softmax_check(j_sm);
+            softmax_check(j_sm, tile_sm);
             sc1 = load_vs(tile_sm, 0);
             if constexpr (__is_same(T, BF16)) {
                 sh2 = load_vsi_hi(tile_sm, 0);

@@ -87,6 +87,37 @@ def test_mla_ragged_and_empty():
     check_out(got[0], ref[0], got[1], ref[1], "mla ragged")
 
 
+@pytest.mark.parametrize("dtype,softcap", [(torch.bfloat16, 0.0), (torch.float16, 0.0), (torch.bfloat16, 15.0)])
+@pytest.mark.parametrize("stored", ["zero", "zero scale", "tiny"])
+def test_mla_weightless_tokens(stored, dtype, softcap):
+    """Tokens whose scale is zero (all-zero rows; the codes may be anything then), or too small for the I/O type to hold a
+    weight times it, add nothing to the output but count in the softmax like any other key."""
+    lens = [31, 40, 300, 64, 1]
+    case = mla_case(len(lens), 128, lens, page=64, seed=12)
+    case["q"] = (case["q"] * 0.2).to(dtype)                       # no key outweighs the others
+    for b, n in enumerate(lens):
+        for at in range(0, n, 3):
+            blk = case["block_table"][b, at // 64]
+            case["k_scale"][blk, at % 64] = 0.0 if stored != "tiny" else 1e-9 if dtype is torch.float16 else 1e-39
+            if stored == "zero":
+                case["k_cache"][blk, at % 64] = 0
+    from flash_attn_npu import flash_attn_with_kvcache
+    kc = case["k_cache"].cuda()
+    out, lse = flash_attn_with_kvcache(case["q"].cuda(), kc, kc[..., :512], cache_seqlens=case["cache_seqlens"].cuda(), softcap=softcap,
+                                       block_table=case["block_table"].cuda(), softmax_scale=192 ** -0.5, causal=True,
+                                       return_softmax_lse=True, k_scale_cache=case["k_scale"].cuda())
+    torch.cuda.synchronize()
+    ref, ref_lse = O.flash_attn_with_kvcache(case["q"], case["k_cache"], case["k_cache"][..., :512], cache_seqlens=case["cache_seqlens"],
+                                             block_table=case["block_table"], softmax_scale=192 ** -0.5, causal=True, softcap=softcap,
+                                             k_scale_cache=case["k_scale"], mode="fp32")
+    out = out.float().cpu()
+    # weights and results are rounded to the I/O type (bf16: 2^-9 each), partial rows to fp16 (2^-12)
+    for b in range(len(lens) - 1):
+        assert ((out[b] - ref[b]).norm() / ref[b].norm()).item() <= 6e-3, (stored, b)
+    assert (out[-1].abs().max() <= (1e-6 if dtype is torch.float16 else 1e-30)).item()     # its only key has no weight at all
+    torch.testing.assert_close(lse.cpu(), ref_lse, rtol=1e-3, atol=1e-3)
+
+
 def test_mla_codes_and_scales_untouched():
     case = mla_case(2, 128, [900, 300], seed=3)
     from flash_attn_npu import flash_attn_with_kvcache
