@@ -73,15 +73,19 @@ __device__ __forceinline__ int unit_cost(int nchunks, int cost, int align) {
 
 // exclusive prefixes over 256 equal segments of the batch: s_pref[t] = chunks of rows [0, t*seg),
 // s_cnt[t] = rows among them with a visible key; [256] = totals.  All threads of the block must call
-// (256 or more threads; the first 256 do the work).  Returns whether some batch row has no visible key.
-__device__ __forceinline__ bool batch_chunk_prefix(const DecodeParams &p, int *s_pref, int *s_cnt, int seg, int M) {
+// (256 or more threads; the first 256 do the work).  Returns whether some batch row has no visible key; LATENT (256 threads):
+// in bit 1, whether one has at most kWholeLatentChunks chunks (and a key), from the same pass over the lengths.
+constexpr int kWholeLatentChunks = 4;
+template <bool LATENT = false> __device__ __forceinline__ int batch_chunk_prefix(const DecodeParams &p, int *s_pref, int *s_cnt, int seg, int M) {
     __shared__ int s_wave[4], s_wave_cnt[4];
     const int tid = threadIdx.x;
     int sum = 0, cnt = 0;
+    bool short_row = false;
     for (int b = tid * seg; b < min(p.batch, (tid + 1) * seg); ++b) {
         const int n = unit_range(p, b, M).nchunks;
         sum += n;
         cnt += (n > 0);
+        short_row |= n > 0 && n <= kWholeLatentChunks;
     }
     const bool empty_row = tid * seg < p.batch && cnt < min(p.batch, (tid + 1) * seg) - tid * seg;
     int inc = sum, inc_cnt = cnt;
@@ -98,7 +102,16 @@ __device__ __forceinline__ bool batch_chunk_prefix(const DecodeParams &p, int *s
         s_wave[tid >> 6] = inc;
         s_wave_cnt[tid >> 6] = inc_cnt;
     }
-    const bool any_empty = __syncthreads_or(empty_row ? 1 : 0) != 0;
+    int votes = 0;
+    if constexpr (LATENT) {
+        __shared__ int s_votes[4];
+        votes = (__any(empty_row) ? 1 : 0) | (__any(short_row) ? 2 : 0);
+        if ((tid & 63) == 0) s_votes[tid >> 6] = votes;
+        __syncthreads();
+        votes = s_votes[0] | s_votes[1] | s_votes[2] | s_votes[3];
+    } else {
+        votes = __syncthreads_or(empty_row ? 1 : 0) != 0;
+    }
     if (tid < 256) {
         int base = 0, base_cnt = 0;
         for (int w = 0; w < (tid >> 6); ++w) {
@@ -110,7 +123,7 @@ __device__ __forceinline__ bool batch_chunk_prefix(const DecodeParams &p, int *s
     }
     if (tid == 0) s_pref[0] = s_cnt[0] = 0;
     __syncthreads();
-    return any_empty;
+    return votes;
 }
 
 // Query token and query head of row `row` of unit `kvh` of a batch row.  Ordinary caches: the unit
@@ -302,19 +315,31 @@ struct Partition {
     }
 };
 
+// Least share of the latent kernel: p.min_share (4 chunks), or p.min_share_short (2) where the units are of middling length.
+// A unit of at most kWholeLatentChunks chunks is never cut for it: whole, it is written straight from the fp32
+// accumulators; its pieces would be rounded to fp16 and clamped to that type's range.  Longer units are cut either way.
+// One sequence, whole call with shares of 2 / 4 chunks: 2048 keys 28.8 / 30.6 us, 4096 30.4 / 32.7, 8192 (twice the
+// partials to merge) 36.7 / 35.0: kLongLatentUnitChunks lies between the last two.
+constexpr int kLongLatentUnitChunks = 192;
+__device__ __forceinline__ int latent_least_share(const DecodeParams &p, const Partition &pt, const int *s_pref, int units, bool short_rows) {
+    // (more rows than prefix segments: the merge kernel works the partition out again, by the common rule)
+    const bool middling = pt.seg == 1 && !short_rows && pt.cost == 0 && s_pref[256] < (int64_t)kLongLatentUnitChunks * units;
+    return p.min_share_short > 0 && middling ? p.min_share_short : p.min_share;
+}
+
 // A share that holds the end of one unit and the start of the next pays the fixed cost of a piece (lengths -> table ->
 // keys, q rows, stores: ~12 us of a workgroup of the latent kernel) twice, and the launch lasts as long as its slowest
 // worker.  With shares of a few chunks (~2 us each) that is most of the launch, so the units are padded to multiples of
-// the share there, if the device has workers enough for it at the same share or one up to p.align_slack chunks longer;
-// long shares are left as they are (a longer one would cost more than the second start).
-// Latent kernel, whole call, shares that cross units / aligned: 3 sequences of 916..2489 keys 47.1 / 39.1 us, 8 of
-// 1000..10000 52.4 / 44.5, 64 of 300..3000 83.5 / 62.9 (85.0 without a longer share); one sequence 24.9 / 27.1 (nothing to
+// the share there, if the device has workers enough for it at the same share or one up to two chunks longer; long shares
+// are left as they are (a longer one would cost more than the second start).
+// Latent kernel, whole call, shares that cross units / aligned: 3 sequences of 916..2489 keys 44.5 / 31.8 us, 8 of
+// 1000..10000 52.5 / 44.1, 64 of 300..3000 80.1 / 62.5 (80 without a longer share); one sequence 24.9 / 27.1 (nothing to
 // cross: the host leaves it off).  The wave-level kernel, whose pieces start in ~6 us, gains nothing: 4 sequences x 8 kv
 // heads x 4096 visible keys 27.1 / 29.1, 8 x 4 heads x 2000..20000 keys 44.9 / 45.8.
-constexpr int kAlignTries = 4, kAlignMaxShare = 16;
+constexpr int kAlignTries = 3, kAlignMaxShare = 16;
 __device__ __forceinline__ void align_partition(const DecodeParams &p, Partition &pt, int *s_pref, int64_t shares) {
     __shared__ int s_need[4][kAlignTries], s_sum[4];
-    if (pt.seg != 1 || pt.cost != 0 || p.align_slack < 0 || pt.S > kAlignMaxShare) return;   // the same in every thread
+    if (!p.align_units || pt.seg != 1 || pt.cost != 0 || pt.S > kAlignMaxShare) return;   // the same in every thread
     const int tid = threadIdx.x, S0 = (int)pt.S;
     const int n = tid < 256 ? s_pref[tid + 1] - s_pref[tid] : 0;   // this batch row's chunks
     int need[kAlignTries];
@@ -330,7 +355,7 @@ __device__ __forceinline__ void align_partition(const DecodeParams &p, Partition
 #pragma unroll
     for (int i = kAlignTries - 1; i >= 0; --i) {
         const int64_t all = (int64_t)(s_need[0][i] + s_need[1][i] + s_need[2][i] + s_need[3][i]) * pt.list_heads;
-        if (i <= p.align_slack && all <= shares) S = S0 + i;
+        if (all <= shares) S = S0 + i;
     }
     if (S == 0) return;
     int inc = unit_cost(n, 0, S);
@@ -352,14 +377,15 @@ __device__ __forceinline__ void align_partition(const DecodeParams &p, Partition
 }
 
 // Block-level (256 threads, contains barriers): prefix sums into s_pref[257], share size for
-// p.num_workers workers (never below p.min_share chunks).
-// ALIGN: shares of a few chunks may be aligned to the units (align_partition); batches of more than 256 rows never are.
-template <bool ALIGN = false> __device__ __forceinline__ Partition make_partition(const DecodeParams &p, int *s_pref) {
+// p.num_workers workers (never below p.min_share chunks; LATENT: latent_least_share()).
+// LATENT: shares of a few chunks may be aligned to the units (align_partition); batches of more than 256 rows never are.
+template <bool LATENT = false> __device__ __forceinline__ Partition make_partition(const DecodeParams &p, int *s_pref) {
     Partition pt;
     pt.seg = (p.batch + 255) / 256;
     pt.M = window_norm_m(p);
     __shared__ int s_cnt[257];
-    pt.any_empty = batch_chunk_prefix(p, s_pref, s_cnt, pt.seg, pt.M);
+    const int votes = batch_chunk_prefix<LATENT>(p, s_pref, s_cnt, pt.seg, pt.M);
+    pt.any_empty = (votes & 1) != 0;
     pt.list_heads = p.head_interleave ? 1 : p.nheads_k;
     const int64_t shares = p.head_interleave ? max(p.num_workers / p.nheads_k, 1) : p.num_workers;
     const int64_t chunks = (int64_t)s_pref[256] * pt.list_heads;
@@ -370,10 +396,27 @@ template <bool ALIGN = false> __device__ __forceinline__ Partition make_partitio
         __syncthreads();
     }
     pt.W = (int64_t)s_pref[256] * pt.list_heads;
-    const bool long_units = p.min_share_long > 0 && (int64_t)s_pref[256] >= (int64_t)p.long_unit_chunks * max(s_cnt[256], 1) + (int64_t)pt.cost * s_cnt[256];
-    pt.S = max((pt.W + shares - 1) / shares, (int64_t)max(long_units ? p.min_share_long : p.min_share, 1));
+    int least;
+    if constexpr (LATENT) {
+        least = latent_least_share(p, pt, s_pref, s_cnt[256], (votes & 2) != 0);
+    } else {
+        const bool long_units = p.min_share_long > 0 && (int64_t)s_pref[256] >= (int64_t)kLongUnitChunks * max(s_cnt[256], 1) + (int64_t)pt.cost * s_cnt[256];
+        least = long_units ? p.min_share_long : p.min_share;
+    }
+    pt.S = max((pt.W + shares - 1) / shares, (int64_t)max(least, 1));
     pt.align = 1;
-    if constexpr (ALIGN) align_partition(p, pt, s_pref, shares);
+    if constexpr (LATENT) {
+        align_partition(p, pt, s_pref, shares);
+        // the same in every lane, which the compiler cannot see behind the votes and LDS reads: vector registers are what
+        // the latent kernel is short of
+        auto uniform = [](int64_t x) -> int64_t {
+            return ((int64_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+        };
+        pt.S = uniform(pt.S);
+        pt.W = uniform(pt.W);
+        pt.align = __builtin_amdgcn_readfirstlane(pt.align);
+        pt.cost = __builtin_amdgcn_readfirstlane(pt.cost);
+    }
     return pt;
 }
 
@@ -490,10 +533,10 @@ template <int DV> __device__ __forceinline__ void init_empty_units(const DecodeP
 }
 
 // Workgroup-level worker: the share `worker` (a permutation of the workgroup numbers), then the empty-unit duty.
-template <int DV, bool ALIGN = false, typename PieceFn>
+template <int DV, bool LATENT = false, typename PieceFn>
 __device__ __forceinline__ void balanced_driver(const DecodeParams &p, int worker, PieceFn piece) {
     __shared__ int s_pref[257];
-    const Partition pt = make_partition<ALIGN>(p, s_pref);
+    const Partition pt = make_partition<LATENT>(p, s_pref);
     publish_partition(p, pt, s_pref);
     walk_share(p, pt, s_pref, worker, piece);
     init_empty_units<DV>(p, pt);

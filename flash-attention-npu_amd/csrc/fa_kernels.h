@@ -49,8 +49,9 @@ struct DecodeParams {
     int32_t nsplits, split_keys;   // grid mode: split slots per unit, keys per split
     int32_t balanced, num_wgs;     // balanced mode: workgroups launched
     int32_t num_workers, min_share;  // workers sharing the chunk list (workgroups, or waves), least chunks per share
-    int32_t min_share_long, long_unit_chunks;   // > 0: the least share when the units have long_unit_chunks chunks or more on average
-    int32_t align_slack;             // balanced mode: how many chunks longer a share may become so that none crosses units (-1: never)
+    int32_t min_share_long;          // > 0: the least share when the units are long (kLongUnitChunks chunks on average)
+    int32_t min_share_short;         // latent kernel, > 0: the least share when the units are of middling length (decode_common.h)
+    int32_t align_units;             // latent kernel, 1: shares of a few chunks may be aligned to the units (decode_common.h)
     int32_t wave_workers;          // 1: every wave is a worker (num_workers = 4 * num_wgs)
     int32_t head_interleave;       // 1: worker w streams share w / Hk of the per-head list for kv head w % Hk
     int32_t piece_cost;            // balanced mode: list length charged for starting on a unit, in chunks (decode_common.h)
@@ -179,9 +180,6 @@ constexpr bool partials_are_half(int dv) { return dv == 512; }
 // short units (64 x 8 heads x 8 chunks) go the other way (28.8 against 33.4 us).  The lengths live on the device, so
 // the choice is made there.
 constexpr int kLongUnitChunks = 64;
-// Latent kernel, one sequence, whole call with shares of 2 / 4 chunks: 2048 keys 28.8 / 30.6 us, 4096 30.4 / 32.7, 8192
-// (twice the partials to merge) 36.7 / 35.0.
-constexpr int kLongLatentUnitChunks = 192;
 constexpr int kPartitionHeaderInts = 8;                 // M, cost, W (2), S (2), align, 1 spare; then prefix[0 .. batch]
 constexpr size_t kPartitionHeaderBytes = 2048;          // 8 + 257 ints, rounded up
 

@@ -420,9 +420,8 @@ int fa_rocm_plan_kvcache(const fa_kvcache_args *a, int num_cus, fa_split_plan *p
         const int per_cu = is_mla_i8(a) ? 1 : fa::decode_wgs_per_cu(a->headdim_qk, wave_workers ? 16 : (int)rows);
         plan->num_wgs = num_cus * per_cu;
         // latent kernel: a piece costs ~12 us of pipeline fill and a 131 KB partial, so tiny launches are not cut below
-        // 2 chunks per workgroup (1 sequence x 4096 tokens: 34.8 us with 1, 30.4 with 2, 32.7 with 4), long units not
-        // below 4 (fa::kLongLatentUnitChunks)
-        plan->min_share = is_mla_i8(a) ? 2 : 1;
+        // 4 chunks per workgroup (1 sequence x 8 K tokens: 46 -> 37 us); down to 2 where the lengths on the device allow it
+        plan->min_share = is_mla_i8(a) ? 4 : 1;
         // tuning aid: FA_ROCM_DECODE_WGS overrides the workgroup count of the balanced partition
         if (env().decode_wgs > 0) plan->num_wgs = env().decode_wgs;
         plan->num_workers = wave_workers ? plan->num_wgs * 4 : plan->num_wgs;
@@ -742,8 +741,8 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
     p.min_share = plan.min_share;
     p.wave_workers = waves_of_unit > 0 || plan.num_workers != plan.num_wgs;
     p.unit_waves = waves_of_unit;
-    p.min_share_long = ((p.wave_workers || is_mla_i8(a)) && env().min_share <= 0) ? 4 : 0;
-    p.long_unit_chunks = is_mla_i8(a) ? fa::kLongLatentUnitChunks : fa::kLongUnitChunks;
+    p.min_share_long = (p.wave_workers && env().min_share <= 0) ? 4 : 0;
+    p.min_share_short = (is_mla_i8(a) && env().min_share <= 0) ? 2 : 0;
     // wave workers of neighbouring kv heads walk the same token range together
     // Fixed cost of starting on a unit, in chunk times.  Latent kernel: ~15 us of q staging and pipeline
     // fill against ~2 us per chunk; charging 7 chunks takes the workgroups that start a second unit off
@@ -796,7 +795,7 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
     if (is_mla_i8(a)) {
         p.units_per_token = (a->nheads + 127) / 128;      // 128-head groups (the last one may be partly empty)
         p.nheads_k = a->seqlen_q * p.units_per_token;     // units per batch row
-        p.align_slack = (int64_t)a->batch * p.nheads_k > 1 ? 2 : -1;   // (one unit: no share can cross into another)
+        p.align_units = (int64_t)a->batch * p.nheads_k > 1;   // (one unit: no share can cross into another)
         p.group = 128;
         p.rows = 128;
         e = fa::launch_decode_mla_i8(p, a->io_dtype, stream);
