@@ -327,11 +327,20 @@ __device__ __forceinline__ int latent_least_share(const DecodeParams &p, const P
     return p.min_share_short > 0 && middling ? p.min_share_short : p.min_share;
 }
 
+// Whether `pred` holds for some batch row's chunks (one row per prefix segment).  Every wave looks at all the rows: a vote of
+// the workgroup would cost three barriers.
+template <typename Pred> __device__ __forceinline__ bool any_row(const DecodeParams &p, const int *s_pref, Pred pred) {
+    bool any = false;
+    for (int b = threadIdx.x & 63; b < p.batch; b += 64) any |= pred(s_pref[b + 1] - s_pref[b]);
+    return __any(any);
+}
+
 // A share that holds the end of one unit and the start of the next pays the fixed cost of a piece (lengths -> table ->
 // keys, q rows, stores: ~12 us of a workgroup of the latent kernel) twice, and the launch lasts as long as its slowest
 // worker.  With shares of a few chunks (~2 us each) that is most of the launch, so the units are padded to multiples of
 // the share there, if the device has workers enough for it at the same share or one up to two chunks longer; long shares
-// are left as they are (a longer one would cost more than the second start).
+// are left as they are (a longer one would cost more than the second start), and so is a batch in which no share crosses
+// units as it is (the search below takes ~2 us).
 // Latent kernel, whole call, shares that cross units / aligned: 3 sequences of 916..2489 keys 44.5 / 31.8 us, 8 of
 // 1000..10000 52.5 / 44.1, 64 of 300..3000 80.1 / 62.5 (80 without a longer share); one sequence 24.9 / 27.1 (nothing to
 // cross: the host leaves it off).  The wave-level kernel, whose pieces start in ~6 us, gains nothing: 4 sequences x 8 kv
@@ -342,6 +351,7 @@ __device__ __forceinline__ void align_partition(const DecodeParams &p, Partition
     if (!p.align_units || pt.seg != 1 || pt.cost != 0 || pt.S > kAlignMaxShare) return;   // the same in every thread
     const int tid = threadIdx.x, S0 = (int)pt.S;
     const int n = tid < 256 ? s_pref[tid + 1] - s_pref[tid] : 0;   // this batch row's chunks
+    if (!any_row(p, s_pref, [&](int m) { return m % S0 != 0; })) return;
     int need[kAlignTries];
 #pragma unroll
     for (int i = 0; i < kAlignTries; ++i) {
