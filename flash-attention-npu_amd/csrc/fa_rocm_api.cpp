@@ -231,18 +231,30 @@ int64_t live_keys_bound(const fa_kvcache_args *a) {
 // units are cut over the device instead.
 // The partition over the device costs ~10 us whatever the work: the lengths' prefix pass, partials of every wave, a merge
 // launch.  A workgroup per unit costs ~6 us and ~2.6 us per chunk of its longest wave (one chunk of a wave is in flight, a
-// trip to memory each), so it is ahead while the longest unit is short, and for longer ones where there are units enough to
-// keep every compute unit busy; the host knows the longest unit's bound, the keys that the table or the window allows.
-// Whole call in us, partition / workgroup per unit, 4 q heads per kv head, all units of the stated keys unless a range:
-//   D = 128:  8 units x 512 keys 16.5 / 10.1, x 1024 16.6 / 16.1, x 2048 20.7 / 27.4;  64 x 1024 21.5 / 18.1, x 2048 27.9 / 30.1
-//             128 x 1500 34.2 / 26.2, x 200..2000 31.3 / 28.8, x 400..4000 41.4 / 50.9;  320 x 200..2000 45.9 / 45.5, x 400..4000 70.9 / 83.8
-//             1024 x 128 33.1 / 20.3, x 200..2048 115.9 / 111.0;  2048 x 128 36.8 / 37.2, x 512 96.6 / 91.9;  4096 x 128 63.2 / 70.2
-//   D = 64:   256 x 1024 30.9 / 16.8;  2048 x 512 55.2 / 52.4;  6400 x 40 49.6 / 45.1, x 512 154.1 / 151.2
-//   D = 256:  8 x 512 21.2 / 19.1, x 1024 21.1 / 29.4;  256 x 2048 99.9 / 81.1;  512 x 2048 180.1 / 162.1;  1024 x 128 38.8 / 48.8
-//   17-32 rows, D = 128, against the tiled kernel or two tiles per wave:  16 units x 700 22.1 / 18.7, x 1000 24.3 / 26.4
-//             64 x 8000 68.7 / 101.7;  128 x 300..3000 52.9 / 47.9;  192 x 1000 47.2 / 31.8, x 400..4000 84.8 / 65.2, x 8000 240 / 136
-//             256 x 800..8000 152 / 133;  512 x 400..4000 140 / 132;  1024 x 2048 227 / 191;  2048 x 128 52.9 / 67.0
-// Workgroups of 8 waves up to one per compute unit, of 4 beyond (512 units x 512 keys 29.6 with 8, 26.0 with 4).
+// trip to memory each), and cannot be cut: the lengths are on the device, so whatever the host admits has to hold for any
+// of them, for one long row among short ones (only its workgroups still run) as for equal rows.  The host knows two things:
+// the most keys a unit can have (what the table or the window allows), and whether the workgroups all run at once.
+//   * All at once: a compute unit holds two workgroups of 4 waves at D = 128, one at 256, four at 64 (two of 8 up to 16
+//     rows); 8 waves where they fit.  Whole call at the limits below, workgroup per unit over partition, the worst and the
+//     best of: equal rows, one or two long ones, every tenth, every second, lengths spread over a factor of ten; and the worst
+//     one step further:
+//       D = 128, 8 waves, 1024 keys: 0.73-0.93 (8 units 16.6 -> 12.6 us, 256 of one long row 17.5 -> 15.2); 1536: 1.23
+//       D = 128, 4 waves, 768: 0.69-1.02 (512 units of one long row 17.8 -> 16.5); 1024: 1.17;  768 units x 768: 1.18
+//       D = 64, 8 waves, 1024: 0.47-0.84;  4 waves, 1024: 0.58-1.00 (640 units of 33..900: 31.1 -> 20.7); 2048: 1.47
+//       D = 256, 4 waves, 512: 0.55-0.92; 768: 1.06, 264 units x 384: 1.21
+//       17-32 rows, D = 128, 768: 0.42-0.97; 1024: 1.15, 1024 units x 768: 1.40;  D = 64, 1024: 0.38-0.95
+//   * Several rounds, D = 64, up to 16 rows: 512 keys 0.62-0.98 (2048 units x 512 55.2 -> 52.4 us); 768: 1.04.  Wider rows
+//     lose from the second round on (D = 128, 1024 units, every tenth row of 512 keys among short ones: 1.17).
+//   * 17-32 rows at D = 128 with fewer units than compute units have the tiled kernel on the other side, which cuts a unit
+//     into 512 / units ranges.  From three quarters of the compute units on these are too few to outrun eight waves, whatever
+//     the lengths: 192 units x 8000 keys 236 -> 135 us, one long row 90.7 -> 78.7, every second 4096 63.4 -> 65.2; 176 units,
+//     every second 4096 60.3 -> 64.6, 160 units with one of 8000 1.25; 16000 keys, 192 units: 1.07; 256 units (two tiles per
+//     wave on the other side) with one of 8000: 2.05.  Only where the heads of a row take every XCD (workgroup x runs on XCD
+//     x % 8): with four heads a row, every second one long, half of the device is idle (192 units x 4096: 60.0 -> 67.1).
+//     Up to 128 keys the tiled kernel is ahead by 4-11 % unless q has to be rotated for it.
+//   * New keys of 17-32-row blocks: the wave that owns them writes them one after the other, ~0.65 us each, where the tiled
+//     kernel and the workgroup-level one (D = 64) have them written by a launch of ~5 us.  D = 128, 64 units x 768 keys, 5
+//     new 0.91, 8 new 1.07, 16 new 1.36, 32 new 1.91; D = 64, 8 units x 128 keys, 32 new 1.38.
 int unit_waves(const fa_kvcache_args *a, size_t rows, int num_cus) {
     const EnvKnobs &e = env();
     const int width = fa::tile_headdim(a->headdim_qk);
@@ -253,18 +265,19 @@ int unit_waves(const fa_kvcache_args *a, size_t rows, int num_cus) {
         e.no_head_interleave || e.separate_append)
         return 0;
     const int64_t units = (int64_t)a->batch * a->nheads_k, keys = live_keys_bound(a), cus = num_cus;
-    const bool few = units < cus / 2;
-    int64_t most;   // keys of the longest unit
-    if (width > 128)
-        most = units < cus ? 512 : units <= 2 * cus ? 2048 : 0;
-    else if (rows > 16)
-        most = few ? 768 : units <= 4 * cus ? (4 * units >= 3 * cus && units <= cus ? 8192 : 3072) : 0;
-    else if (units > 6 * cus)
-        most = (width == 64 ? units <= 32 * cus : units <= 8 * cus) ? 512 : 0;
-    else
-        most = few ? 1024 : 2048;
-    if (keys > most) return 0;
-    return width <= 128 && units <= cus && (rows <= 16 || keys > 512) ? 8 : 4;
+    const bool tall = rows > 16;
+    const int64_t held8 = width > 128 ? 0 : width == 64 && !tall ? 2 * cus : cus;   // workgroups that run at once, of 8 waves
+    const int64_t held4 = (width == 64 ? 4 : width == 128 ? 2 : 1) * cus;           // ... and of 4
+    if (units > held4) return width == 64 && !tall && units <= 32 * cus && keys <= 512 ? 4 : 0;
+    const int waves = units <= held8 ? 8 : 4;
+    int64_t most = width > 128 ? 512 : width == 64 || (waves == 8 && !tall) ? 1024 : 768;
+    const bool cut_appends = width == 128 && units >= cus;   // the kernel on the other side writes the new keys like this one
+    if (tall && !cut_appends && a->k_new && a->seqlen_new > 6) return 0;
+    if (width == 128 && tall && units < cus) {
+        if (4 * units >= 3 * cus && a->nheads_k % 8 == 0) most = 8192;
+        if (keys < 256 && !a->rotary_cos) return 0;
+    }
+    return keys <= most ? waves : 0;
 }
 
 }  // namespace
