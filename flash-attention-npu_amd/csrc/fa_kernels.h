@@ -143,7 +143,7 @@ struct PrefillParams {
     int32_t *list_state;
     int32_t list_wgs;
     int32_t num_mb, units8;        // set by the launcher: 128-row blocks per unit, units rounded up to 8
-    int32_t mb_run;                // set by the launcher: blocks of a unit that are neighbours in the launch order
+    int32_t mb_run;                // set by the launcher: tiles of a unit that are neighbours in the launch order
     int32_t seqlen_q_fixed, seqlen_k_add;   // kvcache layout: Sq per row, keys appended this call
     int32_t max_seqlen_q, total_q;
     int32_t page_size, max_blocks, num_blocks;
@@ -198,6 +198,69 @@ inline int prefill_pack(int group, int max_seqlen_q) {
     const int64_t tiles_plain = (int64_t)group * (((int64_t)max_seqlen_q + kPrefillTileRows - 1) / kPrefillTileRows);
     const int64_t tiles_packed = ((int64_t)max_seqlen_q * group + kPrefillTileRows - 1) / kPrefillTileRows;
     return tiles_packed * 4 <= tiles_plain * 3 ? group : 1;
+}
+// Causal launches that prefill_pack() leaves unpacked: whether the heads of a group share the tiles all the same.  The 128
+// rows of a tile are then 128 / group queries of all the heads rather than 128 queries of one, so that a tile's keys end
+// closer behind its queries (half a tile of hidden keys per row less at a group of 4) and short sequences fill their
+// tiles.  Unpacked / packed, in us: 80 x 3..350 tokens, 28q/4kv 91.1 / 74.3; 40 x 50..900, 28q/4kv 163.2 / 153.2; 16 x
+// 512..4096, 32q/8kv 796 / 761 (d = 64: 446.7 / 424.4); 64 x 512, 64q/32kv 583 / 570; 24 x 100..500, 16q/2kv, d = 256
+// 119.6 / 107.1.  Bidirectional launches gain nothing (30 x 100..900, 32q/8kv 218.3 / 219.8).  Nor do launches of less than
+// two rounds of the device, which last as long as their tallest tile either way (D = 128: 2 x 649 tokens, 32q/8kv 21.9 /
+// 23.0, 6 x 300..700, 16q/8kv 22.8 / 23.6); from there on the worst measured are 1-3 %
+// behind (4 x 2048, 24q/8kv 119.7 / 121.1; 12 x 100..500, 64q/32kv 60.6 / 62.3), and at D = 256 none is (20 x 200, 16q/2kv
+// 57.3 / 44.5; 12 x 100..500, 16q/8kv 53.2 / 51.2).
+inline bool prefill_pack_causal(int group, int nheads, int max_seqlen_q, int total_q) {
+    return group > 1 && group <= kPrefillTileRows && (int64_t)max_seqlen_q * group < (1ll << 30) &&
+           (int64_t)total_q * nheads >= 1024ll * kPrefillTileRows;
+}
+// Heads per tile, tiles of a unit that are neighbours in the launch order, tiles of a unit.  causal_packs: the launch may follow
+// prefill_pack_causal() (causal, no key ranges, no device-side list).
+struct PrefillTiles { int32_t pack, mb_run, num_mb; };
+inline PrefillTiles prefill_tiling(int group, int nheads, int max_seqlen_q, int total_q, bool causal_packs) {
+    PrefillTiles t = {prefill_pack(group, max_seqlen_q), 1, 0};
+    if (t.pack == 1 && causal_packs && prefill_pack_causal(group, nheads, max_seqlen_q, total_q)) t.pack = t.mb_run = group;
+    t.num_mb = (int32_t)(((int64_t)max_seqlen_q * t.pack + kPrefillTileRows - 1) / kPrefillTileRows);
+    return t;
+}
+// Tile of workgroup `bid` of the tiled forward.  Workgroup i of the 1-D grid runs on XCD i % 8.  The grid is ordered by
+// 128-row block, tallest first, and inside a block by position e: XCD lane e % 8 walks the units (sequence, key range, kv head)
+// congruent to it, the q heads of a unit one after the other.  Every XCD so gets the same mix of tall and short causal blocks
+// whatever the number of blocks is, and the heads that share a unit's K/V meet in one L2.
+// mb_run > 1 (causal launches with packed heads, heads_per_unit = 1): the mb_run = group tiles that hold 128 queries of all the
+// heads stand where the blocks of the single heads would.  They share their keys in an L2 like those, and in a batch whose
+// every other sequence is short the workgroups of an XCD, which go round its shader engines in launch order whether or not
+// they find anything to do, do not leave half of the engines idle.  Tile by tile the packed launch takes, of the unpacked
+// one's time: 8 x 512 + 8 x 3584 tokens, 32q/8kv 1.55 (in runs 0.99); 64 x 512 tokens, 64q/32kv 1.20 (0.98).
+struct PrefillPlace { int mb, unit, head; };
+__host__ __device__ inline PrefillPlace prefill_place(unsigned bid, int num_mb, int mb_run, int units8, int heads_per_unit) {
+    PrefillPlace r;
+    if (num_mb > 2 && mb_run > 1) {
+        const int top = num_mb % mb_run;                      // tiles of the last 128 queries, if they are not all there
+        const bool whole = bid >= (unsigned)(units8 * top);
+        const int run = whole ? mb_run : top;
+        const unsigned rest = whole ? bid - (unsigned)(units8 * top) : bid;
+        const int nth = (int)(rest / (unsigned)(units8 * run));
+        const int e = (int)(rest - (unsigned)nth * (unsigned)(units8 * run));
+        const int j = (e >> 3) / run;
+        r.unit = j * 8 + (e & 7);
+        r.head = 0;
+        r.mb = num_mb - 1 - (whole ? top + nth * run : 0) - ((e >> 3) - j * run);
+    } else if (num_mb > 2) {
+        const int per_block = units8 * heads_per_unit;
+        r.mb = num_mb - 1 - (int)(bid / per_block);
+        const int e = bid % per_block;
+        r.unit = ((e >> 3) / heads_per_unit) * 8 + (e & 7);
+        r.head = (e >> 3) % heads_per_unit;
+    } else {
+        // one or two blocks per unit (short sequences, all equally light): a unit's blocks stay
+        // neighbours in their XCD's queue, so its K/V are fetched into that L2 once
+        const int per_unit = num_mb * heads_per_unit;
+        const int q = bid >> 3;
+        r.unit = (q / per_unit) * 8 + (bid & 7);
+        r.head = (q % per_unit) / num_mb;
+        r.mb = num_mb - 1 - q % num_mb;
+    }
+    return r;
 }
 // 1 when the blocks of a token-major launch that does not pack (prefill_pack == 1) pack on their own where they are
 // short: blocks that differ in length and whose average would pack (mixed prefill / decode batches).

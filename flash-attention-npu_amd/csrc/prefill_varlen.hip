@@ -67,46 +67,13 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     const int ln = lane & 31;   // MFMA row / column
     const int hd = PART ? p.headdim : D;
 
-    // Workgroup i of the 1-D grid runs on XCD i % 8.  The grid is ordered by 128-row block, tallest
-    // first, and inside a block by position e: XCD lane e % 8 walks the units (sequence, key range,
-    // kv head) congruent to it, the q heads of a unit one after the other.  Every XCD so gets the same
-    // mix of tall and short causal blocks whatever the number of blocks is, and the heads that share
-    // a unit's K/V meet in one L2.
     const int nsplits = EXT ? max(p.nsplits, 1) : 1;
     const int heads_per_unit = (EXT && p.pack > 1) ? 1 : p.group;
     const bool listed = EXT && n_long >= 0;
     const int n_units = (listed ? n_long : p.batch) * nsplits * p.nheads_k;
     const int units8 = listed ? (n_units + 7) / 8 * 8 : p.units8;
-    int mb, unit, head_in_unit;
-    if (p.num_mb > 2) {
-        const int per_block = units8 * heads_per_unit;
-        if (EXT && p.mb_run > 1) {
-            // Packed heads (heads_per_unit = 1).  Inside an XCD the workgroups go round its shader engines in launch order,
-            // whether or not a workgroup finds anything to do.  With one workgroup per unit and block, a batch in which
-            // every other sequence is short would leave half of the engines idle (8 x 512 + 8 x 3584 tokens, 32q/8kv:
-            // 1537 us), so mb_run = 4 blocks of a unit are neighbours then (988 us), as its heads are where they are not packed.
-            const int per_run = units8 * p.mb_run;
-            const int first = (int)(bid / per_run);
-            const int e = bid - first * per_run;
-            const int j = (e >> 3) / p.mb_run;
-            unit = j * 8 + (e & 7);
-            head_in_unit = 0;
-            mb = p.num_mb - 1 - first * p.mb_run - ((e >> 3) - j * p.mb_run);
-        } else {
-            mb = p.num_mb - 1 - (int)(bid / per_block);
-            const int e = bid % per_block;
-            unit = ((e >> 3) / heads_per_unit) * 8 + (e & 7);
-            head_in_unit = (e >> 3) % heads_per_unit;
-        }
-    } else {
-        // one or two blocks per unit (short sequences, all equally light): a unit's blocks stay
-        // neighbours in their XCD's queue, so its K/V are fetched into that L2 once
-        const int per_unit = p.num_mb * heads_per_unit;
-        const int r = bid >> 3;
-        unit = (r / per_unit) * 8 + (bid & 7);
-        head_in_unit = (r % per_unit) / p.num_mb;
-        mb = p.num_mb - 1 - r % p.num_mb;
-    }
+    const PrefillPlace place = prefill_place(bid, p.num_mb, EXT ? p.mb_run : 1, units8, heads_per_unit);
+    const int mb = place.mb, unit = place.unit, head_in_unit = place.head;
     if (unit >= n_units) return;
     const int z = unit / p.nheads_k;
     const int hk = unit - z * p.nheads_k;
@@ -704,28 +671,12 @@ __global__ void __launch_bounds__(256) prefill_combine_kernel(const PrefillParam
 
 static_assert(kBM == kPrefillTileRows, "the planning rules in fa_kernels.h assume this tile height");
 
-// Causal blocks of a group of heads: the 128 rows of a tile are 128 / group queries of all the heads rather than 128 queries
-// of one, so that a tile's keys end closer behind its queries (half a tile of hidden keys per row less at a group of 4)
-// and short sequences fill their tiles: 80 x 3..350 tokens, 28q/4kv 94.3 -> 77.9 us; 40 x 50..900, 28q/4kv 170.2 -> 163.6;
-// 16 prompts of 512..4096, 32q/8kv 802.6 -> 799.2 (d = 64: 453.1 -> 443.5); 4 x 8192 under a window of 1024 keys 686.6 -> 656.6.
-// Bidirectional blocks gain nothing (30 x 100..900, 32q/8kv 218.3 -> 219.8) and stay as prefill_pack() has them, and so do
-// launches of fewer tiles than two rounds of the device (1024: two per workgroup slot), which last as long as their tallest
-// tile either way (2 x 649 tokens, 32q/4kv 23.1 -> 24.4; 43 x 18..182, 8q/1kv 15.8 -> 16.3).
-static bool prefill_pack_causal(const PrefillParams &p) {
-    return p.causal && p.group > 1 && p.group <= kBM && (int64_t)p.max_seqlen_q * p.group < (1ll << 30) &&
-           (int64_t)p.total_q * p.nheads >= 1024ll * kBM;
-}
-
 template <typename T, int D> static hipError_t launch_prefill_d(const PrefillParams &p_in, hipStream_t stream) {
     PrefillParams p = p_in;
-    p.pack = prefill_pack(p.group, p.max_seqlen_q);
-    if (p.nsplits <= 1 && !p.long_ids && prefill_pack_causal(p)) p.pack = p.group;
-    p.num_mb = (p.max_seqlen_q * p.pack + kBM - 1) / kBM;
-    // packed blocks of sequences that differ in length: four of a unit side by side (prefill_block; equal lengths leave no
-    // gaps, and runs would only blur the order of the heights: D = 256, 4 x 2048 tokens 222 us without, 238 us with)
-    const bool ragged = p.cu_seqlens_q && (int64_t)p.batch * p.max_seqlen_q != p.total_q;
-    p.mb_run = (p.pack > 1 && p.num_mb > 2 && ragged && !p.long_ids) ? 4 : 1;
-    p.num_mb = (p.num_mb + p.mb_run - 1) / p.mb_run * p.mb_run;
+    const PrefillTiles tiles = prefill_tiling(p.group, p.nheads, p.max_seqlen_q, p.total_q, p.causal && p.nsplits <= 1 && !p.long_ids);
+    p.pack = tiles.pack;
+    p.mb_run = tiles.mb_run;
+    p.num_mb = tiles.num_mb;
     if (p.nsplits > 1 && (!p.block_table || !p.o_partial || !p.lse_partial)) return hipErrorInvalidValue;
     const int64_t units = (int64_t)p.batch * max(p.nsplits, 1) * p.nheads_k;
     p.units8 = (int32_t)((units + 7) / 8 * 8);

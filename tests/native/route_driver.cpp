@@ -1,7 +1,9 @@
-// Host-only: which kernel the library's routing rule gives a kvcache call.  Links the real fa_rocm_api.cpp; the launchers are
-// stubs that say that they were called.  One call per line of standard input,
-//     batch seqlen_q heads kv_heads head_dim page pages_per_row new_keys window_left
-// one route per line of output: "unit W" (a workgroup of W waves per unit), "cut" (units cut over the device) or "tiled".
+// Host-only: what the library's routing rules decide.  Links the real fa_rocm_api.cpp; the launchers are stubs that say that
+// they were called.  One question per line of standard input, one answer per line of output:
+//     call batch seqlen_q heads kv_heads head_dim page pages_per_row new_keys window_left
+//         -> "unit W" (a workgroup of W waves per unit), "cut" (units cut over the device), "tiled" or "latent"
+//     tiling group heads max_seqlen_q total_q causal -> heads per tile, tiles side by side, tiles of a unit
+//     order tiles tiles_side_by_side units heads_per_unit -> unit/tile/head of every workgroup of the tiled forward
 #include <cstdio>
 #include <cstring>
 
@@ -33,8 +35,27 @@ hipError_t launch_scatter_short_blocks(const ShortBlocksParams &, hipStream_t) {
 
 int main() {
     void *const some = reinterpret_cast<void *>(0x1000);   // never dereferenced
-    int batch, sq, hq, hk, d, page, pages, fresh, window;
-    while (std::scanf("%d %d %d %d %d %d %d %d %d", &batch, &sq, &hq, &hk, &d, &page, &pages, &fresh, &window) == 9) {
+    char what[16];
+    while (std::scanf("%15s", what) == 1) {
+        if (!std::strcmp(what, "tiling")) {
+            int group, heads, longest, total, causal;
+            if (std::scanf("%d %d %d %d %d", &group, &heads, &longest, &total, &causal) != 5) return 1;
+            const fa::PrefillTiles t = fa::prefill_tiling(group, heads, longest, total, causal != 0);
+            std::printf("%d %d %d\n", t.pack, t.mb_run, t.num_mb);
+            continue;
+        }
+        if (!std::strcmp(what, "order")) {
+            int tiles, run, units, heads;
+            if (std::scanf("%d %d %d %d", &tiles, &run, &units, &heads) != 4) return 1;
+            for (int i = 0; i < tiles * units * heads; ++i) {
+                const fa::PrefillPlace w = fa::prefill_place((unsigned)i, tiles, run, units, heads);
+                std::printf("%d/%d/%d ", w.unit, w.mb, w.head);
+            }
+            std::printf("\n");
+            continue;
+        }
+        int batch, sq, hq, hk, d, page, pages, fresh, window;
+        if (std::scanf("%d %d %d %d %d %d %d %d %d", &batch, &sq, &hq, &hk, &d, &page, &pages, &fresh, &window) != 9) return 1;
         fa_kvcache_args a;
         std::memset(&a, 0, sizeof(a));
         a.q = a.out = a.k_cache = a.v_cache = a.workspace = some;
