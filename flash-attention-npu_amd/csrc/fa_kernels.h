@@ -144,6 +144,7 @@ struct PrefillParams {
     int32_t list_wgs;
     int32_t num_mb, units8;        // set by the launcher: 128-row blocks per unit, units rounded up to 8
     int32_t mb_run;                // set by the launcher: tiles of a unit that are neighbours in the launch order
+    int32_t num_cus;               // compute units of the device
     int32_t seqlen_q_fixed, seqlen_k_add;   // kvcache layout: Sq per row, keys appended this call
     int32_t max_seqlen_q, total_q;
     int32_t page_size, max_blocks, num_blocks;
@@ -199,6 +200,8 @@ inline int prefill_pack(int group, int max_seqlen_q) {
     const int64_t tiles_packed = ((int64_t)max_seqlen_q * group + kPrefillTileRows - 1) / kPrefillTileRows;
     return tiles_packed * 4 <= tiles_plain * 3 ? group : 1;
 }
+// Workgroups of the tiled forward that a compute unit holds.
+constexpr int prefill_wgs_per_cu(int headdim) { return headdim <= 128 ? 2 : 1; }
 // Causal launches that prefill_pack() leaves unpacked: whether the heads of a group share the tiles all the same.  The 128
 // rows of a tile are then 128 / group queries of all the heads rather than 128 queries of one, so that a tile's keys end
 // closer behind its queries (half a tile of hidden keys per row less at a group of 4) and short sequences fill their
@@ -206,19 +209,19 @@ inline int prefill_pack(int group, int max_seqlen_q) {
 // 512..4096, 32q/8kv 796 / 761 (d = 64: 446.7 / 424.4); 64 x 512, 64q/32kv 583 / 570; 24 x 100..500, 16q/2kv, d = 256
 // 119.6 / 107.1.  Bidirectional launches gain nothing (30 x 100..900, 32q/8kv 218.3 / 219.8).  Nor do launches of less than
 // two rounds of the device, which last as long as their tallest tile either way (D = 128: 2 x 649 tokens, 32q/8kv 21.9 /
-// 23.0, 6 x 300..700, 16q/8kv 22.8 / 23.6); from there on the worst measured are 1-3 %
-// behind (4 x 2048, 24q/8kv 119.7 / 121.1; 12 x 100..500, 64q/32kv 60.6 / 62.3), and at D = 256 none is (20 x 200, 16q/2kv
-// 57.3 / 44.5; 12 x 100..500, 16q/8kv 53.2 / 51.2).
-inline bool prefill_pack_causal(int group, int nheads, int max_seqlen_q, int total_q) {
+// 23.0, 6 x 300..700, 16q/8kv 22.8 / 23.6); from there on the worst measured are 1-3 % behind (4 x 2048, 24q/8kv 119.7 /
+// 121.1; 12 x 100..500, 64q/32kv 60.6 / 62.3), and at D = 256 none is (20 x 200, 16q/2kv 57.3 / 44.5; 12 x 100..500, 16q/8kv
+// 53.2 / 51.2).
+inline bool prefill_pack_causal(int group, int nheads, int max_seqlen_q, int total_q, int headdim, int num_cus) {
     return group > 1 && group <= kPrefillTileRows && (int64_t)max_seqlen_q * group < (1ll << 30) &&
-           (int64_t)total_q * nheads >= 1024ll * kPrefillTileRows;
+           (int64_t)total_q * nheads >= 2ll * num_cus * prefill_wgs_per_cu(headdim) * kPrefillTileRows;
 }
 // Heads per tile, tiles of a unit that are neighbours in the launch order, tiles of a unit.  causal_packs: the launch may follow
 // prefill_pack_causal() (causal, no key ranges, no device-side list).
 struct PrefillTiles { int32_t pack, mb_run, num_mb; };
-inline PrefillTiles prefill_tiling(int group, int nheads, int max_seqlen_q, int total_q, bool causal_packs) {
+inline PrefillTiles prefill_tiling(int group, int nheads, int max_seqlen_q, int total_q, int headdim, int num_cus, bool causal_packs) {
     PrefillTiles t = {prefill_pack(group, max_seqlen_q), 1, 0};
-    if (t.pack == 1 && causal_packs && prefill_pack_causal(group, nheads, max_seqlen_q, total_q)) t.pack = t.mb_run = group;
+    if (t.pack == 1 && causal_packs && prefill_pack_causal(group, nheads, max_seqlen_q, total_q, headdim, num_cus)) t.pack = t.mb_run = group;
     t.num_mb = (int32_t)(((int64_t)max_seqlen_q * t.pack + kPrefillTileRows - 1) / kPrefillTileRows);
     return t;
 }

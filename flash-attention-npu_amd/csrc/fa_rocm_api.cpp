@@ -409,7 +409,7 @@ int fa_rocm_plan_kvcache(const fa_kvcache_args *a, int num_cus, fa_split_plan *p
             n = a->num_splits;
         } else if (a->num_splits == 0) {
             const int64_t tiles = (int64_t)a->batch * fa::prefill_tiles(a->nheads, a->nheads_k, a->seqlen_q);
-            const int64_t slots = (int64_t)num_cus * (a->headdim_qk <= 128 ? 2 : 1);
+            const int64_t slots = (int64_t)num_cus * fa::prefill_wgs_per_cu(a->headdim_qk);
             if (tiles * 2 <= slots) n = (slots + tiles - 1) / tiles;
         }
         const int64_t most = (bound + 255) / 256;   // at least 256 keys (four tiles) per range
@@ -585,6 +585,7 @@ static int fwd_kvcache_impl(const fa_kvcache_args *a, void *stream_, void *const
         pp.seqlen_k_add = a->seqlen_new;
         pp.max_seqlen_q = a->seqlen_q;
         pp.total_q = a->batch * a->seqlen_q;
+        pp.num_cus = cus_t;
         pp.page_size = a->page_size;
         pp.max_blocks = a->max_blocks_per_seq;
         pp.num_blocks = a->num_blocks;
@@ -1056,7 +1057,7 @@ int fa_rocm_varlen_num_splits(const fa_varlen_args *a, int num_cus) {
     if (a->num_splits > 1) {
         n = a->num_splits;
     } else {
-        const int64_t slots = (int64_t)num_cus * (a->headdim <= 128 ? 2 : 1);
+        const int64_t slots = (int64_t)num_cus * fa::prefill_wgs_per_cu(a->headdim);
         // query blocks far shorter than the longest one on average (a prompt chunk among decode rows): the
         // longest block is the critical path long before the tiles fill the device, so it is cut earlier
         const bool uneven = uneven_blocks(a);
@@ -1147,6 +1148,7 @@ int fa_rocm_varlen_fwd(const fa_varlen_args *a, void *stream_) {
     pp.group = a->nheads / a->nheads_k;
     pp.max_seqlen_q = a->max_seqlen_q;
     pp.total_q = a->total_q;
+    pp.num_cus = cus;
     pp.page_size = a->page_size;
     pp.max_blocks = a->max_blocks_per_seq;
     pp.num_blocks = a->num_blocks;
@@ -1184,7 +1186,7 @@ int fa_rocm_varlen_fwd(const fa_varlen_args *a, void *stream_) {
         // the sequences left to the tiled kernel are listed on the device by the gather kernel
         pp.long_ids = sr.long_ids;
         pp.list_state = sr.list_state;
-        pp.list_wgs = cus * (a->headdim <= 128 ? 2 : 1);
+        pp.list_wgs = cus * fa::prefill_wgs_per_cu(a->headdim);
     }
     if (!w.decode_only) {
         const hipError_t e = fa::launch_prefill(pp, a->io_dtype, fa::tile_headdim(a->headdim), stream);

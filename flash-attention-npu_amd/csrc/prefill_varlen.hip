@@ -673,7 +673,7 @@ static_assert(kBM == kPrefillTileRows, "the planning rules in fa_kernels.h assum
 
 template <typename T, int D> static hipError_t launch_prefill_d(const PrefillParams &p_in, hipStream_t stream) {
     PrefillParams p = p_in;
-    const PrefillTiles tiles = prefill_tiling(p.group, p.nheads, p.max_seqlen_q, p.total_q, p.causal && p.nsplits <= 1 && !p.long_ids);
+    const PrefillTiles tiles = prefill_tiling(p.group, p.nheads, p.max_seqlen_q, p.total_q, D, p.num_cus, p.causal && p.nsplits <= 1 && !p.long_ids);
     p.pack = tiles.pack;
     p.mb_run = tiles.mb_run;
     p.num_mb = tiles.num_mb;

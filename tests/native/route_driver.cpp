@@ -2,7 +2,7 @@
 // they were called.  One question per line of standard input, one answer per line of output:
 //     call batch seqlen_q heads kv_heads head_dim page pages_per_row new_keys window_left
 //         -> "unit W" (a workgroup of W waves per unit), "cut" (units cut over the device), "tiled" or "latent"
-//     tiling group heads max_seqlen_q total_q causal -> heads per tile, tiles side by side, tiles of a unit
+//     tiling group heads max_seqlen_q total_q head_dim compute_units causal -> heads per tile, tiles side by side, tiles of a unit
 //     order tiles tiles_side_by_side units heads_per_unit -> unit/tile/head of every workgroup of the tiled forward
 #include <cstdio>
 #include <cstring>
@@ -38,9 +38,9 @@ int main() {
     char what[16];
     while (std::scanf("%15s", what) == 1) {
         if (!std::strcmp(what, "tiling")) {
-            int group, heads, longest, total, causal;
-            if (std::scanf("%d %d %d %d %d", &group, &heads, &longest, &total, &causal) != 5) return 1;
-            const fa::PrefillTiles t = fa::prefill_tiling(group, heads, longest, total, causal != 0);
+            int group, heads, longest, total, d, cus, causal;
+            if (std::scanf("%d %d %d %d %d %d %d", &group, &heads, &longest, &total, &d, &cus, &causal) != 7) return 1;
+            const fa::PrefillTiles t = fa::prefill_tiling(group, heads, longest, total, d, cus, causal != 0);
             std::printf("%d %d %d\n", t.pack, t.mb_run, t.num_mb);
             continue;
         }

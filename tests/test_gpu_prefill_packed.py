@@ -1,5 +1,6 @@
 """Causal packed prompts whose tiles hold the queries of a whole group of heads: lengths around a tile's share of queries
-(128 / group), around the 64-key tiles and the four blocks that stand side by side, equal and unequal, against the oracle."""
+(128 / group), around the 64-key tiles and the tiles that stand side by side, equal and unequal, against the oracle.  Few tokens
+are packed or not by the heads that a tile saves; many (`fill`) are packed at every group."""
 import pytest
 import torch
 
@@ -26,12 +27,20 @@ def ends(lens):
     ([1, 17, 18, 19, 31, 32, 33, 63, 64, 65, 127, 128, 129, 300], None),
     ([257, 3, 258, 2, 256, 1, 255, 4], None),                               # every other sequence is short
     ([160, 160, 160], None),                                                # equal lengths
-    ([1, 700, 18, 511, 129, 513, 33, 640] * 3, None),                       # many tiles (the packed launch at every group here)
+    ([1, 700, 18, 511, 129, 513, 33, 640] * 3, None),                       # long and short
     ([5, 70, 130, 1], [200, 70, 61, 1]),                                    # more and fewer keys than queries
 ])
-def test_packed_causal(lens_q, lens_k, d, group, hk, dtype, opts):
+@pytest.mark.parametrize("fill", [False, True])
+def test_packed_causal(lens_q, lens_k, d, group, hk, dtype, opts, fill):
     from flash_attn_npu import flash_attn_varlen_func
     lens_k = lens_k or lens_q
+    if fill:
+        # two rounds of the device in 128-row tiles (two workgroups per compute unit up to D = 128, one at 256): from there on a
+        # causal launch packs its heads whatever their tiles save
+        rows = 2 * torch.cuda.get_device_properties(0).multi_processor_count * (2 if d <= 128 else 1) * 128
+        times = -(-rows // (sum(lens_q) * group * hk))
+        lens_q, lens_k = lens_q * times, lens_k * times
+        assert sum(lens_q) * group * hk >= rows
     g = torch.Generator().manual_seed(d + group + len(lens_q))
     q = torch.randn(sum(lens_q), group * hk, d, generator=g).to(dtype)
     k, v = (torch.randn(sum(lens_k), hk, d, generator=g).to(dtype) for _ in range(2))

@@ -15,12 +15,12 @@ CALLS = [
     # one workgroup of eight waves per compute unit, at most four chunks of 32 keys per wave
     (8, 4, 128, 1024, 1, "unit 8"), (256, 4, 128, 1024, 0, "unit 8"), (256, 4, 128, 1056, 1, "cut"), (128, 4, 96, 2048, 1, "cut"),
     (264, 4, 128, 768, 1, "unit 4"), (512, 4, 128, 768, 1, "unit 4"), (264, 4, 128, 800, 1, "cut"), (264, 4, 128, 2048, 1, "cut"),
-    (520, 4, 1, "cut"), (1536, 4, 128, 512, 1, "cut"),
+    (520, 4, 128, 256, 1, "cut"), (1536, 4, 128, 512, 1, "cut"),
     (512, 4, 64, 1024, 1, "unit 8"), (520, 4, 64, 1024, 1, "unit 4"), (1024, 4, 40, 1024, 1, "unit 4"), (1024, 4, 64, 1056, 1, "cut"),
     (1032, 4, 64, 512, 1, "unit 4"), (1032, 4, 64, 544, 1, "cut"), (8192, 4, 64, 512, 1, "unit 4"), (8200, 4, 64, 512, 1, "cut"),
     (256, 4, 256, 512, 1, "unit 4"), (264, 4, 256, 512, 1, "cut"), (256, 4, 192, 2048, 1, "cut"), (64, 4, 256, 544, 1, "cut"),
     # 17-32 rows: the tiled kernel or two tiles per wave on the other side
-    (64, 20, 128, 768, 5, "unit 8"), (64, 20, 128, 800, 5, "tiled"), (64, 20, 128, 224, 0, "tiled"), (64, 20, 128, 224, 5, "tiled"), (64, 20, 0, "unit 8"),
+    (64, 20, 128, 768, 5, "unit 8"), (64, 20, 128, 800, 5, "tiled"), (64, 20, 128, 224, 0, "tiled"), (64, 20, 128, 224, 5, "tiled"), (64, 20, 128, 256, 0, "unit 8"),
     (184, 20, 128, 8000, 5, "tiled"), (192, 20, 128, 8192, 5, "unit 8"), (193, 20, 128, 8192, 5, "tiled"), (248, 20, 128, 8192, 0, "unit 8"), (192, 20, 128, 8224, 5, "tiled"),
     (256, 20, 128, 8000, 5, "cut"), (256, 20, 128, 768, 5, "unit 8"), (264, 20, 128, 768, 5, "unit 4"), (512, 32, 128, 2048, 8, "cut"),
     (64, 32, 128, 768, 8, "tiled"), (64, 24, 128, 768, 6, "unit 8"), (256, 32, 128, 768, 8, "unit 8"), (64, 32, 64, 768, 8, "cut"),
@@ -63,14 +63,18 @@ def test_decode_routes(ask):
 
 
 def test_prefill_tiling(ask):
-    # (group, heads, longest, tokens, causal) -> heads per tile, tiles side by side, tiles of a unit
+    # (group, heads, longest, tokens, head dimension, compute units, causal) -> heads per tile, tiles side by side, tiles of a unit
     cases = {
-        (4, 32, 182, 4043, 1): "4 1 6",         # packed whatever the mask: one by one
-        (4, 32, 182, 4043, 0): "4 1 6",
-        (4, 32, 4096, 32768, 1): "4 4 128",     # causal, many tiles: packed, the tiles of 128 queries side by side
-        (7, 28, 350, 14000, 1): "7 7 20",
-        (4, 32, 4096, 32768, 0): "1 1 32",
-        (1, 32, 4096, 32768, 1): "1 1 32",
+        (4, 32, 182, 4043, 128, 256, 1): "4 1 6",         # packed whatever the mask: one by one
+        (4, 32, 182, 4043, 128, 256, 0): "4 1 6",
+        (4, 32, 4096, 32768, 128, 256, 1): "4 4 128",     # causal, many tiles: packed, the tiles of 128 queries side by side
+        (7, 28, 350, 14000, 128, 256, 1): "7 7 20",
+        (4, 32, 4096, 32768, 128, 256, 0): "1 1 32",
+        (1, 32, 4096, 32768, 128, 256, 1): "1 1 32",
+        # two rounds of the device: two workgroups per compute unit up to D = 128, one at 256
+        (4, 32, 4096, 4096, 128, 256, 1): "4 4 128", (4, 32, 4096, 4095, 128, 256, 1): "1 1 32",
+        (4, 32, 2048, 2048, 256, 256, 1): "4 4 64", (4, 32, 2048, 2047, 256, 256, 1): "1 1 16",
+        (4, 32, 2048, 2048, 128, 128, 1): "4 4 64", (4, 32, 4096, 4096, 128, 304, 1): "1 1 32",
     }
     assert dict(zip(cases, ask("tiling", cases))) == cases
 
