@@ -234,13 +234,13 @@ int64_t live_keys_bound(const fa_kvcache_args *a) {
 // trip to memory each), and cannot be cut: the lengths are on the device, so whatever the host admits has to hold for any
 // of them, for one long row among short ones (only its workgroups still run) as for equal rows.  The host knows two things:
 // the most keys a unit can have (what the table or the window allows), and whether the workgroups all run at once.
-//   * All at once: a compute unit holds two workgroups of 4 waves at D = 128, one at 256, four at 64 (two of 8 up to 16
-//     rows); 8 waves where they fit.  Whole call at the limits below, workgroup per unit over partition, the worst and the
-//     best of: equal rows, one or two long ones, every tenth, every second, lengths spread over a factor of ten; and the worst
-//     one step further:
+//   * All at once: a compute unit holds two workgroups of 4 waves at D = 128, one at 256, four at 64; with a unit or less per
+//     compute unit 8 waves take it (two workgroups of 8 fit at D = 64, but 512 units x 1000 keys run 24.9 us with 4 and 26.5
+//     with 8).  Whole call at the limits below, workgroup per unit over partition, the best and the worst of: equal rows, one
+//     or two long ones, every tenth, every second, lengths spread over a factor of ten; and the worst one step further:
 //       D = 128, 8 waves, 1024 keys: 0.73-0.93 (8 units 16.6 -> 12.6 us, 256 of one long row 17.5 -> 15.2); 1536: 1.23
 //       D = 128, 4 waves, 768: 0.69-1.02 (512 units of one long row 17.8 -> 16.5); 1024: 1.17;  768 units x 768: 1.18
-//       D = 64, 8 waves, 1024: 0.47-0.84;  4 waves, 1024: 0.58-1.00 (640 units of 33..900: 31.1 -> 20.7); 2048: 1.47
+//       D = 64, 8 waves, 1024: 0.47-0.76;  4 waves, 1024: 0.58-1.00 (640 units of 33..900: 31.1 -> 20.7); 2048: 1.47
 //       D = 256, 4 waves, 512: 0.55-0.92; 768: 1.06, 264 units x 384: 1.21
 //       17-32 rows, D = 128, 768: 0.42-0.97; 1024: 1.15, 1024 units x 768: 1.40;  D = 64, 1024: 0.38-0.95
 //   * Several rounds, D = 64, up to 16 rows: 512 keys 0.62-0.98 (2048 units x 512 55.2 -> 52.4 us); 768: 1.04.  Wider rows
@@ -266,10 +266,9 @@ int unit_waves(const fa_kvcache_args *a, size_t rows, int num_cus) {
         return 0;
     const int64_t units = (int64_t)a->batch * a->nheads_k, keys = live_keys_bound(a), cus = num_cus;
     const bool tall = rows > 16;
-    const int64_t held8 = width > 128 ? 0 : width == 64 && !tall ? 2 * cus : cus;   // workgroups that run at once, of 8 waves
-    const int64_t held4 = (width == 64 ? 4 : width == 128 ? 2 : 1) * cus;           // ... and of 4
+    const int64_t held4 = (width == 64 ? 4 : width == 128 ? 2 : 1) * cus;   // workgroups of 4 waves that run at once
     if (units > held4) return width == 64 && !tall && units <= 32 * cus && keys <= 512 ? 4 : 0;
-    const int waves = units <= held8 ? 8 : 4;
+    const int waves = width <= 128 && units <= cus ? 8 : 4;
     int64_t most = width > 128 ? 512 : width == 64 || (waves == 8 && !tall) ? 1024 : 768;
     const bool cut_appends = width == 128 && units >= cus;   // the kernel on the other side writes the new keys like this one
     if (tall && !cut_appends && a->k_new && a->seqlen_new > 6) return 0;

@@ -16,7 +16,7 @@ CALLS = [
     (8, 4, 128, 1024, 1, "unit 8"), (256, 4, 128, 1024, 0, "unit 8"), (256, 4, 128, 1056, 1, "cut"), (128, 4, 96, 2048, 1, "cut"),
     (264, 4, 128, 768, 1, "unit 4"), (512, 4, 128, 768, 1, "unit 4"), (264, 4, 128, 800, 1, "cut"), (264, 4, 128, 2048, 1, "cut"),
     (520, 4, 128, 256, 1, "cut"), (1536, 4, 128, 512, 1, "cut"),
-    (512, 4, 64, 1024, 1, "unit 8"), (520, 4, 64, 1024, 1, "unit 4"), (1024, 4, 40, 1024, 1, "unit 4"), (1024, 4, 64, 1056, 1, "cut"),
+    (256, 4, 64, 1024, 1, "unit 8"), (264, 4, 64, 1024, 1, "unit 4"), (520, 4, 64, 1024, 1, "unit 4"), (1024, 4, 40, 1024, 1, "unit 4"), (1024, 4, 64, 1056, 1, "cut"),
     (1032, 4, 64, 512, 1, "unit 4"), (1032, 4, 64, 544, 1, "cut"), (8192, 4, 64, 512, 1, "unit 4"), (8200, 4, 64, 512, 1, "cut"),
     (256, 4, 256, 512, 1, "unit 4"), (264, 4, 256, 512, 1, "cut"), (256, 4, 192, 2048, 1, "cut"), (64, 4, 256, 544, 1, "cut"),
     # 17-32 rows: the tiled kernel or two tiles per wave on the other side
