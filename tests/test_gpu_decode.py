@@ -3,9 +3,16 @@ import pytest
 import torch
 
 import fa_oracle as O
-from helpers import check_out, check_vs_golden, make_paged_case, rotary_tables, to_dev
+from helpers import check_out, check_vs_golden, library_env, make_paged_case, rotary_tables, to_dev
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(params=["rule", "cut"])
+def units(request):
+    """Short units go to one workgroup each; "cut" has them cut over the device as long ones are."""
+    with library_env(**({"FA_ROCM_UNIT_WAVES": 0} if request.param == "cut" else {})):
+        yield
 
 
 def run_both(case, **kw):
@@ -43,6 +50,7 @@ def test_decode_split_invariance(num_splits):
     check_out(got[0], ref[0], got[1], ref[1], f"splits={num_splits}")
 
 
+@pytest.mark.usefixtures("units")
 @pytest.mark.parametrize("lens", [[1, 31, 32, 33], [255, 256, 257, 512], [0, 5, 0, 700]])
 def test_decode_ragged_edges(lens):
     case = make_paged_case(4, 8, 2, 128, 256, lens, seed=3)
@@ -57,6 +65,7 @@ def test_decode_uniform5_distribution():
     check_vs_golden(got[0], gold[0], got[1], gold[1], "uniform5")
 
 
+@pytest.mark.usefixtures("units")
 @pytest.mark.parametrize("window", [(64, 0), (542, 647), (4095, 0), (0, 0), (-1, 3)])
 def test_decode_window(window):
     case = make_paged_case(2, 8, 1, 128, 256, [5000, 1300], seed=5)
@@ -64,6 +73,7 @@ def test_decode_window(window):
     check_out(got[0], ref[0], got[1], ref[1], f"window={window}")
 
 
+@pytest.mark.usefixtures("units")
 @pytest.mark.parametrize("sq,hq,hk", [(2, 8, 2), (4, 4, 1), (3, 16, 8), (5, 8, 8), (2, 32, 1)])
 def test_decode_multi_token_causal(sq, hq, hk):
     case = make_paged_case(2, hq, hk, 128, 256, [700, 259], seqlen_q=sq, seed=6)
@@ -71,6 +81,7 @@ def test_decode_multi_token_causal(sq, hq, hk):
     check_out(got[0], ref[0], got[1], ref[1], f"sq={sq}")
 
 
+@pytest.mark.usefixtures("units")
 def test_decode_sq_longer_than_keys():
     # bottom-right causal with Sq > Sk: the first Sq-Sk rows see nothing -> 0 / +inf
     case = make_paged_case(1, 4, 2, 128, 256, [2], seqlen_q=5, seed=7)
@@ -88,12 +99,14 @@ def test_decode_headdims(d):
     check_out(got[0], ref[0], got[1], ref[1], f"d={d} split")
 
 
+@pytest.mark.usefixtures("units")
 def test_decode_softcap():
     case = make_paged_case(2, 8, 2, 128, 256, [600, 300], seed=9)
     got, ref, gold, _ = run_both(case, causal=True, softcap=3.0)
     check_out(got[0], ref[0], got[1], ref[1], "softcap")
 
 
+@pytest.mark.usefixtures("units")
 @pytest.mark.parametrize("interleaved", [False, True])
 @pytest.mark.parametrize("rot", [128, 64])
 def test_append_rotary_bit_exact(interleaved, rot):
@@ -140,6 +153,7 @@ def double_rounding_pairs(count, seed=0):
     return x1[idx], x2[idx], sn[idx]
 
 
+@pytest.mark.usefixtures("units")
 @pytest.mark.parametrize("num_splits", [0, 2])        # 0: rows appended by the attention kernel, 2: by the append kernel
 @pytest.mark.parametrize("interleaved", [False, True])
 def test_append_rotary_fp16_rounds_in_fp32_first(interleaved, num_splits):
@@ -174,6 +188,7 @@ def test_append_rotary_fp16_rounds_in_fp32_first(interleaved, num_splits):
     assert torch.equal(dev["v_cache"].cpu().view(torch.int16), vc.view(torch.int16))
 
 
+@pytest.mark.usefixtures("units")
 def test_append_multi_token_crosses_page():
     case = make_paged_case(2, 8, 2, 128, 256, [254, 510], seqlen_q=3, seqlen_new=3, seed=12)
     got, ref, gold, (dev, kc, vc) = run_both(case, causal=True)
@@ -182,6 +197,7 @@ def test_append_multi_token_crosses_page():
     check_out(got[0], ref[0], got[1], ref[1], "append3")
 
 
+@pytest.mark.usefixtures("units")
 @pytest.mark.parametrize("window", [(0, -1), (-1, 1), (1, 1), (3, 0), (-1, 7)])
 def test_decode_window_more_queries_than_keys(window):
     # Sq > Sk: the reference's host normalisation (side >= Sk unbounded, unbounded side := Sk) is not
@@ -191,6 +207,7 @@ def test_decode_window_more_queries_than_keys(window):
     check_out(got[0], ref[0], got[1], ref[1], f"sq>sk window={window}")
 
 
+@pytest.mark.usefixtures("units")
 @pytest.mark.parametrize("B,num_splits", [(300, 0), (700, 0), (300, 2)])
 def test_decode_batch_larger_than_prefix_segments(B, num_splits):
     # the balanced partition scans the batch in 256 segments: more than 256 rows puts several rows

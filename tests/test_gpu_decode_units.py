@@ -47,15 +47,26 @@ def test_units(d, hq, hk, sq, dtype, opts, waves):
     check_out(out, cut, lse, cut_lse, f"units against cut units d={d}")
 
 
+@pytest.mark.parametrize("waves", [0, 4, 8])
 @pytest.mark.parametrize("interleaved", [False, True])
-@pytest.mark.parametrize("d,hq,hk,new", [(128, 8, 2, 1), (64, 4, 4, 3), (128, 20, 4, 5), (256, 4, 2, 2)])
-def test_units_append(d, hq, hk, new, interleaved):
+@pytest.mark.parametrize("d,hq,hk,sq,new,opts", [
+    (128, 8, 2, 1, 1, {}),
+    (64, 4, 4, 3, 3, {}),
+    (128, 20, 4, 5, 5, {}),
+    (256, 4, 2, 2, 2, {}),
+    (128, 8, 2, 1, 40, {}),                                  # more new rows than a chunk holds, one query
+    (128, 12, 2, 3, 2, {"softcap": 25.0}),
+    (64, 8, 2, 4, 2, {"window_size": (50, 0)}),
+    (128, 8, 2, 1, 9, {"window_size": (4, 0)}),              # new rows behind the window: written by their own launch
+    (96, 4, 1, 2, 3, {"window_size": (70, 5), "causal": False}),
+])
+def test_units_append(d, hq, hk, sq, new, opts, interleaved, waves):
     """The rows that the waves append are those of the append kernel to the bit, whichever wave owns their chunk."""
     lens = [0, 1, 30, 31, 32, 95, 126, 255, 700]
-    case = make_paged_case(len(lens), hq, hk, d, 32, lens, seqlen_q=new, seqlen_new=new, seed=new)
+    case = make_paged_case(len(lens), hq, hk, d, 32, lens, seqlen_q=sq, seqlen_new=new, seed=new)
     cos, sin = rotary_tables(800, d)
-    kw = dict(causal=True, rotary_cos=cos, rotary_sin=sin, rotary_interleaved=interleaved)
-    with library_env(FA_ROCM_UNIT_WAVES=8):
+    kw = {"causal": True, "rotary_cos": cos, "rotary_sin": sin, "rotary_interleaved": interleaved, **opts}
+    with library_env(FA_ROCM_UNIT_WAVES=waves):
         out, lse, kc, vc = call(case, **kw)
     ref_k, ref_v = case["k_cache"].clone(), case["v_cache"].clone()
     ref, ref_lse = O.flash_attn_with_kvcache(case["q"], ref_k, ref_v, case["k"], case["v"], cache_seqlens=case["cache_seqlens"],
