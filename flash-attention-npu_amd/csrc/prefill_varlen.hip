@@ -6,10 +6,11 @@
 // flash_api.cpp:848-1089).  Where the reference ping-pongs S, P and O_tmp between its matrix and
 // vector cores through global memory, everything between the K/V tile loads and the final store
 // stays in registers here:
-//   * one workgroup = 128 query rows of one (sequence, q head); 4 waves x 32 rows.  Short query
-//     blocks under GQA are packed instead (p.pack = group): the 128 rows are (query, head of the
-//     group) pairs of one kv head, query-major, so a 16-token block of an 8-head group fills a tile
-//     and K/V are read once per kv head (the reference packs heads the same way, flash_api.cpp:33-95);
+//   * one workgroup = 128 query rows of one (sequence, q head); 4 waves x 32 rows.  Under GQA short
+//     query blocks, and causal launches of many tiles, are packed instead (p.pack = group): the 128 rows are
+//     (query, head of the group) pairs of one kv head, query-major, so a 16-token block of an 8-head group
+//     fills a tile and K/V are read once per kv head (the reference packs heads the same way,
+//     flash_api.cpp:33-95), and a causal tile's keys end closer behind its queries (prefill_tiling());
 //   * K/V tiles of 64 keys are fetched once per workgroup, 16 bytes per lane, straight from global memory
 //     into LDS (no register holds them and no LDS store instruction moves them: such a store keeps the
 //     wave from issuing anything else for ~50 cycles, and the tile stores were a tenth of the kernel's

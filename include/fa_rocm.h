@@ -173,9 +173,12 @@ int fa_rocm_num_cus(void);
  *                        (each holds it for its own check's round trip), whatever their threads and streams.
  *                        Without it these cases are the caller's contract, as in the reference, whose host
  *                        never reads the table either (csrc/ascend910/flash_attn_npu/flash_api.cpp:386-420).
- *   FA_ROCM_DECODE_MAX_ROWS, FA_ROCM_DECODE_WGS, FA_ROCM_DECODE_BLOCK_WORKERS, FA_ROCM_MIN_SHARE, FA_ROCM_PIECE_COST,
- *   FA_ROCM_NO_HEAD_INTERLEAVE, FA_ROCM_SEPARATE_APPEND, FA_ROCM_NO_SHORT_BLOCKS: experiment switches of the decode
- *   partition and the kernel choice; results do not depend on them beyond rounding.
+ *   FA_ROCM_UNIT_WAVES   0: units are always cut over the device; 4 or 8: one workgroup of that many waves takes a whole
+ *                        unit wherever it can (up to 32 query rows, 16 beyond head dimension 128, where 8 means 4).
+ *   FA_ROCM_DECODE_MAX_ROWS, FA_ROCM_WAVE_MAX_ROWS, FA_ROCM_WAVE_TWO_TILES, FA_ROCM_DECODE_WGS, FA_ROCM_DECODE_BLOCK_WORKERS,
+ *   FA_ROCM_MIN_SHARE, FA_ROCM_PIECE_COST, FA_ROCM_NO_HEAD_INTERLEAVE, FA_ROCM_SEPARATE_APPEND, FA_ROCM_NO_SHORT_BLOCKS:
+ *   experiment switches of the decode partition and the kernel choice (all but the last also turn the choice of one
+ *   workgroup per unit off); results do not depend on any of them beyond rounding.
  */
 void fa_rocm_reload_env(void);
 
@@ -194,6 +197,10 @@ void fa_rocm_reload_env(void);
  *     always get this mode: num_splits == 0 then picks as many ranges as it takes to fill the device
  *     when the tiles alone cannot (at most 64, at least 256 addressable keys each), and
  *     `split_keys` is 0: the range length is set on the device from the longest sequence.
+ * With num_splits == 0 a call whose table or window allows only short units, or that has many of them, may be given one
+ * workgroup per (batch row, kv head) instead, which neither cuts nor merges anything.  The plan does not tell: it is that of
+ * the partition (or, above 16 query rows, of the tiled kernel) the call would have otherwise, and the call asks for its
+ * workspace all the same, though it leaves the workspace alone.
  * Pure host integer code: needs no GPU.  `num_cus` <= 0 means 256.
  */
 enum fa_split_mode { FA_SPLIT_GRID = 0, FA_SPLIT_BALANCED = 1 };
@@ -203,7 +210,7 @@ typedef struct fa_split_plan {
     int32_t split_keys;       /* grid mode: keys per split                       */
     int32_t num_wgs;          /* balanced mode: workgroups launched              */
     int32_t num_workers;      /* balanced mode: workers sharing the chunk list (a workgroup, or each of its 4 waves) */
-    int32_t min_share;        /* balanced mode: least 32-key chunks per share    */
+    int32_t min_share;        /* balanced mode: least 32-key chunks per share (int8 latent cache: 2 where the device finds every sequence longer than that) */
     size_t workspace_bytes;   /* partial outputs + LSEs the call needs           */
 } fa_split_plan;
 int fa_rocm_plan_kvcache(const fa_kvcache_args *args, int num_cus, fa_split_plan *plan);
