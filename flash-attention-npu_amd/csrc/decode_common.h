@@ -74,7 +74,7 @@ __device__ __forceinline__ int unit_cost(int nchunks, int cost, int align) {
 // exclusive prefixes over 256 equal segments of the batch: s_pref[t] = chunks of rows [0, t*seg),
 // s_cnt[t] = rows among them with a visible key; [256] = totals.  All threads of the block must call
 // (256 or more threads; the first 256 do the work).  Returns whether some batch row has no visible key; LATENT (256 threads):
-// in bit 1, whether one has at most kWholeLatentChunks chunks (and a key), from the same pass over the lengths.
+// in bit 1, whether one has 2 .. kWholeLatentChunks chunks, from the same pass over the lengths.
 constexpr int kWholeLatentChunks = 4;
 template <bool LATENT = false> __device__ __forceinline__ int batch_chunk_prefix(const DecodeParams &p, int *s_pref, int *s_cnt, int seg, int M) {
     __shared__ int s_wave[4], s_wave_cnt[4];
@@ -85,7 +85,7 @@ template <bool LATENT = false> __device__ __forceinline__ int batch_chunk_prefix
         const int n = unit_range(p, b, M).nchunks;
         sum += n;
         cnt += (n > 0);
-        short_row |= n > 0 && n <= kWholeLatentChunks;
+        short_row |= n > 1 && n <= kWholeLatentChunks;   // (a single chunk cannot be cut)
     }
     const bool empty_row = tid * seg < p.batch && cnt < min(p.batch, (tid + 1) * seg) - tid * seg;
     int inc = sum, inc_cnt = cnt;
@@ -315,24 +315,29 @@ struct Partition {
     }
 };
 
-// Least share of the latent kernel: p.min_share (4 chunks), or p.min_share_short (2) where the units are of middling length.
-// A unit of at most kWholeLatentChunks chunks is never cut for it: whole, it is written straight from the fp32
-// accumulators; its pieces would be rounded to fp16 and clamped to that type's range.  Longer units are cut either way.
-// One sequence, whole call with shares of 2 / 4 chunks: 2048 keys 28.8 / 30.6 us, 4096 30.4 / 32.7, 8192 (twice the
-// partials to merge) 36.7 / 35.0: kLongLatentUnitChunks lies between the last two.
-constexpr int kLongLatentUnitChunks = 192;
-__device__ __forceinline__ int latent_least_share(const DecodeParams &p, const Partition &pt, const int *s_pref, int units, bool short_rows) {
-    // (more rows than prefix segments: the merge kernel works the partition out again, by the common rule)
-    const bool middling = pt.seg == 1 && !short_rows && pt.cost == 0 && s_pref[256] < (int64_t)kLongLatentUnitChunks * units;
-    return p.min_share_short > 0 && middling ? p.min_share_short : p.min_share;
-}
-
 // Whether `pred` holds for some batch row's chunks (one row per prefix segment).  Every wave looks at all the rows: a vote of
 // the workgroup would cost three barriers.
 template <typename Pred> __device__ __forceinline__ bool any_row(const DecodeParams &p, const int *s_pref, Pred pred) {
     bool any = false;
     for (int b = threadIdx.x & 63; b < p.batch; b += 64) any |= pred(s_pref[b + 1] - s_pref[b]);
     return __any(any);
+}
+
+// Least share of the latent kernel: p.min_share (4 chunks), or p.min_share_short (2) where the units are of middling length.
+// A unit of at most kWholeLatentChunks chunks is never cut for it: whole, it is written straight from the fp32
+// accumulators; its pieces would be rounded to fp16 and clamped to that type's range.  Longer units are cut either way.
+// One sequence, whole call with shares of 2 / 4 chunks: 2048 keys 28.8 / 30.6 us, 4096 30.4 / 32.7, 8192 (twice the
+// partials to merge) 36.7 / 35.0: kLongLatentUnitChunks lies between the last two.  With more chunks than workers the partials
+// weigh more, and only what could not be cut into whole shares of four gains: 10 sequences of 1792 keys 39.8 / 36.6, 10 of
+// 2048 39.7 / 37.1, but 40 of 60..570 36.7 / 39.9 and 20 of 160..1600 38.0 / 39.9.
+constexpr int kLongLatentUnitChunks = 192;
+__device__ __forceinline__ int latent_least_share(const DecodeParams &p, const Partition &pt, const int *s_pref, int units, bool short_rows,
+                                                  int64_t shares) {
+    // (more rows than prefix segments: the merge kernel works the partition out again, by the common rule)
+    const bool middling = pt.seg == 1 && !short_rows && pt.cost == 0 && s_pref[256] < (int64_t)kLongLatentUnitChunks * units;
+    if (p.min_share_short <= 0 || !middling || pt.W > shares * (p.min_share - 1)) return p.min_share;   // (last: the shares are that long anyway)
+    if (pt.W > shares && !any_row(p, s_pref, [&](int n) { return n % p.min_share != 0; })) return p.min_share;
+    return p.min_share_short;
 }
 
 // A share that holds the end of one unit and the start of the next pays the fixed cost of a piece (lengths -> table ->
@@ -346,9 +351,10 @@ template <typename Pred> __device__ __forceinline__ bool any_row(const DecodePar
 // cross: the host leaves it off).  The wave-level kernel, whose pieces start in ~6 us, gains nothing: 4 sequences x 8 kv
 // heads x 4096 visible keys 27.1 / 29.1, 8 x 4 heads x 2000..20000 keys 44.9 / 45.8.
 constexpr int kAlignTries = 3, kAlignMaxShare = 16;
-__device__ __forceinline__ void align_partition(const DecodeParams &p, Partition &pt, int *s_pref, int64_t shares) {
+__device__ __forceinline__ void align_partition(const DecodeParams &p, Partition &pt, int *s_pref, int units, int64_t shares) {
     __shared__ int s_need[4][kAlignTries], s_sum[4];
-    if (!p.align_units || pt.seg != 1 || pt.cost != 0 || pt.S > kAlignMaxShare) return;   // the same in every thread
+    // (the same in every thread; units: batch rows with a key)
+    if (!p.align_units || pt.seg != 1 || pt.cost != 0 || pt.S > kAlignMaxShare || (int64_t)units * pt.list_heads > shares) return;
     const int tid = threadIdx.x, S0 = (int)pt.S;
     const int n = tid < 256 ? s_pref[tid + 1] - s_pref[tid] : 0;   // this batch row's chunks
     if (!any_row(p, s_pref, [&](int m) { return m % S0 != 0; })) return;
@@ -408,7 +414,7 @@ template <bool LATENT = false> __device__ __forceinline__ Partition make_partiti
     pt.W = (int64_t)s_pref[256] * pt.list_heads;
     int least;
     if constexpr (LATENT) {
-        least = latent_least_share(p, pt, s_pref, s_cnt[256], (votes & 2) != 0);
+        least = latent_least_share(p, pt, s_pref, s_cnt[256], (votes & 2) != 0, shares);
     } else {
         const bool long_units = p.min_share_long > 0 && (int64_t)s_pref[256] >= (int64_t)kLongUnitChunks * max(s_cnt[256], 1) + (int64_t)pt.cost * s_cnt[256];
         least = long_units ? p.min_share_long : p.min_share;
@@ -416,7 +422,7 @@ template <bool LATENT = false> __device__ __forceinline__ Partition make_partiti
     pt.S = max((pt.W + shares - 1) / shares, (int64_t)max(least, 1));
     pt.align = 1;
     if constexpr (LATENT) {
-        align_partition(p, pt, s_pref, shares);
+        align_partition(p, pt, s_pref, s_cnt[256], shares);
         // the same in every lane, which the compiler cannot see behind the votes and LDS reads: vector registers are what
         // the latent kernel is short of
         auto uniform = [](int64_t x) -> int64_t {

@@ -13,7 +13,8 @@ EDGES = [0, 1, 31, 32, 33, 63, 64, 65, 96, 500, 2049]
 
 
 @pytest.mark.parametrize("wgs", [0, 13, 40])          # 0: the device's; 13: a worker takes several units; 40: barely enough to align
-@pytest.mark.parametrize("lens", [[700, 33], EDGES, [1500, 916, 2489], [40 + 37 * i for i in range(30)]])
+@pytest.mark.parametrize("lens", [[700, 33], EDGES, [1500, 916, 2489], [40 + 37 * i for i in range(30)],
+                                  [20] * 40, [1792] * 10, [160 + 37 * i for i in range(30)]])
 def test_ragged_shares(lens, wgs):
     case = mla_case(len(lens), 128, lens, page=64, seed=len(lens) + wgs)
     with library_env(**({"FA_ROCM_DECODE_WGS": wgs} if wgs else {})):
