@@ -329,7 +329,7 @@ template <typename Pred> __device__ __forceinline__ bool any_row(const DecodePar
 // One sequence, whole call with shares of 2 / 4 chunks: 2048 keys 28.8 / 30.6 us, 4096 30.4 / 32.7, 8192 (twice the
 // partials to merge) 36.7 / 35.0: kLongLatentUnitChunks lies between the last two.  With more chunks than workers the partials
 // weigh more, and only what could not be cut into whole shares of four gains: 10 sequences of 1792 keys 39.8 / 36.6, 10 of
-// 2048 39.7 / 37.1, but 40 of 60..570 36.7 / 39.9 and 20 of 160..1600 38.0 / 39.9.
+// 2048 39.7 / 37.1, but 40 of 170..345 36.7 / 39.9 and 20 of 170..1440 38.0 / 39.9.
 constexpr int kLongLatentUnitChunks = 192;
 __device__ __forceinline__ int latent_least_share(const DecodeParams &p, const Partition &pt, const int *s_pref, int units, bool short_rows,
                                                   int64_t shares) {
