@@ -14,8 +14,8 @@
 //   * K/V tiles of 64 keys are fetched once per workgroup, 16 bytes per lane, straight from global memory
 //     into LDS (no register holds them and no LDS store instruction moves them: such a store keeps the
 //     wave from issuing anything else for ~50 cycles, and the tile stores were a tenth of the kernel's
-//     time), double-buffered (K rows XOR-swizzled so MFMA operand reads are conflict free: the lane that
-//     fills a piece's place in LDS fetches the piece that belongs there);
+//     time), swizzled so that the operand reads are conflict free (the lane that fills a piece's place in
+//     LDS fetches the piece that belongs there); K tiles double-buffered, V tiles as far as LDS allows;
 //   * S^T = K Q^T and O^T = V^T P^T on the 32x32x16 MFMA: a query row is one lane column in both
 //     products, so the running max / sum / rescale never leave the lane (one xor-32 exchange);
 //   * V^T operands come straight from the transposing LDS read (ds_read_b64_tr_b16);
@@ -30,24 +30,42 @@ namespace fa {
 constexpr int kBM = 128;  // query rows per workgroup
 constexpr int kBN = 64;   // keys per tile
 
+// Workgroups (and so waves per SIMD) that a compute unit holds.  A wave alone takes 1.5 times as long for a tile as its matrix and
+// vector instructions need (operand reads, the barrier, the tile's arrival), and on a SIMD the matrix instructions of one wave
+// run beside the vector instructions of another, so one more wave is worth more than anything it costs: at D = 128 a second
+// barrier per tile, which one V buffer instead of two asks for (48 KB of LDS per workgroup), and operand reads only two k-steps
+// ahead.  Two / three waves at D = 128 (the former with both V buffers), three / four at D = 64, TFLOP/s: 4 x 8192 tokens, 32q/8kv,
+// bidirectional 993 / 1049 (d = 64: 864 / 882); 16 x 2048 causal 800 / 894; 4 x 4096, 32q/32kv 895 / 987; us: 16 x 512..4096 causal
+// 791.6 / 718.8, 80 x 3..350, 28q/4kv 85.9 / 78.3, 8 x 2050, 16q/16kv, d = 64, fp16 205.8 / 198.8.  Random values hold the
+// clock down (1.6-1.9 GHz; all-zero inputs run the same code 1.6 times as fast), so that half of the saved cycles do not show.
+// `spare`: kernels that keep more beside the tile loop (a head dimension below D, a list of blocks), which would spill.
+constexpr int prefill_occupancy(int d, bool spare) { return d == 64 ? 4 - spare : d == 128 ? 3 - spare : 1; }
+
 template <int D> struct PrefillCfg {
     static constexpr int kKSteps = D / 16;        // MFMA k-steps of QK^T
     static constexpr int kMT = D / 32;            // 32-column tiles of O^T
-    static constexpr int kCPL = D / 32;           // V columns a lane owns per key row
     static constexpr int kChunks = D / 8;         // 16-byte pieces per row
-    // XOR swizzle of the 16-byte pieces of a K row; the mask must not see the row step of the
-    // tile stores (256 / kChunks rows), so it is 7 for D = 256
-    static constexpr int kSwz = (kChunks == 16) ? 15 : 7;
-    static constexpr int kTileBytes = kBN * D * 2;
-    static constexpr int kVRowBytes = D * 2 + 64;        // padded V rows: transposing reads spread over all banks
-    static constexpr int kVTileBytes = kBN * kVRowBytes;
+    static constexpr int kRowBytes = D * 2;
+    static constexpr int kTileBytes = kBN * kRowBytes;
+    static constexpr int kVBufs = D == 128 ? 1 : 2;                // (see prefill_occupancy)
     // A tile is filled by loads that go from global memory straight to LDS (global_load_lds_dwordx4): one instruction
     // of a wave fills 64 consecutive 16-byte pieces, lane l the piece at the instruction's LDS base + 16 l, from
     // whatever address the lane names.  The four waves share the pieces of a tile, instruction by instruction.
-    static constexpr int kKLoads = kBN * kChunks / 256;            // per wave and K tile
-    static constexpr int kVRowPieces = kVRowBytes / 16;            // data pieces and padding
-    static constexpr int kVLoads = kBN * kVRowPieces / 256;        // per wave and V tile
-    static_assert(kBN * kChunks % 256 == 0 && kBN * kVRowPieces % 256 == 0, "whole instructions per wave");
+    static constexpr int kLoads = kBN * kChunks / 256;             // per wave and tile (K or V)
+    static constexpr int kLoadRows = 256 / kChunks;                // rows between a wave's consecutive loads
+    static_assert(kBN * kChunks % 256 == 0, "whole instructions per wave");
+    // Swizzles that spread the operand reads over all banks (256 bytes wide).  K: 16 rows of an operand are read 16
+    // bytes each, so their pieces have to stand in 16 different places; V: the transposing read takes 64 bytes (32
+    // columns) of each of 4 rows.  Rows of 128 bytes lie two in a line of banks and change place every other row.
+    static __device__ __forceinline__ int k_place(int row, int piece) { return piece ^ (D == 64 ? (row >> 1) & 7 : row & 15); }
+    static __device__ __forceinline__ int v_place(int row, int piece) { return piece ^ ((D == 64 ? (row >> 1) & 1 : row & 3) << 2); }
+    static constexpr int kPatterns = D == 256 ? 2 : 1;             // loads after which the places of a lane's pieces repeat
+};
+
+// K tiles: the one being read and the one on its way; V tiles likewise, or a single one (kVBufs)
+template <int D> struct PrefillTileLds {
+    __attribute__((aligned(1024))) uint8_t k[2][PrefillCfg<D>::kTileBytes];   // (operand addresses are formed by XOR inside a row)
+    __attribute__((aligned(1024))) uint8_t v[PrefillCfg<D>::kVBufs][PrefillCfg<D>::kTileBytes];
 };
 
 // EXT: packed heads and / or a split of the keys (p.pack, p.nsplits); without it both are compiled out
@@ -57,9 +75,7 @@ template <int D> struct PrefillCfg {
 // PART: the head dimension p.headdim is below D: pieces of the q / k / v rows behind it are zeros that nobody loads,
 // k-steps and output tiles that only see such pieces are skipped, and the stores stop at the head dimension.
 template <typename T, int D, bool PAGED, bool SOFTCAP, bool EXT, bool PART>
-__device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsigned bid, const int n_long,
-                                              uint8_t (&s_k)[2][PrefillCfg<D>::kTileBytes],
-                                              uint8_t (&s_v)[2][PrefillCfg<D>::kVTileBytes]) {
+__device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsigned bid, const int n_long, PrefillTileLds<D> &lds) {
     using Cfg = PrefillCfg<D>;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -221,35 +237,24 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     const uint16_t *vbase = reinterpret_cast<const uint16_t *>(p.v) + (int64_t)hk * p.v_stride_h;
     const int32_t *bt_row = PAGED ? p.block_table + (int64_t)b * p.bt_stride_b : nullptr;
 
-    // Load i of this wave covers the LDS pieces 64 (wave + 4i) .. + 63 of the tile, piece = (row, place in the row);
-    // a K row's place c' holds the row's piece c' ^ (row & kSwz), a V row is followed by its padding (nobody loads it).
+    // Load i of this wave covers the LDS pieces 64 (wave + 4i) .. + 63 of the tile, piece = (row, place in the row); a row's
+    // place c' holds the row's piece k_place(row, c') or v_place(row, c') (their own inverses).
     // Rows past the last key re-read the last key (never memory nobody wrote; they are masked); with PART the pieces
     // behind the head dimension are not loaded: their places hold the zeros written when the block started.
-    int k_row[Cfg::kKLoads], v_row[Cfg::kVLoads];
-    uint32_t k_col[Cfg::kKLoads], v_col[Cfg::kVLoads];          // byte offset of the lane's piece inside its row
-    bool k_on[Cfg::kKLoads], v_on[Cfg::kVLoads];
+    const int t_row = (64 * wave + lane) / Cfg::kChunks;      // of load 0; load i: kLoadRows * i rows further on
+    uint32_t k_off[Cfg::kPatterns], v_off[Cfg::kPatterns];    // offsets of load 0 (1) in an interior tile: one wave-uniform base serves all lanes
+    bool k_on[Cfg::kPatterns], v_on[Cfg::kPatterns];
+    auto col_of = [&](bool is_k, int i) -> int {              // the lane's piece in the row of load i
+        const int c = lane % Cfg::kChunks, row = t_row + i * Cfg::kLoadRows;
+        return is_k ? Cfg::k_place(row, c) : Cfg::v_place(row, c);
+    };
 #pragma unroll
-    for (int i = 0; i < Cfg::kKLoads; ++i) {
-        const int piece = 64 * (wave + 4 * i) + lane;
-        k_row[i] = piece / Cfg::kChunks;
-        const int c = (piece % Cfg::kChunks) ^ (k_row[i] & Cfg::kSwz);
-        k_col[i] = c * 16;
-        k_on[i] = !PART || c * 8 < hd;
+    for (int i = 0; i < Cfg::kPatterns; ++i) {
+        k_on[i] = !PART || col_of(true, i) * 8 < hd;
+        v_on[i] = !PART || col_of(false, i) * 8 < hd;
+        k_off[i] = (uint32_t)t_row * (uint32_t)p.k_stride_t * 2u + col_of(true, i) * 16;
+        v_off[i] = (uint32_t)t_row * (uint32_t)p.v_stride_t * 2u + col_of(false, i) * 16;
     }
-#pragma unroll
-    for (int i = 0; i < Cfg::kVLoads; ++i) {
-        const int piece = 64 * (wave + 4 * i) + lane;
-        v_row[i] = piece / Cfg::kVRowPieces;
-        const int c = piece % Cfg::kVRowPieces;
-        v_col[i] = c * 16;
-        v_on[i] = c < Cfg::kChunks && (!PART || c * 8 < hd);
-    }
-    // per-lane offsets of an interior tile of dense K/V (one wave-uniform base per tile serves all its loads)
-    uint32_t k_off[Cfg::kKLoads], v_off[Cfg::kVLoads];
-#pragma unroll
-    for (int i = 0; i < Cfg::kKLoads; ++i) k_off[i] = (uint32_t)k_row[i] * (uint32_t)p.k_stride_t * 2u + k_col[i];
-#pragma unroll
-    for (int i = 0; i < Cfg::kVLoads; ++i) v_off[i] = (uint32_t)v_row[i] * (uint32_t)p.v_stride_t * 2u + v_col[i];
     auto lds_of = [](const void *ptr) -> uint32_t { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)ptr; };
     // The loads are written out: the compiler would wait for such a load in front of every LDS read that follows (it
     // cannot tell the two buffers apart).  tiles_landed() is the wait that orders them.
@@ -259,65 +264,68 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     auto load_lds_addr = [&](uint32_t lds, const void *addr) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(addr) : "memory", "m0");
     };
+    auto uniform = [](const uint8_t *ptr) -> const uint8_t * {   // (for the compiler; it is)
+        const uint64_t x = reinterpret_cast<uint64_t>(ptr);
+        return reinterpret_cast<const uint8_t *>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32 |
+                                                 (uint32_t)__builtin_amdgcn_readfirstlane((int)x));
+    };
     auto tiles_landed = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
-    auto fetch_tile = [&](int kt, int buf) {
-        const uint32_t k_lds = lds_of(&s_k[buf][0]) + (uint32_t)wave * 1024u, v_lds = lds_of(&s_v[buf][0]) + (uint32_t)wave * 1024u;
+    // page of tile kt, for tiles that lie inside one (asked for a step before its loads: a scalar load, not one that would be
+    // waited for behind the tiles on their way)
+    const bool tile_in_page = !PAGED || p.page_size % kBN == 0;
+    auto page_of = [&](int kt) -> int {
+        if constexpr (!PAGED) return 0;
+        if (!tile_in_page) return 0;
+        const int page = min((kt * kBN) / p.page_size, p.max_blocks - 1);
+        return ((const __attribute__((address_space(4))) int32_t *)(uintptr_t)bt_row)[page];
+    };
+    // K (IS_K) or V tile kt into its buffer
+    auto fetch = [&](auto is_k_c, int kt, int blk_raw) {
+        constexpr bool IS_K = decltype(is_k_c)::value;
+        const uint32_t dst = lds_of(IS_K ? &lds.k[kt & 1][0] : &lds.v[kt & (Cfg::kVBufs - 1)][0]) + (uint32_t)wave * 1024u;
+        const uint16_t *base = IS_K ? kbase : vbase;
+        const int64_t stride_t = IS_K ? p.k_stride_t : p.v_stride_t, stride_block = IS_K ? p.k_stride_block : p.v_stride_block;
+        const uint32_t(&off)[Cfg::kPatterns] = IS_K ? k_off : v_off;
+        const bool(&on)[Cfg::kPatterns] = IS_K ? k_on : v_on;
         // A tile inside the sequence, of dense K/V or inside one page: one wave-uniform base serves all its loads
-        if (kt * kBN + kBN <= Sk && (!PAGED || p.page_size % kBN == 0)) {
-            int64_t koff, voff;
+        if (kt * kBN + kBN <= Sk && tile_in_page) {
+            int64_t first;
             if constexpr (PAGED) {
-                const int page = (kt * kBN) / p.page_size;
-                const int blk = min(max(__builtin_amdgcn_readfirstlane(bt_row[page]), 0), p.num_blocks - 1);
-                const int inpage = kt * kBN - page * p.page_size;
-                koff = (int64_t)blk * p.k_stride_block + (int64_t)inpage * p.k_stride_t;
-                voff = (int64_t)blk * p.v_stride_block + (int64_t)inpage * p.v_stride_t;
+                const int blk = min(max(__builtin_amdgcn_readfirstlane(blk_raw), 0), p.num_blocks - 1);
+                first = (int64_t)blk * stride_block + (int64_t)(kt * kBN % p.page_size) * stride_t;
             } else {
-                koff = (int64_t)(k0 + kt * kBN) * p.k_stride_t;
-                voff = (int64_t)(k0 + kt * kBN) * p.v_stride_t;
+                first = (int64_t)(k0 + kt * kBN) * stride_t;
             }
-            const uint8_t *kb = reinterpret_cast<const uint8_t *>(kbase + koff);
-            const uint8_t *vb = reinterpret_cast<const uint8_t *>(vbase + voff);
+            const uint8_t *src = reinterpret_cast<const uint8_t *>(base + first);
 #pragma unroll
-            for (int i = 0; i < Cfg::kKLoads; ++i)
-                if (k_on[i]) load_lds_base(k_lds + i * 4096u, k_off[i], kb);
-#pragma unroll
-            for (int i = 0; i < Cfg::kVLoads; ++i)
-                if (v_on[i]) load_lds_base(v_lds + i * 4096u, v_off[i], vb);
+            for (int i = 0; i < Cfg::kLoads; ++i)
+                if (on[i % Cfg::kPatterns]) load_lds_base(dst + i * 4096u, off[i % Cfg::kPatterns], uniform(src + (int64_t)(i * Cfg::kLoadRows) * stride_t * 2));
             return;
         }
         // The ragged end of a sequence, or pages that a tile straddles: an address per row.  All addresses first (their
         // page-table entries are then fetched together), the loads behind them.
-        auto row_addr = [&](int row, bool is_k) -> const uint8_t * {
-            const int key = min(kt * kBN + row, Sk - 1);
-            int64_t off;
+        const uint8_t *addr[Cfg::kLoads];
+#pragma unroll
+        for (int i = 0; i < Cfg::kLoads; ++i) {
+            const int key = min(kt * kBN + t_row + i * Cfg::kLoadRows, Sk - 1);
+            int64_t at;
             if constexpr (PAGED) {
                 const int page = key / p.page_size;
                 int blk = bt_row[page];
                 blk = min(max(blk, 0), p.num_blocks - 1);
-                const int inpage = key - page * p.page_size;
-                off = is_k ? (int64_t)blk * p.k_stride_block + (int64_t)inpage * p.k_stride_t
-                           : (int64_t)blk * p.v_stride_block + (int64_t)inpage * p.v_stride_t;
+                at = (int64_t)blk * stride_block + (int64_t)(key - page * p.page_size) * stride_t;
             } else {
-                off = (int64_t)(k0 + key) * (is_k ? p.k_stride_t : p.v_stride_t);
+                at = (int64_t)(k0 + key) * stride_t;
             }
-            return reinterpret_cast<const uint8_t *>((is_k ? kbase : vbase) + off);
-        };
-        const uint8_t *ka[Cfg::kKLoads], *va[Cfg::kVLoads];
+            addr[i] = reinterpret_cast<const uint8_t *>(base + at) + col_of(IS_K, i) * 16;
+        }
 #pragma unroll
-        for (int i = 0; i < Cfg::kKLoads; ++i) ka[i] = row_addr(k_row[i], true) + k_col[i];
-#pragma unroll
-        for (int i = 0; i < Cfg::kVLoads; ++i) va[i] = row_addr(v_row[i], false) + v_col[i];
-#pragma unroll
-        for (int i = 0; i < Cfg::kKLoads; ++i)
-            if (k_on[i]) load_lds_addr(k_lds + i * 4096u, ka[i]);
-#pragma unroll
-        for (int i = 0; i < Cfg::kVLoads; ++i)
-            if (v_on[i]) load_lds_addr(v_lds + i * 4096u, va[i]);
+        for (int i = 0; i < Cfg::kLoads; ++i)
+            if (on[i % Cfg::kPatterns]) load_lds_addr(dst + i * 4096u, addr[i]);
     };
     if constexpr (PART) {
         // the places of the pieces that nobody loads
-        for (int i = tid * 16; i < 2 * Cfg::kTileBytes; i += 256 * 16) *reinterpret_cast<u32x4_t *>(&s_k[0][0] + i) = u32x4_t{0, 0, 0, 0};
-        for (int i = tid * 16; i < 2 * Cfg::kVTileBytes; i += 256 * 16) *reinterpret_cast<u32x4_t *>(&s_v[0][0] + i) = u32x4_t{0, 0, 0, 0};
+        for (int i = tid * 16; i < (2 + Cfg::kVBufs) * Cfg::kTileBytes; i += 256 * 16) *reinterpret_cast<u32x4_t *>(&lds.k[0][0] + i) = u32x4_t{0, 0, 0, 0};
         __syncthreads();
     }
 
@@ -328,50 +336,78 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
 #pragma unroll
         for (int r = 0; r < 16; ++r) o_acc[t][r] = 0.f;
 
-    const int kt_begin = k_lo / kBN;
-    const int kt_end = (k_hi + kBN - 1) / kBN;
+    // (uniform, which the compiler cannot see behind the batch maximum that comes out of LDS)
+    const int kt_begin = __builtin_amdgcn_readfirstlane(k_lo / kBN);
+    const int kt_end = __builtin_amdgcn_readfirstlane((k_hi + kBN - 1) / kBN);
     const bool wave_live = __builtin_amdgcn_readfirstlane(R0 + wave * 32 < n_rows);
-    fetch_tile(kt_begin, 0);
+    const std::true_type K_TILE{};
+    const std::false_type V_TILE{};
+    // Step kt: behind the barrier in front of it K tile kt is there and every wave has used K tile kt - 1 and V tile kt - 1.  With
+    // one V buffer the V tile of the step itself is asked for here, and waited for (with a barrier) behind the softmax; with two
+    // it was asked for a step ago.
+    auto landed_but = [&](auto n_c) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n_c)::value) : "memory"); };
+    auto barrier = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int blk = page_of(kt_begin), blk_next = page_of(kt_begin + 1);
+    fetch(K_TILE, kt_begin, blk);
+    if (Cfg::kVBufs == 2) fetch(V_TILE, kt_begin, blk);
     tiles_landed();
-    __syncthreads();
+    barrier();
 
-    int cur = 0;
+    float16_t s[2];                 // scores of a tile: keys 0-31 and 32-63
+    u32x4_t ka[Cfg::kKSteps][2];
+    // LDS addresses of this lane's operand pieces in buffer 0: K row ln, piece lh (k-step t: XOR t << 5), V row tr_row, its 8
+    // bytes of column tile 0 (tile t: XOR t << 6)
+    const int tr_row = 4 * lh + ((lane & 15) >> 2);
+    const uint32_t k_lane = lds_of(&lds.k[0][0]) + (uint32_t)ln * Cfg::kRowBytes + ((uint32_t)Cfg::k_place(ln, lh) << 4);
+    const uint32_t v_lane = lds_of(&lds.v[0][0]) + (uint32_t)tr_row * Cfg::kRowBytes +
+                            ((uint32_t)Cfg::v_place(tr_row, ((lane >> 4) & 1) * 2 + ((lane >> 1) & 1)) << 4) + (uint32_t)(lane & 1) * 8u;
+    auto in_buffer = [](uint32_t addr, int buf) -> uint32_t {   // (made anew each step: kept, the address of every operand would take a register)
+        addr += (uint32_t)buf * Cfg::kTileBytes;
+        asm volatile("" : "+v"(addr));
+        return addr;
+    };
+    uint32_t k_at = 0;
+    auto read_k = [&](int t) {
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+            ka[t][tt] = *(const __attribute__((address_space(3))) u32x4_t *)(uintptr_t)((k_at ^ (uint32_t)(t << 5)) + tt * 32 * Cfg::kRowBytes);
+    };
+    constexpr int kPf = 2;          // operand reads run kPf k-steps ahead of the MFMAs that use them
+    const float16_t zero16 = {};
+    auto score_step = [&](int t) {
+        if (t + kPf < Cfg::kKSteps) read_k(t + kPf);
+        s[0] = mfma32<T>(ka[t][0], qreg[t], t == 0 ? zero16 : s[0]);
+        s[1] = mfma32<T>(ka[t][1], qreg[t], t == 0 ? zero16 : s[1]);
+    };
     for (int kt = kt_begin; kt < kt_end; ++kt) {
         const bool more = kt + 1 < kt_end;
-        if (more) fetch_tile(kt + 1, cur ^ 1);   // the other buffer: its readers passed the barrier that ended the last step
+        if (Cfg::kVBufs == 1) fetch(V_TILE, kt, blk);
+        if (more) {
+            fetch(K_TILE, kt + 1, blk_next);
+            if (Cfg::kVBufs == 2) fetch(V_TILE, kt + 1, blk_next);
+        }
+        blk = blk_next;
+        blk_next = page_of(kt + 2);
         __builtin_amdgcn_sched_barrier(0);
-
+        u32x4_t pk[2][2];
         // a wave whose 32 rows all lie past the block's end (short blocks: a decode row among prompt chunks
         // fills four rows of one wave) only helps to move the tiles, and leaves the matrix pipe to the others
         if (wave_live) {
         // ---- S^T = K Q^T for the two 32-key halves of the tile
         // the wave in a matrix phase goes first: its MFMAs then issue back to back and the vector work of the SIMD's other
-        // wave fills the gaps between them (c5: 870 -> 856 us)
+        // waves fills the gaps between them (c5: 870 -> 856 us)
         __builtin_amdgcn_s_setprio(1);
-        float16_t s[2];
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[tt][r] = 0.f;
-        // operand reads run kPf k-steps ahead of the MFMAs that use them
-        constexpr int kPf = 2;
-        u32x4_t ka[Cfg::kKSteps][2];
-        auto read_k = [&](int t) {
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const int row = tt * 32 + ln;
-                ka[t][tt] = *reinterpret_cast<const u32x4_t *>(
-                    &s_k[cur][row * (D * 2) + (((t * 2 + lh) ^ (row & Cfg::kSwz)) << 4)]);
-            }
-        };
+        k_at = in_buffer(k_lane, kt & 1);
 #pragma unroll
         for (int t = 0; t < kPf; ++t) read_k(t);
 #pragma unroll
         for (int t = 0; t < Cfg::kKSteps; ++t) {
             if (PART && t * 16 >= hd) break;   // wave-uniform; at least D/2 columns are live
-            if (t + kPf < Cfg::kKSteps) read_k(t + kPf);
-            s[0] = mfma32<T>(ka[t][0], qreg[t], s[0]);
-            s[1] = mfma32<T>(ka[t][1], qreg[t], s[1]);
+            score_step(t);
             __builtin_amdgcn_sched_barrier(0);
         }
 
@@ -381,63 +417,53 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
         const int tile0 = kt * kBN;
         // wave-uniform by construction; made scalar so the two softmax paths stay separate branches
         const bool need_mask = __builtin_amdgcn_readfirstlane((tile0 < wave_klo_max) || (tile0 + kBN - 1 > wave_khi_min));
-        // Fast path (no softcap, no element masks, positive scale): the maximum is taken on the raw
-        // scores and the scale rides in the exponent's fused multiply-add.
-        const bool raw_path = !SOFTCAP && !need_mask && p.scale_log2 > 0.f;
-        float mloc = -INFINITY;
-        if (raw_path) {
+        // The scores are left unscaled where that can be (no softcap, positive scale): the maximum is taken on them as they
+        // are, and the scale rides in the exponent's fused multiply-add.
+        if constexpr (SOFTCAP) {
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, s[tt][r]);
-            mloc *= p.scale_log2;
-        } else if (!SOFTCAP && need_mask) {
+                for (int r = 0; r < 16; ++r) {
+                    const float y = s[tt][r] * p.softcap_pre;
+                    const float e2 = __expf(2.f * y);
+                    s[tt][r] = p.softcap_post * (1.f - 2.f / (e2 + 1.f));
+                }
+        } else if (!(p.scale_log2 > 0.f)) {
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[tt][r] *= p.scale_log2;
+        }
+        const float scale = (!SOFTCAP && p.scale_log2 > 0.f) ? p.scale_log2 : 1.f;
+        if (need_mask) {
             // masked tile (the diagonal of a causal block, window edges, the ragged end): element r
             // of half tt is key tile0 + 4*lh + e(tt, r) with e a compile-time constant, so the
             // row's bounds are compared in tile coordinates; a side that cannot bite is skipped
             const int lo_rel = klo_r - tile0 - 4 * lh;
             const int hi_rel = khi_r - tile0 - 4 * lh;
-            const bool need_lo = __builtin_amdgcn_readfirstlane(tile0 < wave_klo_max);
-            if (!need_lo) {
-#pragma unroll
-                for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int e = tt * 32 + 8 * (r >> 2) + (r & 3);
-                        const float v = (e <= hi_rel) ? s[tt][r] * p.scale_log2 : -INFINITY;
-                        s[tt][r] = v;
-                        mloc = fmaxf(mloc, v);
-                    }
-            } else {
-#pragma unroll
-                for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int e = tt * 32 + 8 * (r >> 2) + (r & 3);
-                        const float v = (e >= lo_rel && e <= hi_rel) ? s[tt][r] * p.scale_log2 : -INFINITY;
-                        s[tt][r] = v;
-                        mloc = fmaxf(mloc, v);
-                    }
-            }
-        } else {
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    float v = s[tt][r];
-                    if constexpr (SOFTCAP) {
-                        const float y = v * p.softcap_pre;
-                        const float e2 = __expf(2.f * y);
-                        v = p.softcap_post * (1.f - 2.f / (e2 + 1.f));
-                    } else {
-                        v *= p.scale_log2;
-                    }
                     const int e = tt * 32 + 8 * (r >> 2) + (r & 3);
-                    v = (!need_mask || (e >= klo_r - tile0 - 4 * lh && e <= khi_r - tile0 - 4 * lh)) ? v : -INFINITY;
-                    s[tt][r] = v;
-                    mloc = fmaxf(mloc, v);
+                    s[tt][r] = (e <= hi_rel) ? s[tt][r] : -INFINITY;
                 }
+            if (__builtin_amdgcn_readfirstlane(tile0 < wave_klo_max)) {
+#pragma unroll
+                for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int e = tt * 32 + 8 * (r >> 2) + (r & 3);
+                        s[tt][r] = (e >= lo_rel) ? s[tt][r] : -INFINITY;
+                    }
+            }
         }
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, s[tt][r]);
+        mloc *= scale;
         mloc = halves_max(mloc);
         // The accumulator rescale is skipped for the whole wave when no row of it saw a new maximum
         // (most tiles once a row is a few hundred keys in).  m_run stays the exact running maximum,
@@ -456,18 +482,10 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
         }
         const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
         float psum = 0.f;
-        u32x4_t pk[2][2];
-        if (raw_path) {
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[tt][r] = fast_exp2(__builtin_fmaf(s[tt][r], p.scale_log2, -m_use));
-        } else {
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s[tt][r] = fast_exp2(s[tt][r] - m_use);
-        }
+            for (int r = 0; r < 16; ++r) s[tt][r] = fast_exp2(__builtin_fmaf(s[tt][r], scale, -m_use));
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt) {
 #pragma unroll
@@ -479,43 +497,54 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
         }
         l_run += psum;
 
+        }   // wave_live
+        if (Cfg::kVBufs == 1) {
+            // V tile kt (the loads of K tile kt + 1 behind it may still be on their way; with PART some of those are left out)
+            if (more && !PART) landed_but(std::integral_constant<int, Cfg::kLoads>{}); else tiles_landed();
+            barrier();
+        }
+        if (wave_live) {
         __builtin_amdgcn_s_setprio(1);
         // ---- O^T += V^T P^T, 16 keys per step.  The V^T operand comes from the transposing LDS read
         //      (ds_read_b64_tr_b16): in every 16-lane group, lane s points at 4 columns of key row
         //      s/4 and receives column s (of the group's 16) for the group's 4 key rows.  Column tile
         //      t is V columns t*32 .. t*32+31 in lane order.
         typedef short v4s_t __attribute__((ext_vector_type(4)));
-        const int tr_row = 4 * lh + ((lane & 15) >> 2);
-        const int tr_col = ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+        const uint32_t v_at = in_buffer(v_lane, kt & (Cfg::kVBufs - 1));
+        constexpr int kVG = Cfg::kMT < 4 ? Cfg::kMT : 4;         // column tiles whose operands are read together
+        constexpr int kVSteps = 4 * Cfg::kMT / kVG;
+        u32x4_t va[2][kVG];
+        auto read_v = [&](int step) {
+            const int ks = step / (Cfg::kMT / kVG), t0 = step % (Cfg::kMT / kVG) * kVG;
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+            for (int u = 0; u < kVG; ++u) {
+                if (PART && (t0 + u) * 32 >= hd) continue;
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                u32x4_t va[Cfg::kMT];
-#pragma unroll
-                for (int t = 0; t < Cfg::kMT; ++t)
-#pragma unroll
-                    for (int hv = 0; hv < 2; ++hv) {
-                        if (PART && t * 32 >= hd) continue;
-                        const int row = tt * 32 + 16 * ks + 8 * hv + tr_row;
-                        const v4s_t r4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                            (__attribute__((address_space(3))) v4s_t *)(&s_v[cur][row * Cfg::kVRowBytes + (t * 32 + tr_col) * 2]));
-                        const uint2 r2 = __builtin_bit_cast(uint2, r4);
-                        va[t][2 * hv] = r2.x;
-                        va[t][2 * hv + 1] = r2.y;
-                    }
-#pragma unroll
-                for (int t = 0; t < Cfg::kMT; ++t) {
-                    if (PART && t * 32 >= hd) continue;
-                    o_acc[t] = mfma32<T>(va[t], pk[tt][ks], o_acc[t]);
+                for (int hv = 0; hv < 2; ++hv) {
+                    const v4s_t r4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) v4s_t *)(uintptr_t)((v_at ^ (uint32_t)((t0 + u) << 6)) + (16 * ks + 8 * hv) * Cfg::kRowBytes));
+                    const uint2 r2 = __builtin_bit_cast(uint2, r4);
+                    va[step & 1][u][2 * hv] = r2.x;
+                    va[step & 1][u][2 * hv + 1] = r2.y;
                 }
             }
+        };
+        read_v(0);
+#pragma unroll
+        for (int step = 0; step < kVSteps; ++step) {
+            const int ks = step / (Cfg::kMT / kVG), t0 = step % (Cfg::kMT / kVG) * kVG;
+            if (step + 1 < kVSteps) read_v(step + 1);
+#pragma unroll
+            for (int u = 0; u < kVG; ++u) {
+                if (PART && (t0 + u) * 32 >= hd) continue;
+                o_acc[t0 + u] = mfma32<T>(va[step & 1][u], pk[ks >> 1][ks & 1], o_acc[t0 + u]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
         __builtin_amdgcn_s_setprio(0);
         }   // wave_live
-
         tiles_landed();
-        __syncthreads();
-        cur ^= 1;
+        barrier();
     }
 
     // ---- epilogue: O^T / l, store.  Register r of column tile t is V column
@@ -542,8 +571,8 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     // after the last barrier of the loop; each wave uses its own part, so no workgroup barrier) and
     // leaves as whole rows, 16 bytes per lane.
     constexpr int kStageRow = D * 2 + 16;                      // padded: the 8-byte writes of a column spread over the banks
-    static_assert(4 * 32 * kStageRow <= 2 * Cfg::kVTileBytes, "staging tile must fit the V tiles");
-    uint8_t *stage = &s_v[0][0] + wave * (32 * kStageRow);
+    static_assert(4 * 32 * kStageRow <= (2 + Cfg::kVBufs) * Cfg::kTileBytes, "staging tile must fit the tiles");
+    uint8_t *stage = &lds.k[0][0] + wave * (32 * kStageRow);
 #pragma unroll
     for (int t = 0; t < Cfg::kMT; ++t)
 #pragma unroll
@@ -575,11 +604,9 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
 }
 
 template <typename T, int D, bool PAGED, bool SOFTCAP, bool EXT, bool PART>
-__global__ void __launch_bounds__(256, (D <= 128) ? 2 : 1) prefill_kernel(const PrefillParams p) {
-    using Cfg = PrefillCfg<D>;
-    __shared__ __attribute__((aligned(16))) uint8_t s_k[2][Cfg::kTileBytes];
-    __shared__ __attribute__((aligned(16))) uint8_t s_v[2][Cfg::kVTileBytes];
-    prefill_block<T, D, PAGED, SOFTCAP, EXT, PART>(p, blockIdx.x, -1, s_k, s_v);
+__global__ void __launch_bounds__(256, prefill_occupancy(D, PART)) prefill_kernel(const PrefillParams p) {
+    __shared__ PrefillTileLds<D> lds;
+    prefill_block<T, D, PAGED, SOFTCAP, EXT, PART>(p, blockIdx.x, -1, lds);
 }
 
 // The same blocks for a launch whose live sequences are known on the device only (token-major batches whose
@@ -590,10 +617,8 @@ __global__ void __launch_bounds__(256, (D <= 128) ? 2 : 1) prefill_kernel(const 
 // of a unit still meet in one L2, through one counter per XCD (p.list_state[1 + x], zeroed by the kernel that
 // wrote the list).  Every workgroup leaves when its counter passes the end of the list.
 template <typename T, int D, bool SOFTCAP, bool PART>
-__global__ void __launch_bounds__(256, (D <= 128) ? 2 : 1) prefill_list_kernel(const PrefillParams p) {
-    using Cfg = PrefillCfg<D>;
-    __shared__ __attribute__((aligned(16))) uint8_t s_k[2][Cfg::kTileBytes];
-    __shared__ __attribute__((aligned(16))) uint8_t s_v[2][Cfg::kVTileBytes];
+__global__ void __launch_bounds__(256, prefill_occupancy(D, true)) prefill_list_kernel(const PrefillParams p) {
+    __shared__ PrefillTileLds<D> lds;
     __shared__ int s_item;
     const int n_long = p.list_state[0];
     const int heads_per_unit = (p.pack > 1) ? 1 : p.group;
@@ -604,9 +629,9 @@ __global__ void __launch_bounds__(256, (D <= 128) ? 2 : 1) prefill_list_kernel(c
         __syncthreads();   // the last block's LDS tiles and s_item are free
         if (threadIdx.x == 0) s_item = atomicAdd(&p.list_state[1 + x], 1);
         __syncthreads();
-        const int64_t bid = (int64_t)s_item * 8 + x;
+        const int64_t bid = (int64_t)__builtin_amdgcn_readfirstlane(s_item) * 8 + x;
         if (bid >= total) break;
-        prefill_block<T, D, true, SOFTCAP, true, PART>(p, (unsigned)bid, n_long, s_k, s_v);
+        prefill_block<T, D, true, SOFTCAP, true, PART>(p, (unsigned)bid, n_long, lds);
     }
 }
 
