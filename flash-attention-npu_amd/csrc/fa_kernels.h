@@ -200,8 +200,21 @@ inline int prefill_pack(int group, int max_seqlen_q) {
     const int64_t tiles_packed = ((int64_t)max_seqlen_q * group + kPrefillTileRows - 1) / kPrefillTileRows;
     return tiles_packed * 4 <= tiles_plain * 3 ? group : 1;
 }
-// Workgroups of the tiled forward that a compute unit holds.
-constexpr int prefill_wgs_per_cu(int headdim) { return headdim <= 128 ? 2 : 1; }
+// Workgroups of four waves (and so waves per SIMD) of the tiled forward that a compute unit holds.  A wave alone takes 1.5 times as
+// long for a tile as its matrix and vector instructions need (operand reads, the barrier, the tile's arrival), and on a SIMD the
+// matrix instructions of one wave run beside the vector instructions of another, so one more wave is worth more than anything
+// it costs: at D = 128 a second barrier per tile, which one V buffer instead of two asks for (48 KB of LDS per workgroup), and
+// operand reads only two k-steps ahead.  Two / three waves at D = 128 (the former with both V buffers), three / four at D = 64,
+// TFLOP/s: 4 x 8192 tokens, 32q/8kv, bidirectional 993 / 1049 (d = 64: 864 / 882); 16 x 2048 causal 800 / 894; 4 x 4096, 32q/32kv
+// 895 / 987; us: 16 x 512..4096 causal 791.6 / 718.8, 80 x 3..350, 28q/4kv 85.9 / 78.3, 8 x 2050, 16q/16kv, d = 64, fp16 205.8 /
+// 198.8.  Random values hold the clock down (1.6-1.9 GHz; all-zero inputs run the same code 1.6 times as fast), so that half of the
+// saved cycles do not show.  `spare`: kernels that keep more beside the tile loop, a head dimension below D or a list of blocks.
+// (A list kernel of three waves spilled: 63 decode rows + a 1024-token chunk 592 us against 525.)
+constexpr int prefill_wgs_resident(int d, bool spare) { return d == 64 ? 4 - spare : d == 128 ? 3 - spare : 1; }
+// ... by head dimension
+constexpr int prefill_wgs_per_cu(int headdim) {
+    return headdim <= 64 ? prefill_wgs_resident(64, headdim < 64) : headdim <= 128 ? prefill_wgs_resident(128, headdim < 128) : 1;
+}
 // Causal launches that prefill_pack() leaves unpacked: whether the heads of a group share the tiles all the same.  The 128
 // rows of a tile are then 128 / group queries of all the heads rather than 128 queries of one, so that a tile's keys end
 // closer behind its queries (half a tile of hidden keys per row less at a group of 4) and short sequences fill their
@@ -214,7 +227,7 @@ constexpr int prefill_wgs_per_cu(int headdim) { return headdim <= 128 ? 2 : 1; }
 // 53.2 / 51.2).
 inline bool prefill_pack_causal(int group, int nheads, int max_seqlen_q, int total_q, int headdim, int num_cus) {
     return group > 1 && group <= kPrefillTileRows && (int64_t)max_seqlen_q * group < (1ll << 30) &&
-           (int64_t)total_q * nheads >= 2ll * num_cus * prefill_wgs_per_cu(headdim) * kPrefillTileRows;
+           (int64_t)total_q * nheads >= 2ll * num_cus * (headdim <= 128 ? 2 : 1) * kPrefillTileRows;
 }
 // Heads per tile, tiles of a unit that are neighbours in the launch order, tiles of a unit.  causal_packs: the launch may follow
 // prefill_pack_causal() (causal, no key ranges, no device-side list).

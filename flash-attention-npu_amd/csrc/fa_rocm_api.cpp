@@ -408,8 +408,16 @@ int fa_rocm_plan_kvcache(const fa_kvcache_args *a, int num_cus, fa_split_plan *p
             n = a->num_splits;
         } else if (a->num_splits == 0) {
             const int64_t tiles = (int64_t)a->batch * fa::prefill_tiles(a->nheads, a->nheads_k, a->seqlen_q);
-            const int64_t slots = (int64_t)num_cus * fa::prefill_wgs_per_cu(a->headdim_qk);
-            if (tiles * 2 <= slots) n = (slots + tiles - 1) / tiles;
+            auto ranges = [&](int per_cu) -> int64_t {
+                const int64_t slots = (int64_t)num_cus * per_cu;
+                return tiles * 2 <= slots ? (slots + tiles - 1) / tiles : 1;
+            };
+            n = ranges(fa::prefill_wgs_per_cu(a->headdim_qk));
+            // (no more than the static scratch holds where the ranges of two workgroups per compute unit fit it: callers that
+            // cannot allocate count on it)
+            const int64_t per_range = (int64_t)a->batch * a->nheads_k * (int64_t)slot_bytes;
+            const int64_t room = ((int64_t)FA_ROCM_STATIC_SCRATCH_BYTES - (int64_t)tall_q_bytes(a)) / std::max<int64_t>(per_range, 1);
+            if (n > room) n = std::max(std::min(n, ranges(a->headdim_qk <= 128 ? 2 : 1)), std::max<int64_t>(room, 1));
         }
         const int64_t most = (bound + 255) / 256;   // at least 256 keys (four tiles) per range
         if (n > most) n = most;
@@ -1056,10 +1064,12 @@ int fa_rocm_varlen_num_splits(const fa_varlen_args *a, int num_cus) {
     if (a->num_splits > 1) {
         n = a->num_splits;
     } else {
-        const int64_t slots = (int64_t)num_cus * fa::prefill_wgs_per_cu(a->headdim);
         // query blocks far shorter than the longest one on average (a prompt chunk among decode rows): the
-        // longest block is the critical path long before the tiles fill the device, so it is cut earlier
+        // longest block is the critical path long before the tiles fill the device, so it is cut earlier, for the two
+        // workgroups per compute unit of the kernel that takes such a batch from a list (20 decode rows + 2000 tokens that
+        // end 30000 keys: 1117 us with two ranges, 1180 with three)
         const bool uneven = uneven_blocks(a);
+        const int64_t slots = (int64_t)num_cus * (!uneven ? fa::prefill_wgs_per_cu(a->headdim) : a->headdim <= 128 ? 2 : 1);
         if (uneven) {
             if (tiles < 2 * slots) n = (2 * slots + tiles - 1) / tiles;
         } else if (tiles * 2 <= slots) {
@@ -1185,7 +1195,7 @@ int fa_rocm_varlen_fwd(const fa_varlen_args *a, void *stream_) {
         // the sequences left to the tiled kernel are listed on the device by the gather kernel
         pp.long_ids = sr.long_ids;
         pp.list_state = sr.list_state;
-        pp.list_wgs = cus * fa::prefill_wgs_per_cu(a->headdim);
+        pp.list_wgs = cus * fa::prefill_wgs_resident(fa::tile_headdim(a->headdim), true);
     }
     if (!w.decode_only) {
         const hipError_t e = fa::launch_prefill(pp, a->io_dtype, fa::tile_headdim(a->headdim), stream);

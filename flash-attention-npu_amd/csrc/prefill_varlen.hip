@@ -30,24 +30,13 @@ namespace fa {
 constexpr int kBM = 128;  // query rows per workgroup
 constexpr int kBN = 64;   // keys per tile
 
-// Workgroups (and so waves per SIMD) that a compute unit holds.  A wave alone takes 1.5 times as long for a tile as its matrix and
-// vector instructions need (operand reads, the barrier, the tile's arrival), and on a SIMD the matrix instructions of one wave
-// run beside the vector instructions of another, so one more wave is worth more than anything it costs: at D = 128 a second
-// barrier per tile, which one V buffer instead of two asks for (48 KB of LDS per workgroup), and operand reads only two k-steps
-// ahead.  Two / three waves at D = 128 (the former with both V buffers), three / four at D = 64, TFLOP/s: 4 x 8192 tokens, 32q/8kv,
-// bidirectional 993 / 1049 (d = 64: 864 / 882); 16 x 2048 causal 800 / 894; 4 x 4096, 32q/32kv 895 / 987; us: 16 x 512..4096 causal
-// 791.6 / 718.8, 80 x 3..350, 28q/4kv 85.9 / 78.3, 8 x 2050, 16q/16kv, d = 64, fp16 205.8 / 198.8.  Random values hold the
-// clock down (1.6-1.9 GHz; all-zero inputs run the same code 1.6 times as fast), so that half of the saved cycles do not show.
-// `spare`: kernels that keep more beside the tile loop (a head dimension below D, a list of blocks), which would spill.
-constexpr int prefill_occupancy(int d, bool spare) { return d == 64 ? 4 - spare : d == 128 ? 3 - spare : 1; }
-
 template <int D> struct PrefillCfg {
     static constexpr int kKSteps = D / 16;        // MFMA k-steps of QK^T
     static constexpr int kMT = D / 32;            // 32-column tiles of O^T
     static constexpr int kChunks = D / 8;         // 16-byte pieces per row
     static constexpr int kRowBytes = D * 2;
     static constexpr int kTileBytes = kBN * kRowBytes;
-    static constexpr int kVBufs = D == 128 ? 1 : 2;                // (see prefill_occupancy)
+    static constexpr int kVBufs = D == 128 ? 1 : 2;                // (see prefill_wgs_resident)
     // A tile is filled by loads that go from global memory straight to LDS (global_load_lds_dwordx4): one instruction
     // of a wave fills 64 consecutive 16-byte pieces, lane l the piece at the instruction's LDS base + 16 l, from
     // whatever address the lane names.  The four waves share the pieces of a tile, instruction by instruction.
@@ -62,10 +51,11 @@ template <int D> struct PrefillCfg {
     static constexpr int kPatterns = D == 256 ? 2 : 1;             // loads after which the places of a lane's pieces repeat
 };
 
-// K tiles: the one being read and the one on its way; V tiles likewise, or a single one (kVBufs)
+// K tiles: the one being read and the one on its way; V tiles likewise, or a single one (kVBufs).  Starts at a multiple of two
+// tiles: the buffer, and the place in a row, are chosen by XOR.
 template <int D> struct PrefillTileLds {
-    __attribute__((aligned(1024))) uint8_t k[2][PrefillCfg<D>::kTileBytes];   // (operand addresses are formed by XOR inside a row)
-    __attribute__((aligned(1024))) uint8_t v[PrefillCfg<D>::kVBufs][PrefillCfg<D>::kTileBytes];
+    uint8_t k[2][PrefillCfg<D>::kTileBytes];
+    uint8_t v[PrefillCfg<D>::kVBufs][PrefillCfg<D>::kTileBytes];
 };
 
 // EXT: packed heads and / or a split of the keys (p.pack, p.nsplits); without it both are compiled out
@@ -77,7 +67,8 @@ template <int D> struct PrefillTileLds {
 template <typename T, int D, bool PAGED, bool SOFTCAP, bool EXT, bool PART>
 __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsigned bid, const int n_long, PrefillTileLds<D> &lds) {
     using Cfg = PrefillCfg<D>;
-    const int tid = threadIdx.x;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // (a kernel that walks several blocks would keep what is made of it through all of them)
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lh = lane >> 5;   // half: MFMA k-slot
@@ -96,12 +87,21 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     const int hk = unit - z * p.nheads_k;
     const int zb = z / nsplits;
     const int split = z - zb * nsplits;
-    const int b = listed ? p.long_ids[zb] : zb;
-
+    // Lengths and tables do not change while the kernel runs and are read at the same place by every lane: scalar loads, which leave
+    // what follows from them in scalar registers.  They are asked for together, a trip to memory for all of them.
+    auto constant = [](const int32_t *ptr, int i) -> int { return ((const __attribute__((address_space(4))) int32_t *)(uintptr_t)ptr)[i]; };
+    auto scalar = [](int x) -> int { return __builtin_amdgcn_readfirstlane(x); };   // (values out of LDS)
+    const int b = listed ? constant(p.long_ids, zb) : zb;
     int q0, Sq, k0 = 0, Sk;
+    if constexpr (PAGED) {
+        Sk = constant(p.seqused_k, b);
+    } else {
+        k0 = constant(p.cu_seqlens_k, b);
+        Sk = constant(p.cu_seqlens_k, b + 1);
+    }
     if (p.cu_seqlens_q) {
-        q0 = p.cu_seqlens_q[b];
-        Sq = p.cu_seqlens_q[b + 1] - q0;
+        q0 = constant(p.cu_seqlens_q, b);
+        Sq = constant(p.cu_seqlens_q, b + 1) - q0;
     } else {
         q0 = 0;
         Sq = p.seqlen_q_fixed;
@@ -122,12 +122,10 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     }
     const int h_base = hk * p.group + ((pg > 1) ? 0 : head_in_unit);
     if constexpr (PAGED) {
-        Sk = p.seqused_k[b] + p.seqlen_k_add;
-        Sk = min(Sk, p.max_blocks * p.page_size);
+        Sk = min(Sk + p.seqlen_k_add, p.max_blocks * p.page_size);
     } else {
-        k0 = p.cu_seqlens_k[b];
-        Sk = p.cu_seqlens_k[b + 1] - k0;
-        if (p.seqused_k) Sk = max(0, min(Sk, p.seqused_k[b]));   // only the first seqused_k[b] keys of the sequence are used
+        Sk -= k0;
+        if (p.seqused_k) Sk = max(0, min(Sk, constant(p.seqused_k, b)));   // only the first seqused_k[b] keys of the sequence are used
     }
     // window normalisation: the varlen host passes max_seqlen_k as the reference does
     // (flash_api.cpp:938-943); the kvcache layout has the lengths on the device only, so the batch
@@ -135,13 +133,13 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     int wl = p.window_left, wr_eff = p.window_right;
     int norm_m = p.window_norm_m;
     if constexpr (PAGED) {
-        if (norm_m <= 0 && (wl >= 0 || wr_eff >= 0)) norm_m = block_max_keys(p.seqused_k, p.batch, p.seqlen_k_add);
+        if (norm_m <= 0 && (wl >= 0 || wr_eff >= 0)) norm_m = scalar(block_max_keys(p.seqused_k, p.batch, p.seqlen_k_add));
     }
     if (norm_m <= 0) norm_m = max(Sk, 1);
     normalize_window(wl, wr_eff, p.causal, norm_m);
     int batch_max = 0;
     if constexpr (PAGED) {
-        if (nsplits > 1) batch_max = min(block_max_keys(p.seqused_k, p.batch, p.seqlen_k_add), p.max_blocks * p.page_size);
+        if (nsplits > 1) batch_max = scalar(min(block_max_keys(p.seqused_k, p.batch, p.seqlen_k_add), p.max_blocks * p.page_size));
     }
     const int n_rows = Sq * pg;
     const int R0 = mb * kBM;
@@ -165,62 +163,75 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
         slot = ((int64_t)b * p.nheads_k + hk) * nsplits + split;
     }
 
-    const int my_R = min(R0 + wave * 32 + ln, n_rows - 1);   // rows past the end repeat the last one and are dropped
-    const bool row_ok = R0 + wave * 32 + ln < n_rows;
-    const int my_row = my_R / pg;                            // query position of this lane column
-    const int my_head = h_base + (my_R - my_row * pg);
-    const uint16_t *q_row = reinterpret_cast<const uint16_t *>(p.q) + (int64_t)b * p.q_stride_b +
-                            (int64_t)my_head * p.q_stride_h + (int64_t)(q0 + my_row) * p.q_stride_t;
-    uint16_t *o_row = reinterpret_cast<uint16_t *>(p.out) + (int64_t)b * p.o_stride_b + (int64_t)my_head * p.o_stride_h +
-                      (int64_t)(q0 + my_row) * p.o_stride_t;
-    float *lse_row = p.lse + (int64_t)b * p.lse_stride_b + (int64_t)my_head * p.lse_stride_h + q0 + my_row;
+    // Tile row R0 + i is query `pos` of head `head`; rows past the end (ok: false) repeat the last one and are dropped.  Worked out
+    // where it is needed: kept through the loop, it would take registers that the operands need.
+    const int r_lo = R0 / pg;                                // query positions of the block: r_lo .. r_hi
+    const int r_hi = (min(n_rows, R0 + kBM) - 1) / pg;
+    const uint32_t pg_inv = (EXT && pg > 1) ? 0xffffffffu / (uint32_t)pg + 1u : 0u;   // x / pg = the upper half of x * pg_inv for x < pg + 128
+    struct TileRow {
+        int pos, head;
+        bool ok;
+    };
+    auto tile_row = [&](int i) -> TileRow {
+        const int R = min(R0 + i, n_rows - 1);
+        TileRow t;
+        t.ok = R0 + i < n_rows;
+        t.pos = (EXT && pg > 1) ? r_lo + (int)__umulhi((uint32_t)(R - r_lo * pg), pg_inv) : R;
+        t.head = h_base + (R - t.pos * pg);
+        return t;
+    };
+    auto this_lane = [&]() -> int {                          // (found out anew, so that it need not be kept either)
+        int l;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+        return l;
+    };
+    auto my_row = [&](int l) -> TileRow { return tile_row(wave * 32 + (l & 31)); };   // the row of lane l's column
+    auto lse_of = [&](const TileRow &t) -> float * { return p.lse + (int64_t)b * p.lse_stride_b + (int64_t)t.head * p.lse_stride_h + q0 + t.pos; };
 
     // key range the whole block (query positions r_lo .. r_hi) can see
-    const int r_lo = R0 / pg;
-    const int r_hi = (min(n_rows, R0 + kBM) - 1) / pg;
     int k_lo = 0, k_hi = Sk;
     if (wl >= 0) k_lo = max(0, r_lo + off - wl);
     if (wr_eff >= 0) k_hi = min(Sk, r_hi + off + wr_eff + 1);
     k_lo = max(k_lo, range_lo);
     k_hi = max(min(k_hi, range_hi), 0);
-    // where this lane's row goes when the unit is cut: row (query, head of the group) of the slot
-    float *part_row = nullptr, *part_lse = nullptr;
-    if (!whole) {
+    // where a row goes when the unit is cut: row (query, head of the group) of the slot
+    auto part_of = [&](const TileRow &t) -> int64_t {
         // kvcache layout: (batch row, kv head, range, query x head of the group); token-major q: (token, head, range)
-        const int64_t prow = p.cu_seqlens_q ? ((int64_t)(q0 + my_row) * p.nheads + my_head) * nsplits + split
-                                            : slot * p.rows + (int64_t)my_row * p.group + (my_head - hk * p.group);
-        part_row = p.o_partial + prow * D;
-        part_lse = p.lse_partial + prow;
-    }
+        return p.cu_seqlens_q ? ((int64_t)(q0 + t.pos) * p.nheads + t.head) * nsplits + split
+                              : slot * p.rows + (int64_t)t.pos * p.group + (t.head - hk * p.group);
+    };
 
     if (k_hi <= k_lo) {
         // nothing visible for the whole block: out = 0, lse = +inf
-        if (row_ok && whole) {
+        const TileRow t = my_row(lane);
+        if (t.ok && whole) {
+            uint16_t *o_row = reinterpret_cast<uint16_t *>(p.out) + (int64_t)b * p.o_stride_b + (int64_t)t.head * p.o_stride_h +
+                              (int64_t)(q0 + t.pos) * p.o_stride_t;
             for (int c = lh * (D / 2); c < min((lh + 1) * (D / 2), hd); c += 8) store16(o_row + c, u32x4_t{0, 0, 0, 0});
-            if (lh == 0) *lse_row = INFINITY;
-        } else if (row_ok) {
+            if (lh == 0) *lse_of(t) = INFINITY;
+        } else if (t.ok) {
+            float *part_row = p.o_partial + part_of(t) * D;
             for (int c = lh * (D / 2); c < (lh + 1) * (D / 2); c += 4) *reinterpret_cast<float4 *>(part_row + c) = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (lh == 0) *part_lse = -INFINITY;
+            if (lh == 0) p.lse_partial[part_of(t)] = -INFINITY;
         }
         return;
     }
 
-    // per-lane visible interval of its row (inclusive bounds)
-    int klo_r = 0, khi_r = Sk - 1;
-    if (wl >= 0) klo_r = max(0, my_row + off - wl);
-    if (wr_eff >= 0) khi_r = min(Sk - 1, my_row + off + wr_eff);
-    klo_r = max(klo_r, range_lo);
-    khi_r = min(khi_r, range_hi - 1);
     // bounds that decide, per wave, whether a tile needs element masks
     const int rw0 = min(R0 + wave * 32, n_rows - 1) / pg;        // first and last query position of the wave
     const int rw1 = (min(n_rows, R0 + wave * 32 + 32) - 1) / pg;
     const int wave_klo_max = max(range_lo, (wl >= 0) ? max(0, rw1 + off - wl) : 0);
+    // the keys that any row of the wave sees: halves of a tile beyond them are left out
+    const int wave_klo_first = max(range_lo, (wl >= 0) ? max(0, rw0 + off - wl) : 0);
+    const int wave_khi_last = min(range_hi - 1, (wr_eff >= 0) ? min(Sk - 1, rw1 + off + wr_eff) : Sk - 1);
     const int wave_khi_min = min(range_hi - 1, (wr_eff >= 0) ? min(Sk - 1, rw0 + off + wr_eff) : Sk - 1);
 
     // Q^T operand: lane (lh, ln) holds row ln, elements t*16 + lh*8 .. +7
     u32x4_t qreg[Cfg::kKSteps];
     {
-        const uint16_t *src = q_row + lh * 8;
+        const TileRow row = my_row(lane);
+        const uint16_t *src = reinterpret_cast<const uint16_t *>(p.q) + (int64_t)b * p.q_stride_b + (int64_t)row.head * p.q_stride_h +
+                              (int64_t)(q0 + row.pos) * p.q_stride_t + lh * 8;
 #pragma unroll
         for (int t = 0; t < Cfg::kKSteps; ++t) {
             if (PART && t * 16 + lh * 8 >= hd) {
@@ -228,7 +239,7 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
                 continue;
             }
             qreg[t] = load16(src + t * 16);
-            if (!row_ok) qreg[t] = u32x4_t{0, 0, 0, 0};
+            if (!row.ok) qreg[t] = u32x4_t{0, 0, 0, 0};
         }
     }
 
@@ -241,19 +252,19 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     // place c' holds the row's piece k_place(row, c') or v_place(row, c') (their own inverses).
     // Rows past the last key re-read the last key (never memory nobody wrote; they are masked); with PART the pieces
     // behind the head dimension are not loaded: their places hold the zeros written when the block started.
-    const int t_row = (64 * wave + lane) / Cfg::kChunks;      // of load 0; load i: kLoadRows * i rows further on
+    auto t_row = [&](int l) -> int { return (64 * wave + l) / Cfg::kChunks; };   // lane l's row of load 0; load i: kLoadRows * i rows on
     uint32_t k_off[Cfg::kPatterns], v_off[Cfg::kPatterns];    // offsets of load 0 (1) in an interior tile: one wave-uniform base serves all lanes
     bool k_on[Cfg::kPatterns], v_on[Cfg::kPatterns];
-    auto col_of = [&](bool is_k, int i) -> int {              // the lane's piece in the row of load i
-        const int c = lane % Cfg::kChunks, row = t_row + i * Cfg::kLoadRows;
+    auto col_of = [&](bool is_k, int i, int l) -> int {       // its piece in the row of load i
+        const int c = l % Cfg::kChunks, row = t_row(l) + i * Cfg::kLoadRows;
         return is_k ? Cfg::k_place(row, c) : Cfg::v_place(row, c);
     };
 #pragma unroll
     for (int i = 0; i < Cfg::kPatterns; ++i) {
-        k_on[i] = !PART || col_of(true, i) * 8 < hd;
-        v_on[i] = !PART || col_of(false, i) * 8 < hd;
-        k_off[i] = (uint32_t)t_row * (uint32_t)p.k_stride_t * 2u + col_of(true, i) * 16;
-        v_off[i] = (uint32_t)t_row * (uint32_t)p.v_stride_t * 2u + col_of(false, i) * 16;
+        k_on[i] = !PART || col_of(true, i, lane) * 8 < hd;
+        v_on[i] = !PART || col_of(false, i, lane) * 8 < hd;
+        k_off[i] = (uint32_t)t_row(lane) * (uint32_t)p.k_stride_t * 2u + col_of(true, i, lane) * 16;
+        v_off[i] = (uint32_t)t_row(lane) * (uint32_t)p.v_stride_t * 2u + col_of(false, i, lane) * 16;
     }
     auto lds_of = [](const void *ptr) -> uint32_t { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void *)ptr; };
     // The loads are written out: the compiler would wait for such a load in front of every LDS read that follows (it
@@ -270,58 +281,98 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
                                                  (uint32_t)__builtin_amdgcn_readfirstlane((int)x));
     };
     auto tiles_landed = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
-    // page of tile kt, for tiles that lie inside one (asked for a step before its loads: a scalar load, not one that would be
-    // waited for behind the tiles on their way)
-    const bool tile_in_page = !PAGED || p.page_size % kBN == 0;
-    auto page_of = [&](int kt) -> int {
-        if constexpr (!PAGED) return 0;
-        if (!tile_in_page) return 0;
-        const int page = min((kt * kBN) / p.page_size, p.max_blocks - 1);
-        return ((const __attribute__((address_space(4))) int32_t *)(uintptr_t)bt_row)[page];
+    // Where the tiles of a paged cache are.  A page holds a multiple of 32 keys (or, a page per sequence, all of them), so each half of
+    // a tile lies in one page, and the cursor keeps the addresses of both halves.  Inside a page a step moves them on by 64 rows; where a page ends they are made from the table, whose next two entries were asked for when the page before began: by
+    // scalar loads, which nobody has to wait for behind the tiles on their way.  (All of it is scalar work of every wave: the
+    // addresses made anew for every tile cost a paged launch 8 %, 4 x 2048 tokens over 8 K keys 1136 us against 1048 dense, now 1015
+    // against 985; a page
+    // looked up per row, with 32-row pages, 8 x 51 tokens over 4481..8962 keys, d = 64, 106 us against 79 now.)
+    const int page_rows = !PAGED || p.max_blocks == 1 ? INT32_MAX : p.page_size;
+    auto table = [&](int page) -> int { return constant(bt_row, min(page, p.max_blocks - 1)); };
+    struct Cursor {
+        const uint8_t *k[2], *v[2];     // first row of each half
+        int row[2], page;               // place of the halves in their pages (kept for the second one), its page
+        int id, ahead[2];               // table entry of that page and of the next two
     };
-    // K (IS_K) or V tile kt into its buffer
-    auto fetch = [&](auto is_k_c, int kt, int blk_raw) {
-        constexpr bool IS_K = decltype(is_k_c)::value;
-        const uint32_t dst = lds_of(IS_K ? &lds.k[kt & 1][0] : &lds.v[kt & (Cfg::kVBufs - 1)][0]) + (uint32_t)wave * 1024u;
-        const uint16_t *base = IS_K ? kbase : vbase;
-        const int64_t stride_t = IS_K ? p.k_stride_t : p.v_stride_t, stride_block = IS_K ? p.k_stride_block : p.v_stride_block;
-        const uint32_t(&off)[Cfg::kPatterns] = IS_K ? k_off : v_off;
-        const bool(&on)[Cfg::kPatterns] = IS_K ? k_on : v_on;
-        // A tile inside the sequence, of dense K/V or inside one page: one wave-uniform base serves all its loads
-        if (kt * kBN + kBN <= Sk && tile_in_page) {
-            int64_t first;
-            if constexpr (PAGED) {
-                const int blk = min(max(__builtin_amdgcn_readfirstlane(blk_raw), 0), p.num_blocks - 1);
-                first = (int64_t)blk * stride_block + (int64_t)(kt * kBN % p.page_size) * stride_t;
-            } else {
-                first = (int64_t)(k0 + kt * kBN) * stride_t;
-            }
-            const uint8_t *src = reinterpret_cast<const uint8_t *>(base + first);
-#pragma unroll
-            for (int i = 0; i < Cfg::kLoads; ++i)
-                if (on[i % Cfg::kPatterns]) load_lds_base(dst + i * 4096u, off[i % Cfg::kPatterns], uniform(src + (int64_t)(i * Cfg::kLoadRows) * stride_t * 2));
+    const int64_t k_row = p.k_stride_t * 2, v_row = p.v_stride_t * 2;   // bytes
+    auto set_half = [&](Cursor &c, int h, int id) {
+        const int64_t block = min(max(__builtin_amdgcn_readfirstlane(id), 0), p.num_blocks - 1);
+        c.k[h] = uniform(reinterpret_cast<const uint8_t *>(kbase) + c.row[h] * k_row + block * p.k_stride_block * 2);
+        c.v[h] = uniform(reinterpret_cast<const uint8_t *>(vbase) + c.row[h] * v_row + block * p.v_stride_block * 2);
+    };
+    auto first_tile = [&](int kt) -> Cursor {
+        Cursor c = {};
+        if constexpr (PAGED) {
+            const int page0 = kt * kBN / page_rows;
+            c.page = (kt * kBN + 32) / page_rows;
+            c.row[0] = kt * kBN - page0 * page_rows;
+            c.row[1] = kt * kBN + 32 - c.page * page_rows;
+            c.id = table(c.page);
+            c.ahead[0] = table(c.page + 1);
+            c.ahead[1] = table(c.page + 2);
+            set_half(c, 0, table(page0));
+            set_half(c, 1, c.id);
+        }
+        return c;
+    };
+    auto advance = [&](Cursor &c) {
+        if constexpr (!PAGED) return;
+        if (c.row[1] + kBN < page_rows) {
+            // (the first half may have come from the page before)
+            c.row[1] += kBN;
+            c.k[1] += kBN * k_row;
+            c.v[1] += kBN * v_row;
+            c.k[0] = c.k[1] - 32 * k_row;
+            c.v[0] = c.v[1] - 32 * v_row;
             return;
         }
-        // The ragged end of a sequence, or pages that a tile straddles: an address per row.  All addresses first (their
-        // page-table entries are then fetched together), the loads behind them.
-        const uint8_t *addr[Cfg::kLoads];
+        // the halves stand 32 and 64 rows behind the second half of the tile before
+        const int old = c.page;
+        int at = c.row[1];
 #pragma unroll
-        for (int i = 0; i < Cfg::kLoads; ++i) {
-            const int key = min(kt * kBN + t_row + i * Cfg::kLoadRows, Sk - 1);
-            int64_t at;
-            if constexpr (PAGED) {
-                const int page = key / p.page_size;
-                int blk = bt_row[page];
-                blk = min(max(blk, 0), p.num_blocks - 1);
-                at = (int64_t)blk * stride_block + (int64_t)(key - page * p.page_size) * stride_t;
-            } else {
-                at = (int64_t)(k0 + key) * stride_t;
+        for (int h = 0; h < 2; ++h) {
+            at += 32;
+            if (at >= page_rows) {
+                at -= page_rows;
+                ++c.page;
             }
-            addr[i] = reinterpret_cast<const uint8_t *>(base + at) + col_of(IS_K, i) * 16;
+            c.row[h] = at;
+            set_half(c, h, c.page == old ? c.id : c.ahead[c.page == old + 1 ? 0 : 1]);
         }
+        if (c.page != old) {
+            c.id = c.ahead[c.page == old + 1 ? 0 : 1];
+            c.ahead[0] = table(c.page + 1);
+            c.ahead[1] = table(c.page + 2);
+        }
+    };
+    // K (IS_K) or V tile kt into its buffer
+    auto fetch = [&](auto is_k_c, int kt, const uint8_t *const (&half)[2]) {
+        constexpr bool IS_K = decltype(is_k_c)::value;
+        const uint32_t dst = lds_of(IS_K ? &lds.k[kt & 1][0] : &lds.v[kt & (Cfg::kVBufs - 1)][0]) + (uint32_t)wave * 1024u;
+        const int64_t row_bytes = IS_K ? k_row : v_row;
+        const uint32_t(&off)[Cfg::kPatterns] = IS_K ? k_off : v_off;
+        const bool(&on)[Cfg::kPatterns] = IS_K ? k_on : v_on;
+        const int last = Sk - 1 - kt * kBN;                   // last written key relative to the tile (>= 0)
+        static_assert(32 % Cfg::kLoadRows == 0, "a load lies in one half");
+        const uint8_t *dense = nullptr;                       // (two multiplications: running pointers would take scalar registers)
+        if constexpr (!PAGED) dense = reinterpret_cast<const uint8_t *>(IS_K ? kbase : vbase) + (k0 + kt * kBN) * row_bytes;
+        auto from = [&](int h) -> const uint8_t * { return PAGED ? half[h] : dense + 32 * h * row_bytes; };
+        if (last >= kBN - 1) {
 #pragma unroll
-        for (int i = 0; i < Cfg::kLoads; ++i)
-            if (on[i % Cfg::kPatterns]) load_lds_addr(dst + i * 4096u, addr[i]);
+            for (int i = 0; i < Cfg::kLoads; ++i) {
+                const int row = i * Cfg::kLoadRows, h = row / 32;   // first row of the load over all waves
+                if (on[i % Cfg::kPatterns]) load_lds_base(dst + i * 4096u, off[i % Cfg::kPatterns], from(h) + (row - 32 * h) * row_bytes);
+            }
+        } else {
+            // the ragged end of a sequence: rows past the last key re-read it
+            const int l = this_lane();
+#pragma unroll
+            for (int i = 0; i < Cfg::kLoads; ++i) {
+                const int row = i * Cfg::kLoadRows, h = last < 32 * (row / 32) ? 0 : row / 32;
+                if (on[i % Cfg::kPatterns])
+                    load_lds_addr(dst + i * 4096u, from(h) + (min(t_row(l) + row, last) - 32 * h) * row_bytes + col_of(IS_K, i, l) * 16);
+            }
+        }
     };
     if constexpr (PART) {
         // the places of the pieces that nobody loads
@@ -351,183 +402,187 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     };
-    int blk = page_of(kt_begin), blk_next = page_of(kt_begin + 1);
-    fetch(K_TILE, kt_begin, blk);
-    if (Cfg::kVBufs == 2) fetch(V_TILE, kt_begin, blk);
+    Cursor next = first_tile(kt_begin);
+    fetch(K_TILE, kt_begin, next.k);
+    if (Cfg::kVBufs == 2) fetch(V_TILE, kt_begin, next.v);
+    const uint8_t *v_here[2] = {next.v[0], next.v[1]};       // V tile kt
+    advance(next);
     tiles_landed();
     barrier();
 
     float16_t s[2];                 // scores of a tile: keys 0-31 and 32-63
     u32x4_t ka[Cfg::kKSteps][2];
-    // LDS addresses of this lane's operand pieces in buffer 0: K row ln, piece lh (k-step t: XOR t << 5), V row tr_row, its 8
+    // LDS addresses of this lane's operand pieces in the tile's buffer: K row ln, piece lh (k-step t: XOR t << 5), V row tr_row, its 8
     // bytes of column tile 0 (tile t: XOR t << 6)
     const int tr_row = 4 * lh + ((lane & 15) >> 2);
-    const uint32_t k_lane = lds_of(&lds.k[0][0]) + (uint32_t)ln * Cfg::kRowBytes + ((uint32_t)Cfg::k_place(ln, lh) << 4);
-    const uint32_t v_lane = lds_of(&lds.v[0][0]) + (uint32_t)tr_row * Cfg::kRowBytes +
+    uint32_t k_at = lds_of(&lds.k[0][0]) + (uint32_t)ln * Cfg::kRowBytes + ((uint32_t)Cfg::k_place(ln, lh) << 4);
+    uint32_t v_at = lds_of(&lds.v[0][0]) + (uint32_t)tr_row * Cfg::kRowBytes +
                             ((uint32_t)Cfg::v_place(tr_row, ((lane >> 4) & 1) * 2 + ((lane >> 1) & 1)) << 4) + (uint32_t)(lane & 1) * 8u;
-    auto in_buffer = [](uint32_t addr, int buf) -> uint32_t {   // (made anew each step: kept, the address of every operand would take a register)
-        addr += (uint32_t)buf * Cfg::kTileBytes;
-        asm volatile("" : "+v"(addr));
-        return addr;
-    };
-    uint32_t k_at = 0;
-    auto read_k = [&](int t) {
+    k_at += (uint32_t)(kt_begin & 1) * Cfg::kTileBytes;
+    v_at += (uint32_t)(kt_begin & (Cfg::kVBufs - 1)) * Cfg::kTileBytes;
+    auto read_k = [&](int t, int halves) {
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < halves; ++tt)
             ka[t][tt] = *(const __attribute__((address_space(3))) u32x4_t *)(uintptr_t)((k_at ^ (uint32_t)(t << 5)) + tt * 32 * Cfg::kRowBytes);
     };
     constexpr int kPf = 2;          // operand reads run kPf k-steps ahead of the MFMAs that use them
     const float16_t zero16 = {};
-    auto score_step = [&](int t) {
-        if (t + kPf < Cfg::kKSteps) read_k(t + kPf);
-        s[0] = mfma32<T>(ka[t][0], qreg[t], t == 0 ? zero16 : s[0]);
-        s[1] = mfma32<T>(ka[t][1], qreg[t], t == 0 ? zero16 : s[1]);
-    };
+    // Packed tiles and key ranges end anywhere in a key tile, and a wave's 128 / 4 / group queries end before those of the block:
+    // a half of a tile that no row of the wave sees is left out (its weights are zero).  80 x 3..350 tokens, 28q/4kv 77.8 -> 73.8 us,
+    // 16 x 512..4096, 32q/8kv 714 -> 705; without packing (one tile in 33 at 2050 keys) what it saves the second form of the step takes.
+    constexpr bool kHalves = EXT;
     for (int kt = kt_begin; kt < kt_end; ++kt) {
         const bool more = kt + 1 < kt_end;
-        if (Cfg::kVBufs == 1) fetch(V_TILE, kt, blk);
+        if (Cfg::kVBufs == 1) fetch(V_TILE, kt, v_here);
         if (more) {
-            fetch(K_TILE, kt + 1, blk_next);
-            if (Cfg::kVBufs == 2) fetch(V_TILE, kt + 1, blk_next);
+            fetch(K_TILE, kt + 1, next.k);
+            if (Cfg::kVBufs == 2) fetch(V_TILE, kt + 1, next.v);
         }
-        blk = blk_next;
-        blk_next = page_of(kt + 2);
         __builtin_amdgcn_sched_barrier(0);
         u32x4_t pk[2][2];
-        // a wave whose 32 rows all lie past the block's end (short blocks: a decode row among prompt chunks
-        // fills four rows of one wave) only helps to move the tiles, and leaves the matrix pipe to the others
-        if (wave_live) {
-        // ---- S^T = K Q^T for the two 32-key halves of the tile
-        // the wave in a matrix phase goes first: its MFMAs then issue back to back and the vector work of the SIMD's other
-        // waves fills the gaps between them (c5: 870 -> 856 us)
-        __builtin_amdgcn_s_setprio(1);
-        k_at = in_buffer(k_lane, kt & 1);
-#pragma unroll
-        for (int t = 0; t < kPf; ++t) read_k(t);
-#pragma unroll
-        for (int t = 0; t < Cfg::kKSteps; ++t) {
-            if (PART && t * 16 >= hd) break;   // wave-uniform; at least D/2 columns are live
-            score_step(t);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-
-        __builtin_amdgcn_s_setprio(0);
-        // ---- online softmax; lane column = query row, register r of half tt = key
-        //      kt*64 + tt*32 + 8*(r/4) + 4*lh + r%4
         const int tile0 = kt * kBN;
-        // wave-uniform by construction; made scalar so the two softmax paths stay separate branches
-        const bool need_mask = __builtin_amdgcn_readfirstlane((tile0 < wave_klo_max) || (tile0 + kBN - 1 > wave_khi_min));
-        // The scores are left unscaled where that can be (no softcap, positive scale): the maximum is taken on them as they
-        // are, and the scale rides in the exponent's fused multiply-add.
-        if constexpr (SOFTCAP) {
+        // Halves of the tile (32 keys each, the first one or both) that some row of the wave sees.  A wave without any (its 32 rows
+        // all lie past the block's end, as with a decode row among prompt chunks, or end in front of the tile) only helps to move
+        // the tiles, and leaves the matrix pipe to the others.
+        const int live = __builtin_amdgcn_readfirstlane(!wave_live || tile0 > wave_khi_last || tile0 + kBN <= wave_klo_first ? 0
+                                                        : kHalves && tile0 + 32 > wave_khi_last                            ? 1
+                                                                                                                           : 2);
+        auto weights = [&](auto halves_c) {
+            constexpr int H = decltype(halves_c)::value;
+            // ---- S^T = K Q^T for the 32-key halves of the tile.  The wave in a matrix phase goes first: its MFMAs then issue
+            // back to back and the vector work of the SIMD's other waves fills the gaps between them
+            __builtin_amdgcn_s_setprio(1);
+            asm volatile("" : "+v"(k_at));   // (opaque: kept from step to step, the address of every operand would take a register)
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
+            for (int t = 0; t < kPf; ++t) read_k(t, H);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float y = s[tt][r] * p.softcap_pre;
-                    const float e2 = __expf(2.f * y);
-                    s[tt][r] = p.softcap_post * (1.f - 2.f / (e2 + 1.f));
-                }
-        } else if (!(p.scale_log2 > 0.f)) {
+            for (int t = 0; t < Cfg::kKSteps; ++t) {
+                if (PART && t * 16 >= hd) break;   // wave-uniform; at least D/2 columns are live
+                if (t + kPf < Cfg::kKSteps) read_k(t + kPf, H);
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
+                for (int tt = 0; tt < H; ++tt) s[tt] = mfma32<T>(ka[t][tt], qreg[t], t == 0 ? zero16 : s[tt]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+
+            __builtin_amdgcn_s_setprio(0);
+            // ---- online softmax; lane column = query row, register r of half tt = key
+            //      kt*64 + tt*32 + 8*(r/4) + 4*lh + r%4
+            // wave-uniform by construction; made scalar so the two softmax paths stay separate branches
+            const bool need_mask = __builtin_amdgcn_readfirstlane((tile0 < wave_klo_max) || (tile0 + kBN - 1 > wave_khi_min));
+            // The scores are left unscaled where that can be (no softcap, positive scale): the maximum is taken on them as they
+            // are, and the scale rides in the exponent's fused multiply-add.
+            if constexpr (SOFTCAP) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[tt][r] *= p.scale_log2;
-        }
-        const float scale = (!SOFTCAP && p.scale_log2 > 0.f) ? p.scale_log2 : 1.f;
-        if (need_mask) {
-            // masked tile (the diagonal of a causal block, window edges, the ragged end): element r
-            // of half tt is key tile0 + 4*lh + e(tt, r) with e a compile-time constant, so the
-            // row's bounds are compared in tile coordinates; a side that cannot bite is skipped
-            const int lo_rel = klo_r - tile0 - 4 * lh;
-            const int hi_rel = khi_r - tile0 - 4 * lh;
+                for (int tt = 0; tt < H; ++tt)
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt)
+                    for (int r = 0; r < 16; ++r) {
+                        const float y = s[tt][r] * p.softcap_pre;
+                        const float e2 = __expf(2.f * y);
+                        s[tt][r] = p.softcap_post * (1.f - 2.f / (e2 + 1.f));
+                    }
+            } else if (!(p.scale_log2 > 0.f)) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int e = tt * 32 + 8 * (r >> 2) + (r & 3);
-                    s[tt][r] = (e <= hi_rel) ? s[tt][r] : -INFINITY;
-                }
-            if (__builtin_amdgcn_readfirstlane(tile0 < wave_klo_max)) {
+                for (int tt = 0; tt < H; ++tt)
 #pragma unroll
-                for (int tt = 0; tt < 2; ++tt)
+                    for (int r = 0; r < 16; ++r) s[tt][r] *= p.scale_log2;
+            }
+            const float scale = (!SOFTCAP && p.scale_log2 > 0.f) ? p.scale_log2 : 1.f;
+            if (need_mask) {
+                // masked tile (the diagonal of a causal block, window edges, the ragged end): element r
+                // of half tt is key tile0 + 4*lh + e(tt, r) with e a compile-time constant, so the
+                // row's bounds are compared in tile coordinates; a side that cannot bite is skipped
+                const int l = this_lane(), at = my_row(l).pos + off, first = tile0 + 4 * (l >> 5);
+                const int lo_rel = max(range_lo, (wl >= 0) ? at - wl : 0) - first;
+                const int hi_rel = min(range_hi - 1, (wr_eff >= 0) ? min(Sk - 1, at + wr_eff) : Sk - 1) - first;
+#pragma unroll
+                for (int tt = 0; tt < H; ++tt)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const int e = tt * 32 + 8 * (r >> 2) + (r & 3);
-                        s[tt][r] = (e >= lo_rel) ? s[tt][r] : -INFINITY;
+                        s[tt][r] = (e <= hi_rel) ? s[tt][r] : -INFINITY;
                     }
+                if (__builtin_amdgcn_readfirstlane(tile0 < wave_klo_max)) {
+#pragma unroll
+                    for (int tt = 0; tt < H; ++tt)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            const int e = tt * 32 + 8 * (r >> 2) + (r & 3);
+                            s[tt][r] = (e >= lo_rel) ? s[tt][r] : -INFINITY;
+                        }
+                }
             }
-        }
-        float mloc = -INFINITY;
+            float mloc = -INFINITY;
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+            for (int tt = 0; tt < H; ++tt)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, s[tt][r]);
-        mloc *= scale;
-        mloc = halves_max(mloc);
-        // The accumulator rescale is skipped for the whole wave when no row of it saw a new maximum
-        // (most tiles once a row is a few hundred keys in).  m_run stays the exact running maximum,
-        // so the largest P of a row is exactly 1 as in the reference's golden.
-        const bool bump = mloc > m_run;   // false for fully hidden tiles
-        if (__any(bump)) {
-            const float m_new = bump ? mloc : m_run;
-            const float m_new_use = (m_new == -INFINITY) ? 0.f : m_new;
-            const float alpha = bump ? fast_exp2(m_run - m_new_use) : 1.f;
-            m_run = m_new;
-            l_run *= alpha;
+                for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, s[tt][r]);
+            mloc *= scale;
+            mloc = halves_max(mloc);
+            // The accumulator rescale is skipped for the whole wave when no row of it saw a new maximum
+            // (most tiles once a row is a few hundred keys in).  m_run stays the exact running maximum,
+            // so the largest P of a row is exactly 1 as in the reference's golden.
+            const bool bump = mloc > m_run;   // false for fully hidden tiles
+            if (__any(bump)) {
+                const float m_new = bump ? mloc : m_run;
+                const float m_new_use = (m_new == -INFINITY) ? 0.f : m_new;
+                const float alpha = bump ? fast_exp2(m_run - m_new_use) : 1.f;
+                m_run = m_new;
+                l_run *= alpha;
 #pragma unroll
-            for (int t = 0; t < Cfg::kMT; ++t)
+                for (int t = 0; t < Cfg::kMT; ++t)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) o_acc[t][r] *= alpha;
-        }
-        const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
-        float psum = 0.f;
+                    for (int r = 0; r < 16; ++r) o_acc[t][r] *= alpha;
+            }
+            const float m_use = (m_run == -INFINITY) ? 0.f : m_run;
+            float psum = 0.f;
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+            for (int tt = 0; tt < H; ++tt)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[tt][r] = fast_exp2(__builtin_fmaf(s[tt][r], scale, -m_use));
+                for (int r = 0; r < 16; ++r) s[tt][r] = fast_exp2(__builtin_fmaf(s[tt][r], scale, -m_use));
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
+            for (int tt = 0; tt < H; ++tt) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) psum += s[tt][r];
+                for (int r = 0; r < 16; ++r) psum += s[tt][r];
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
+                for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                for (int u = 0; u < 4; ++u) pk[tt][ks][u] = pack2<T>(s[tt][8 * ks + 2 * u], s[tt][8 * ks + 2 * u + 1]);
-        }
-        l_run += psum;
-
-        }   // wave_live
+                    for (int u = 0; u < 4; ++u) pk[tt][ks][u] = pack2<T>(s[tt][8 * ks + 2 * u], s[tt][8 * ks + 2 * u + 1]);
+            }
+            l_run += psum;
+        };
+        if (live == 2) weights(std::integral_constant<int, 2>{});
+        if (kHalves && live == 1) weights(std::integral_constant<int, 1>{});
         if (Cfg::kVBufs == 1) {
             // V tile kt (the loads of K tile kt + 1 behind it may still be on their way; with PART some of those are left out)
             if (more && !PART) landed_but(std::integral_constant<int, Cfg::kLoads>{}); else tiles_landed();
             barrier();
         }
-        if (wave_live) {
-        __builtin_amdgcn_s_setprio(1);
-        // ---- O^T += V^T P^T, 16 keys per step.  The V^T operand comes from the transposing LDS read
-        //      (ds_read_b64_tr_b16): in every 16-lane group, lane s points at 4 columns of key row
-        //      s/4 and receives column s (of the group's 16) for the group's 4 key rows.  Column tile
-        //      t is V columns t*32 .. t*32+31 in lane order.
-        typedef short v4s_t __attribute__((ext_vector_type(4)));
-        const uint32_t v_at = in_buffer(v_lane, kt & (Cfg::kVBufs - 1));
-        constexpr int kVG = Cfg::kMT < 4 ? Cfg::kMT : 4;         // column tiles whose operands are read together
-        constexpr int kVSteps = 4 * Cfg::kMT / kVG;
-        u32x4_t va[2][kVG];
-        auto read_v = [&](int step) {
-            const int ks = step / (Cfg::kMT / kVG), t0 = step % (Cfg::kMT / kVG) * kVG;
+        auto products = [&](auto halves_c) {
+            constexpr int H = decltype(halves_c)::value;
+            __builtin_amdgcn_s_setprio(1);
+            // ---- O^T += V^T P^T, 16 keys per step.  The V^T operand comes from the transposing LDS read
+            //      (ds_read_b64_tr_b16): in every 16-lane group, lane s points at 4 columns of key row
+            //      s/4 and receives column s (of the group's 16) for the group's 4 key rows.  Column tile
+            //      t is V columns t*32 .. t*32+31 in lane order.
+            typedef short v4s_t __attribute__((ext_vector_type(4)));
+            asm volatile("" : "+v"(v_at));
+            constexpr int kVG = Cfg::kMT < 4 ? Cfg::kMT : 4;         // column tiles whose operands are read together
+            constexpr int kVSteps = 2 * H * Cfg::kMT / kVG;
+            u32x4_t va[2][kVG];
+            auto read_v = [&](int step) {
+                const int ks = step / (Cfg::kMT / kVG), t0 = step % (Cfg::kMT / kVG) * kVG;
 #pragma unroll
-            for (int u = 0; u < kVG; ++u) {
-                if (PART && (t0 + u) * 32 >= hd) continue;
+                for (int u = 0; u < kVG; ++u) {
+                    if (PART && (t0 + u) * 32 >= hd) continue;
 #pragma unroll
-                for (int hv = 0; hv < 2; ++hv) {
-                    const v4s_t r4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (__attribute__((address_space(3))) v4s_t *)(uintptr_t)((v_at ^ (uint32_t)((t0 + u) << 6)) + (16 * ks + 8 * hv) * Cfg::kRowBytes));
-                    const uint2 r2 = __builtin_bit_cast(uint2, r4);
-                    va[step & 1][u][2 * hv] = r2.x;
-                    va[step & 1][u][2 * hv + 1] = r2.y;
+                    for (int hv = 0; hv < 2; ++hv) {
+                        const v4s_t r4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (__attribute__((address_space(3))) v4s_t *)(uintptr_t)((v_at ^ (uint32_t)((t0 + u) << 6)) + (16 * ks + 8 * hv) * Cfg::kRowBytes));
+                        const uint2 r2 = __builtin_bit_cast(uint2, r4);
+                        va[step & 1][u][2 * hv] = r2.x;
+                        va[step & 1][u][2 * hv + 1] = r2.y;
+                    }
                 }
-            }
         };
         read_v(0);
 #pragma unroll
@@ -542,7 +597,13 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
             __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_s_setprio(0);
-        }   // wave_live
+        };
+        if (live == 2) products(std::integral_constant<int, 2>{});
+        if (kHalves && live == 1) products(std::integral_constant<int, 1>{});
+        k_at ^= Cfg::kTileBytes;
+        if (Cfg::kVBufs == 2) v_at ^= Cfg::kTileBytes;
+        v_here[0] = next.v[0], v_here[1] = next.v[1];
+        advance(next);
         tiles_landed();
         barrier();
     }
@@ -553,7 +614,9 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     const float inv = (l_run > 0.f) ? 1.f / l_run : 0.f;
     if (!whole) {
         // one of several ranges of the unit: normalised fp32 partial and base-2 LSE for the combine
-        if (row_ok) {
+        const TileRow row = my_row(this_lane());
+        if (row.ok) {
+            float *part_row = p.o_partial + part_of(row) * D;
 #pragma unroll
             for (int t = 0; t < Cfg::kMT; ++t)
 #pragma unroll
@@ -561,11 +624,12 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
                     *reinterpret_cast<float4 *>(part_row + t * 32 + 8 * j + 4 * lh) =
                         make_float4(o_acc[t][4 * j] * inv, o_acc[t][4 * j + 1] * inv, o_acc[t][4 * j + 2] * inv,
                                     o_acc[t][4 * j + 3] * inv);
-            if (lh == 0) *part_lse = (l_run > 0.f) ? m_run + fast_log2(l_run) : -INFINITY;
+            if (lh == 0) p.lse_partial[part_of(row)] = (l_run > 0.f) ? m_run + fast_log2(l_run) : -INFINITY;
         }
         return;
     }
-    if (row_ok && lh == 0) *lse_row = (l_run > 0.f) ? (m_run + fast_log2(l_run)) * kLn2 : INFINITY;
+    const TileRow my = my_row(this_lane());
+    if (my.ok && lh == 0) *lse_of(my) = (l_run > 0.f) ? (m_run + fast_log2(l_run)) * kLn2 : INFINITY;
     // The lane owns 8-byte pieces of its row, 16 of them: stored as they are, one instruction would touch
     // 32 rows of the output.  The wave's 32 x D tile goes through LDS instead (the V tiles are free
     // after the last barrier of the loop; each wave uses its own part, so no workgroup barrier) and
@@ -588,24 +652,21 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     constexpr int kLanesPerRow = D * 2 / 16;                   // lanes that cover one row with 16 bytes each
     constexpr int kStageRows = 64 / kLanesPerRow;              // rows a wave stores per instruction
     const int piece = lane % kLanesPerRow;
-    const uint32_t pg_inv = (EXT && pg > 1) ? 0xffffffffu / (uint32_t)pg + 1u : 0u;   // x / pg = the upper half of x * pg_inv for x < pg + 128
 #pragma unroll
     for (int r0 = 0; r0 < 32; r0 += kStageRows) {
         const int rr = r0 + lane / kLanesPerRow;               // row of the wave's tile
-        const int R = R0 + wave * 32 + rr;
-        if (R < n_rows && (!PART || piece * 8 < hd)) {
-            const int row = (EXT && pg > 1) ? r_lo + (int)__umulhi((uint32_t)(R - r_lo * pg), pg_inv) : R;
-            const int head = h_base + (R - row * pg);
-            uint16_t *dst = reinterpret_cast<uint16_t *>(p.out) + (int64_t)b * p.o_stride_b + (int64_t)head * p.o_stride_h +
-                            (int64_t)(q0 + row) * p.o_stride_t;
+        const TileRow row = tile_row(wave * 32 + rr);
+        if (row.ok && (!PART || piece * 8 < hd)) {
+            uint16_t *dst = reinterpret_cast<uint16_t *>(p.out) + (int64_t)b * p.o_stride_b + (int64_t)row.head * p.o_stride_h +
+                            (int64_t)(q0 + row.pos) * p.o_stride_t;
             store16(dst + piece * 8, *reinterpret_cast<const u32x4_t *>(stage + rr * kStageRow + piece * 16));
         }
     }
 }
 
 template <typename T, int D, bool PAGED, bool SOFTCAP, bool EXT, bool PART>
-__global__ void __launch_bounds__(256, prefill_occupancy(D, PART)) prefill_kernel(const PrefillParams p) {
-    __shared__ PrefillTileLds<D> lds;
+__global__ void __launch_bounds__(256, prefill_wgs_resident(D, PART)) prefill_kernel(const PrefillParams p) {
+    __shared__ __attribute__((aligned(2 * PrefillCfg<D>::kTileBytes))) PrefillTileLds<D> lds;
     prefill_block<T, D, PAGED, SOFTCAP, EXT, PART>(p, blockIdx.x, -1, lds);
 }
 
@@ -617,8 +678,8 @@ __global__ void __launch_bounds__(256, prefill_occupancy(D, PART)) prefill_kerne
 // of a unit still meet in one L2, through one counter per XCD (p.list_state[1 + x], zeroed by the kernel that
 // wrote the list).  Every workgroup leaves when its counter passes the end of the list.
 template <typename T, int D, bool SOFTCAP, bool PART>
-__global__ void __launch_bounds__(256, prefill_occupancy(D, true)) prefill_list_kernel(const PrefillParams p) {
-    __shared__ PrefillTileLds<D> lds;
+__global__ void __launch_bounds__(256, prefill_wgs_resident(D, true)) prefill_list_kernel(const PrefillParams p) {
+    __shared__ __attribute__((aligned(2 * PrefillCfg<D>::kTileBytes))) PrefillTileLds<D> lds;
     __shared__ int s_item;
     const int n_long = p.list_state[0];
     const int heads_per_unit = (p.pack > 1) ? 1 : p.group;
