@@ -229,11 +229,21 @@ __device__ __forceinline__ void wave_piece(const DecodeParams &p, const int b, c
     };
     const uint32_t v_lane_off = (uint32_t)(lq * 4) * v_row_bytes + v_lane_col;
 
-    auto load_blk = [&](int c) -> int {   // the table entry as loaded (every lane the same address); not waited for
-        if (c >= c_end) return 0;
-        int page = (c * kChunk) / p.page_size;
-        page = min(page, p.max_blocks - 1);
-        return bt_row[page];
+    // Place of a chunk: its page in the table and its first row in the page, stepped along: a division per piece where the start of
+    // a piece and every chunk took two (1 sequence of 700 keys, 8 kv heads: 9.97 -> 9.52 us; calls of more chunks are level).
+    struct ChunkPlace {
+        int page, row;
+    };
+    auto next_place = [&](ChunkPlace t) -> ChunkPlace {
+        t.row += kChunk;
+        if (t.row >= p.page_size) {
+            t.row = 0;
+            ++t.page;
+        }
+        return t;
+    };
+    auto load_blk = [&](int c, const ChunkPlace &t) -> int {   // the table entry as loaded (every lane the same address); not waited for
+        return c >= c_end ? 0 : bt_row[min(t.page, p.max_blocks - 1)];
     };
     auto use_blk = [&](int raw) -> int { return min(max(__builtin_amdgcn_readfirstlane(raw), 0), p.num_blocks - 1); };
     auto load_v = [&](const uint8_t *s2, int e, int hh) {
@@ -252,9 +262,8 @@ __device__ __forceinline__ void wave_piece(const DecodeParams &p, const int b, c
             vreg[e][hh][0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(s2));
         }
     };
-    auto issue_loads = [&](int c, int blk, int kbuf) {
+    auto issue_loads = [&](int c, int blk, int inpage0, int kbuf) {
         const int key0 = c * kChunk;
-        const int inpage0 = key0 % p.page_size;
         const int last = Lk - 1 - key0;  // last written key relative to the chunk (>= 0)
         const uint8_t *kb = kc_base + (int64_t)blk * p.k_stride_block * 2 + (int64_t)inpage0 * k_row_bytes;
         const uint8_t *vb = vc_base + (int64_t)blk * p.v_stride_block * 2 + (int64_t)inpage0 * v_row_bytes;
@@ -301,13 +310,18 @@ __device__ __forceinline__ void wave_piece(const DecodeParams &p, const int b, c
     // first chunk in flight while Q is staged
     int c = c_begin;
     int blk_next;
+    ChunkPlace place;                 // of the chunk whose loads come next
+    place.page = c_begin * kChunk / p.page_size;
+    place.row = c_begin * kChunk - place.page * p.page_size;
     {
         // Both table entries are asked for before the first chunk's loads.  Loads return in order: asked for behind
         // them, the second entry would only be there when the whole chunk is, and the q rows would be requested a
         // memory latency later than they need be.
-        const int blk0 = load_blk(c);
-        blk_next = load_blk(c + 1);
-        if (c < c_end) issue_loads(c, use_blk(blk0), 0);
+        const int blk0 = load_blk(c, place);
+        const int first_row = place.row;
+        place = next_place(place);
+        blk_next = load_blk(c + 1, place);
+        if (c < c_end) issue_loads(c, use_blk(blk0), first_row, 0);
     }
     // the q rows are staged in the wave's second tile: the first chunk that lands there leaves after they have been read
     uint16_t *sq = reinterpret_cast<uint16_t *>(ktile + Cfg::kTileBytes);
@@ -385,10 +399,11 @@ __device__ __forceinline__ void wave_piece(const DecodeParams &p, const int b, c
         __builtin_amdgcn_wave_barrier();
 
         const int cn = c + 1;
-        if (cn < c_end) issue_loads(cn, use_blk(blk_next), kbuf ^ 1);
+        if (cn < c_end) issue_loads(cn, use_blk(blk_next), place.row, kbuf ^ 1);
+        place = next_place(place);
         // asked for behind the chunk's loads, the next table entry is there when they all are: the wave rests here
         // until chunk cn has landed and only then works on chunk c
-        blk_next = __builtin_amdgcn_readfirstlane(load_blk(cn + 1));
+        blk_next = __builtin_amdgcn_readfirstlane(load_blk(cn + 1, place));
         __builtin_amdgcn_sched_barrier(0);
 
         // S^T = K Q^T, two 16-key tiles (for every row tile)
