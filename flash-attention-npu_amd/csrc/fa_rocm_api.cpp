@@ -408,11 +408,12 @@ int fa_rocm_plan_kvcache(const fa_kvcache_args *a, int num_cus, fa_split_plan *p
             n = a->num_splits;
         } else if (a->num_splits == 0) {
             const int64_t tiles = (int64_t)a->batch * fa::prefill_tiles(a->nheads, a->nheads_k, a->seqlen_q);
-            auto ranges = [&](int per_cu) -> int64_t {
-                const int64_t slots = (int64_t)num_cus * per_cu;
-                return tiles * 2 <= slots ? (slots + tiles - 1) / tiles : 1;
-            };
-            n = ranges(fa::prefill_wgs_per_cu(a->headdim_qk));
+            // cut when two workgroups per compute unit would find less than half as many tiles, into as many ranges as fill all
+            // that are resident (with fewer tiles missing, the merge costs more than the ranges give: 3 x 679 tokens over 345
+            // keys, d = 64, 456 tiles: 13 us whole, 36 in three ranges)
+            const int64_t few = (int64_t)num_cus * (a->headdim_qk <= 128 ? 2 : 1);
+            auto ranges = [&](int per_cu) -> int64_t { return tiles * 2 <= few ? ((int64_t)num_cus * per_cu + tiles - 1) / tiles : 1; };
+            n = ranges(std::min(fa::prefill_wgs_per_cu(a->headdim_qk), 3));   // (for the fourth at d = 64 too: 573 tokens over 2498 keys 29.1 -> 31.3 us)
             // (no more than the static scratch holds where the ranges of two workgroups per compute unit fit it: callers that
             // cannot allocate count on it)
             const int64_t per_range = (int64_t)a->batch * a->nheads_k * (int64_t)slot_bytes;
@@ -1069,10 +1070,10 @@ int fa_rocm_varlen_num_splits(const fa_varlen_args *a, int num_cus) {
         // workgroups per compute unit of the kernel that takes such a batch from a list (20 decode rows + 2000 tokens that
         // end 30000 keys: 1117 us with two ranges, 1180 with three)
         const bool uneven = uneven_blocks(a);
-        const int64_t slots = (int64_t)num_cus * (!uneven ? fa::prefill_wgs_per_cu(a->headdim) : a->headdim <= 128 ? 2 : 1);
+        const int64_t few = (int64_t)num_cus * (a->headdim <= 128 ? 2 : 1), slots = (int64_t)num_cus * std::min(fa::prefill_wgs_per_cu(a->headdim), 3);
         if (uneven) {
-            if (tiles < 2 * slots) n = (2 * slots + tiles - 1) / tiles;
-        } else if (tiles * 2 <= slots) {
+            if (tiles < 2 * few) n = (2 * few + tiles - 1) / tiles;
+        } else if (tiles * 2 <= few) {
             n = (slots + tiles - 1) / tiles;
         }
     }
