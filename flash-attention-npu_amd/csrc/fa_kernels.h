@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace fa {
 
 // Parameters of the paged decode kernel and of the split-KV combine kernel.  Passed by value
@@ -214,6 +216,23 @@ constexpr int prefill_wgs_resident(int d, bool spare) { return d == 64 ? 4 - spa
 // ... by head dimension
 constexpr int prefill_wgs_per_cu(int headdim) {
     return headdim <= 64 ? prefill_wgs_resident(64, headdim < 64) : headdim <= 128 ? prefill_wgs_resident(128, headdim < 128) : 1;
+}
+// Key ranges for `tiles` tiles of equal height that leave the device half empty (1: they do not), at most `most` of them; `room`: how
+// many the scratch holds that callers who cannot allocate count on.  The count fills two workgroups per compute unit; with fewer
+// tiles missing the merge costs more than the ranges give (3 x 679 tokens over 345 keys, d = 64, 456 tiles: 13 us whole, 36 in
+// three ranges).  That a third one is resident helps only where two cannot be dealt out evenly: a launch lasts as long as the
+// compute unit with the most workgroups, each 1 / n of the keys.  Two / three per compute unit, us, 32 q heads per kv head, 1 token:
+// 64 units x 8192 keys (8 / 12 ranges) 56.8 / 63.4, 128 x 4096 58.3 / 63.8, 32 x 16384 57.1 / 63.2, 100 x 2048 (6 / 8) 31.5 / 38.5; where
+// the fullest compute unit has less to do, 48 units x 16384 (11 / 16) 101.2 / 84.0; tall blocks, level there, gain a little (2 x
+// 512 tokens, 32q/8kv, over 65536 keys 1223 / 1155) and lose as much elsewhere (4 x 64 tokens over 8192 65.8 / 70.8).  (Never the fourth
+// of d = 64: 573 tokens over 2498 keys 29.1 / 31.3.)
+inline int64_t prefill_key_ranges(int64_t tiles, int64_t most, int64_t room, int num_cus, int headdim) {
+    const int two = headdim <= 128 ? 2 : 1;
+    if (tiles * 2 > (int64_t)num_cus * two) return 1;
+    auto filling = [&](int per_cu) -> int64_t { return std::min(((int64_t)num_cus * per_cu + tiles - 1) / tiles, most); };
+    auto fullest = [&](int64_t n) -> int64_t { return (tiles * n + num_cus - 1) / num_cus; };
+    const int64_t n = filling(two), more = std::min(filling(std::min(prefill_wgs_per_cu(headdim), 3)), room);
+    return more > n && fullest(more) * n < fullest(n) * more ? more : n;
 }
 // Causal launches that prefill_pack() leaves unpacked: whether the heads of a group share the tiles all the same.  The 128
 // rows of a tile are then 128 / group queries of all the heads rather than 128 queries of one, so that a tile's keys end

@@ -402,27 +402,18 @@ int fa_rocm_plan_kvcache(const fa_kvcache_args *a, int num_cus, fa_split_plan *p
         // the number of ranges is planned here.  With rotary embedding the workspace starts with the
         // rotated copy of q.
         plan->mode = FA_SPLIT_GRID;
-        const int64_t bound = live_keys_bound(a);
+        const int64_t most = std::min<int64_t>((live_keys_bound(a) + 255) / 256, 64);   // at least 256 keys (four tiles) per range
         int64_t n = 1;
         if (a->num_splits > 1) {
             n = a->num_splits;
         } else if (a->num_splits == 0) {
             const int64_t tiles = (int64_t)a->batch * fa::prefill_tiles(a->nheads, a->nheads_k, a->seqlen_q);
-            // cut when two workgroups per compute unit would find less than half as many tiles, into as many ranges as fill all
-            // that are resident (with fewer tiles missing, the merge costs more than the ranges give: 3 x 679 tokens over 345
-            // keys, d = 64, 456 tiles: 13 us whole, 36 in three ranges)
-            const int64_t few = (int64_t)num_cus * (a->headdim_qk <= 128 ? 2 : 1);
-            auto ranges = [&](int per_cu) -> int64_t { return tiles * 2 <= few ? ((int64_t)num_cus * per_cu + tiles - 1) / tiles : 1; };
-            n = ranges(std::min(fa::prefill_wgs_per_cu(a->headdim_qk), 3));   // (for the fourth at d = 64 too: 573 tokens over 2498 keys 29.1 -> 31.3 us)
-            // (no more than the static scratch holds where the ranges of two workgroups per compute unit fit it: callers that
-            // cannot allocate count on it)
+            // the scratch of fa_rocm_fwd_kvcache_static bounds what the third workgroup per compute unit may add
             const int64_t per_range = (int64_t)a->batch * a->nheads_k * (int64_t)slot_bytes;
             const int64_t room = ((int64_t)FA_ROCM_STATIC_SCRATCH_BYTES - (int64_t)tall_q_bytes(a)) / std::max<int64_t>(per_range, 1);
-            if (n > room) n = std::max(std::min(n, ranges(a->headdim_qk <= 128 ? 2 : 1)), std::max<int64_t>(room, 1));
+            n = fa::prefill_key_ranges(tiles, most, room, num_cus, a->headdim_qk);
         }
-        const int64_t most = (bound + 255) / 256;   // at least 256 keys (four tiles) per range
         if (n > most) n = most;
-        if (n > 64) n = 64;
         if (n < 1) n = 1;
         plan->nsplits = (int32_t)n;
         plan->split_keys = 0;

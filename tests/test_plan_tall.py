@@ -46,6 +46,31 @@ def test_tall_plan():
     assert p.nsplits == 32 and p.workspace_bytes == q_bytes + 1 * 2 * 32 * (24 * 8) * 129 * 4
 
 
+def test_tall_plan_range_counts():
+    # what two workgroups per compute unit take, unless they leave some compute unit with three anyway
+    for batch, n in ((16, 32), (32, 16), (64, 8), (128, 4), (250, 3), (256, 2), (257, 1)):
+        assert plan_of(batch, 2, 32, 1, 128, 128).nsplits == n, batch
+    assert plan_of(48, 1, 32, 1, 128, 128).nsplits == 16         # 11 would leave 16 compute units with three of 11
+    assert plan_of(48, 1, 32, 1, 128, 10).nsplits == 10          # ... but no range under 256 keys
+    assert plan_of(48, 1, 32, 1, 96, 128).nsplits == 11          # below the compiled width two workgroups are resident
+    assert plan_of(40, 2, 32, 1, 64, 128).nsplits == 20          # D = 64: three of the four that are resident
+    assert plan_of(48, 1, 32, 1, 256, 128).nsplits == 6 and plan_of(129, 1, 32, 1, 256, 128).nsplits == 1
+
+
+def test_tall_plan_static_scratch():
+    # more ranges than two workgroups per compute unit ask for never outgrow the scratch of the call that allocates nothing
+    static = 36 << 20
+    p = plan_of(48, 2, 32, 1, 128, 128)                          # 16 ranges fit ...
+    assert p.nsplits == 16 and p.workspace_bytes == 48 * 16 * 64 * 129 * 4 <= static
+    p = plan_of(3, 100, 32, 8, 128, 20)                          # ... of 8 only 7 do, which still beat the 6 of two per compute unit
+    assert p.nsplits == 7 and p.workspace_bytes <= static < 3 * 8 * 8 * 400 * 129 * 4
+    p = plan_of(4, 32, 32, 1, 128, 256)                          # no count in between that evens out nothing (17 of 24 would fit)
+    assert p.nsplits == 16 and p.workspace_bytes <= static
+    assert plan_of(4, 128, 32, 8, 128, 128).nsplits == 4
+    assert plan_of(17, 60, 32, 1, 128, 128).nsplits == 3         # 255 tiles: three ranges of two per compute unit, beyond the scratch as they always were
+    assert plan_of(17, 60, 32, 1, 128, 128).workspace_bytes > static
+
+
 def test_varlen_split_plan():
     # the planner: paged only, never with num_splits = 1, at least 256 keys per range, at most 64 ranges
     import ctypes as C
