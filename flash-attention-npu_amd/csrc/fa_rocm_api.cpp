@@ -1052,6 +1052,9 @@ int fa_rocm_varlen_num_splits(const fa_varlen_args *a, int num_cus) {
     // the lengths of the query blocks stay on the device: sum_b ceil(rows_b / 128) <= rows / 128 + batch
     const int64_t blocks = ((int64_t)a->total_q * pack + 127) / 128 + a->batch;
     const int64_t tiles = blocks * (pack > 1 ? a->nheads_k : a->nheads);
+    const int64_t bound = std::min<int64_t>(a->max_seqlen_k > 0 ? a->max_seqlen_k : INT32_MAX,
+                                            (int64_t)a->max_blocks_per_seq * a->page_size);
+    const int64_t most = std::min<int64_t>((bound + 255) / 256, 64);   // at least 256 keys (four tiles) per range
     int64_t n = 1;
     if (a->num_splits > 1) {
         n = a->num_splits;
@@ -1065,13 +1068,17 @@ int fa_rocm_varlen_num_splits(const fa_varlen_args *a, int num_cus) {
         if (uneven) {
             if (tiles < 2 * few) n = (2 * few + tiles - 1) / tiles;
         } else if (tiles * 2 <= few) {
-            n = (slots + tiles - 1) / tiles;
+            // `tiles` is a bound, mostly a quarter too high, so that three per compute unit seldom crowd it: 307 tokens over 7400
+            // keys, 32q/1kv, two / three 113 / 84 us; of 99 calls' time on a kernel with two resident, 0.909 / 0.883 on the mean
+            n = std::max<int64_t>(std::min((slots + tiles - 1) / tiles, most), 1);
+            // The device rounds the keys of a range up to 256, which leaves the last ranges of a high count empty.  Their
+            // workgroups find that out one by one and crowd the others meanwhile: 3 x 127..198 tokens over 2007 keys, 32q/1kv,
+            // 79.2 us in seven ranges of which four are filled, 65.3 in four.
+            const int64_t keys = ((bound + n - 1) / n + 255) / 256 * 256;
+            n = (bound + keys - 1) / keys;
         }
     }
-    const int64_t bound = std::min<int64_t>(a->max_seqlen_k > 0 ? a->max_seqlen_k : INT32_MAX,
-                                            (int64_t)a->max_blocks_per_seq * a->page_size);
-    const int64_t most = (bound + 255) / 256;   // at least 256 keys (four tiles) per range
-    n = std::min<int64_t>(std::min<int64_t>(n, most), 64);
+    n = std::min<int64_t>(n, most);
     return (int)std::max<int64_t>(n, 1);
 }
 

@@ -106,6 +106,26 @@ def test_varlen_split_plan():
     assert lib.fa_rocm_varlen_fwd(C.byref(a), None) == -5 and b"workspace" in lib.fa_rocm_last_error()
 
 
+def test_varlen_plans_no_range_that_stays_empty():
+    # the device rounds the keys of a range up to 256: a count is planned for which every range of the longest sequence has some
+    lib = _lib.load()
+    a = _lib.VarlenArgs()
+    fake = 0x1000
+    for f in ("q", "k", "v", "out", "softmax_lse", "cu_seqlens_q", "seqused_k", "block_table"):
+        setattr(a, f, fake)
+    a.nheads, a.nheads_k, a.headdim, a.page_size, a.max_blocks_per_seq, a.num_blocks = 32, 1, 128, 256, 128, 4000
+    a.q_stride_t = a.o_stride_t = 32 * 128
+    a.q_stride_h = a.o_stride_h = a.k_stride_h = a.v_stride_h = a.k_stride_t = a.v_stride_t = 128
+    for batch, total, longest, keys, n in ((3, 510, 198, 2007, 4), (24, 370, 19, 2020, 4), (2, 47, 24, 32735, 43), (8, 210, 31, 7954, 11), (8, 240, 36, 32581, 12),
+                                           (1, 307, 307, 7400, 6), (1, 20, 20, 255, 1)):
+        a.batch, a.total_q, a.max_seqlen_q, a.max_seqlen_k = batch, total, longest, keys
+        assert lib.fa_rocm_varlen_num_splits(C.byref(a), 256) == n, (batch, keys)
+        per = -(-(-(-keys // n)) // 256) * 256
+        assert -(-keys // per) == n
+    a.batch, a.total_q, a.max_seqlen_q, a.max_seqlen_k, a.num_splits = 3, 510, 198, 2007, 7        # the caller's count stays
+    assert lib.fa_rocm_varlen_num_splits(C.byref(a), 256) == 7
+
+
 def test_varlen_short_blocks_workspace():
     # a prompt chunk among decode rows: the one-token blocks are computed by the decode kernels, whose batch-major
     # rows and own workspace follow the partials in the caller's workspace
