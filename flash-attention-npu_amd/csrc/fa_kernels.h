@@ -217,22 +217,29 @@ constexpr int prefill_wgs_resident(int d, bool spare) { return d == 64 ? 4 - spa
 constexpr int prefill_wgs_per_cu(int headdim) {
     return headdim <= 64 ? prefill_wgs_resident(64, headdim < 64) : headdim <= 128 ? prefill_wgs_resident(128, headdim < 128) : 1;
 }
-// Key ranges for `tiles` tiles of equal height that leave the device half empty (1: they do not), at most `most` of them; `room`: how
-// many the scratch holds that callers who cannot allocate count on.  The count fills two workgroups per compute unit; with fewer
-// tiles missing the merge costs more than the ranges give (3 x 679 tokens over 345 keys, d = 64, 456 tiles: 13 us whole, 36 in
-// three ranges).  That a third one is resident helps only where two cannot be dealt out evenly: a launch lasts as long as the
-// compute unit with the most workgroups, each 1 / n of the keys.  Two / three per compute unit, us, 32 q heads per kv head, 1 token:
+// Key ranges for `tiles` tiles of equal height that leave the device half empty (1: they do not), over sequences of up to `keys` keys; at
+// most 64 and none under 256 keys; `room`: how many the scratch holds that callers who cannot allocate count on.  The count fills
+// two workgroups per compute unit; with fewer tiles missing the merge costs more than the ranges give (3 x 679 tokens over 345 keys,
+// d = 64, 456 tiles: 13 us whole, 36 in three ranges).  That a third one is resident helps only where two cannot be dealt out evenly: a
+// launch lasts as long as the compute unit with the most workgroups walks its keys.  The device rounds the keys of a range up to
+// 256, so more ranges may be no shorter, or some of them empty.  Two / three per compute unit, us, 32 q heads per kv head, 1 token:
 // 64 units x 8192 keys (8 / 12 ranges) 56.8 / 63.4, 128 x 4096 58.3 / 63.8, 32 x 16384 57.1 / 63.2, 100 x 2048 (6 / 8) 31.5 / 38.5; where
-// the fullest compute unit has less to do, 48 units x 16384 (11 / 16) 101.2 / 84.0; tall blocks, level there, gain a little (2 x
-// 512 tokens, 32q/8kv, over 65536 keys 1223 / 1155) and lose as much elsewhere (4 x 64 tokens over 8192 65.8 / 70.8).  (Never the fourth
-// of d = 64: 573 tokens over 2498 keys 29.1 / 31.3.)
-inline int64_t prefill_key_ranges(int64_t tiles, int64_t most, int64_t room, int num_cus, int headdim) {
+// the fullest compute unit has less to walk, 48 units x 16384 (11 / 16) 101.2 / 84.0; with the rounding left out of the account 6 x 31 tokens
+// over 14835 keys, 32q/8kv (11 / 12) 92.0 / 108.2, 24 x 14 tokens over 2058, 28q/4kv (6 / 7) 39.8 / 47.1, in it both stay at two.
+// What it cannot see are the lengths, nor how the device deals the workgroups out: 320 calls for which a third one would shorten the walk
+// of equal sequences if ranges were not rounded, tables up to eight times as wide as needed among them, took 0.964 of the time with
+// two on the mean (best 0.75; 27 of them more than 4 % longer, worst 1.23: 6 x 16 tokens over 534..5342 keys, 32q/8kv, under a wide table);
+// without the rounding 0.970.  (Never the fourth of d = 64: 60 calls with three 0.989 of two, with four 0.990.)
+inline int64_t prefill_key_ranges(int64_t tiles, int64_t keys, int64_t room, int num_cus, int headdim) {
     const int two = headdim <= 128 ? 2 : 1;
     if (tiles * 2 > (int64_t)num_cus * two) return 1;
+    const int64_t most = std::min<int64_t>((keys + 255) / 256, 64);
     auto filling = [&](int per_cu) -> int64_t { return std::min(((int64_t)num_cus * per_cu + tiles - 1) / tiles, most); };
-    auto fullest = [&](int64_t n) -> int64_t { return (tiles * n + num_cus - 1) / num_cus; };
-    const int64_t n = filling(two), more = std::min(filling(std::min(prefill_wgs_per_cu(headdim), 3)), room);
-    return more > n && fullest(more) * n < fullest(n) * more ? more : n;
+    auto length = [&](int64_t n) -> int64_t { return ((keys + n - 1) / n + 255) / 256 * 256; };
+    auto filled = [&](int64_t n) -> int64_t { return (keys + length(n) - 1) / length(n); };   // the ranges of n that have keys
+    auto walk = [&](int64_t n) -> int64_t { return (tiles * filled(n) + num_cus - 1) / num_cus * length(n); };
+    const int64_t n = filling(two), third = std::min(filling(std::min(prefill_wgs_per_cu(headdim), 3)), room);
+    return third > n && filled(third) > n && walk(third) * 16 <= walk(n) * 15 ? filled(third) : n;   // (a sixteenth for the longer merge)
 }
 // Causal launches that prefill_pack() leaves unpacked: whether the heads of a group share the tiles all the same.  The 128
 // rows of a tile are then 128 / group queries of all the heads rather than 128 queries of one, so that a tile's keys end

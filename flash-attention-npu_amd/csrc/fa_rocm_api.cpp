@@ -402,7 +402,8 @@ int fa_rocm_plan_kvcache(const fa_kvcache_args *a, int num_cus, fa_split_plan *p
         // the number of ranges is planned here.  With rotary embedding the workspace starts with the
         // rotated copy of q.
         plan->mode = FA_SPLIT_GRID;
-        const int64_t most = std::min<int64_t>((live_keys_bound(a) + 255) / 256, 64);   // at least 256 keys (four tiles) per range
+        const int64_t bound = live_keys_bound(a);
+        const int64_t most = std::min<int64_t>((bound + 255) / 256, 64);   // at least 256 keys (four tiles) per range
         int64_t n = 1;
         if (a->num_splits > 1) {
             n = a->num_splits;
@@ -411,7 +412,7 @@ int fa_rocm_plan_kvcache(const fa_kvcache_args *a, int num_cus, fa_split_plan *p
             // the scratch of fa_rocm_fwd_kvcache_static bounds what the third workgroup per compute unit may add
             const int64_t per_range = (int64_t)a->batch * a->nheads_k * (int64_t)slot_bytes;
             const int64_t room = ((int64_t)FA_ROCM_STATIC_SCRATCH_BYTES - (int64_t)tall_q_bytes(a)) / std::max<int64_t>(per_range, 1);
-            n = fa::prefill_key_ranges(tiles, most, room, num_cus, a->headdim_qk);
+            n = fa::prefill_key_ranges(tiles, bound, room, num_cus, a->headdim_qk);
         }
         if (n > most) n = most;
         if (n < 1) n = 1;

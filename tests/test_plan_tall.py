@@ -53,8 +53,12 @@ def test_tall_plan_range_counts():
     assert plan_of(48, 1, 32, 1, 128, 128).nsplits == 16         # 11 would leave 16 compute units with three of 11
     assert plan_of(48, 1, 32, 1, 128, 10).nsplits == 10          # ... but no range under 256 keys
     assert plan_of(48, 1, 32, 1, 96, 128).nsplits == 11          # below the compiled width two workgroups are resident
-    assert plan_of(40, 2, 32, 1, 64, 128).nsplits == 20          # D = 64: three of the four that are resident
+    assert plan_of(40, 2, 32, 1, 64, 128).nsplits == 19          # D = 64: three of the four that are resident; of 20 one would have no keys
     assert plan_of(48, 1, 32, 1, 256, 128).nsplits == 6 and plan_of(129, 1, 32, 1, 256, 128).nsplits == 1
+    # the device rounds the keys of a range up to 256: 12 ranges of 1280 keys on three workgroups are a longer walk than 10 of 1536 on
+    # two, and 7 of 512 are the 5 that 6 are
+    assert plan_of(6, 31, 32, 8, 128, 58).nsplits == 11
+    assert plan_of(24, 14, 28, 4, 128, 9).nsplits == 6
 
 
 def test_tall_plan_static_scratch():
@@ -62,8 +66,8 @@ def test_tall_plan_static_scratch():
     static = 36 << 20
     p = plan_of(48, 2, 32, 1, 128, 128)                          # 16 ranges fit ...
     assert p.nsplits == 16 and p.workspace_bytes == 48 * 16 * 64 * 129 * 4 <= static
-    p = plan_of(3, 100, 32, 8, 128, 20)                          # ... of 8 only 7 do, which still beat the 6 of two per compute unit
-    assert p.nsplits == 7 and p.workspace_bytes <= static < 3 * 8 * 8 * 400 * 129 * 4
+    p = plan_of(1, 134, 32, 8, 128, 100)                         # ... of 20 only 17 do, which still beat the 13 of two per compute unit
+    assert p.nsplits == 17 and p.workspace_bytes <= static < 1 * 8 * 18 * 536 * 129 * 4
     p = plan_of(4, 32, 32, 1, 128, 256)                          # no count in between that evens out nothing (17 of 24 would fit)
     assert p.nsplits == 16 and p.workspace_bytes <= static
     assert plan_of(4, 128, 32, 8, 128, 128).nsplits == 4
