@@ -211,7 +211,9 @@ inline int prefill_pack(int group, int max_seqlen_q) {
 // 895 / 987; us: 16 x 512..4096 causal 791.6 / 718.8, 80 x 3..350, 28q/4kv 85.9 / 78.3, 8 x 2050, 16q/16kv, d = 64, fp16 205.8 /
 // 198.8.  Random values hold the clock down (1.6-1.9 GHz; all-zero inputs run the same code 1.6 times as fast), so that half of the
 // saved cycles do not show.  `spare`: kernels that keep more beside the tile loop, a head dimension below D or a list of blocks.
-// (A list kernel of three waves spilled: 63 decode rows + a 1024-token chunk 592 us against 525.)
+// (A list kernel of three waves spills nine vector registers and 40 bytes of scratch per lane, one of four at d = 64 four and 20: 63
+// decode rows + a 1024-token chunk, 32q/8kv 531 us with two waves, 596 with three; 20 rows + 2000 tokens 1137 / 1421; d = 64, three /
+// four waves 373.7 / 375.5.)
 constexpr int prefill_wgs_resident(int d, bool spare) { return d == 64 ? 4 - spare : d == 128 ? 3 - spare : 1; }
 // ... by head dimension
 constexpr int prefill_wgs_per_cu(int headdim) {
@@ -244,13 +246,13 @@ inline int64_t prefill_key_ranges(int64_t tiles, int64_t keys, int64_t room, int
 // Causal launches that prefill_pack() leaves unpacked: whether the heads of a group share the tiles all the same.  The 128
 // rows of a tile are then 128 / group queries of all the heads rather than 128 queries of one, so that a tile's keys end
 // closer behind its queries (half a tile of hidden keys per row less at a group of 4) and short sequences fill their
-// tiles.  Unpacked / packed, in us: 80 x 3..350 tokens, 28q/4kv 91.1 / 74.3; 40 x 50..900, 28q/4kv 163.2 / 153.2; 16 x
-// 512..4096, 32q/8kv 796 / 761 (d = 64: 446.7 / 424.4); 64 x 512, 64q/32kv 583 / 570; 24 x 100..500, 16q/2kv, d = 256
-// 119.6 / 107.1.  Bidirectional launches gain nothing (30 x 100..900, 32q/8kv 218.3 / 219.8).  Nor do launches of less than
-// two rounds of the device, which last as long as their tallest tile either way (D = 128: 2 x 649 tokens, 32q/8kv 21.9 /
-// 23.0, 6 x 300..700, 16q/8kv 22.8 / 23.6); from there on the worst measured are 1-3 % behind (4 x 2048, 24q/8kv 119.7 /
-// 121.1; 12 x 100..500, 64q/32kv 60.6 / 62.3), and at D = 256 none is (20 x 200, 16q/2kv 57.3 / 44.5; 12 x 100..500, 16q/8kv
-// 53.2 / 51.2).
+// tiles.  Unpacked / packed, us, over 8 equal (=) or 16 ragged (~, lengths spread 1 : 20) sequences of T x 128 (query, head) rows
+// together: 28q/4kv T = 2048 = 113.8 / 104.2, ~ 88.3 / 81.1; 32q/8kv T = 2048 = 99.9 / 99.6, ~ 78.9 / 76.0, T = 4096 ~ 233.5 / 227.2;
+// 16q/2kv T = 1536 ~ 92.6 / 87.1; d = 64, 28q/4kv T = 2048 = 66.6 / 61.7; d = 256, 28q/4kv T = 1024 = 115.1 / 97.9.  Bidirectional
+// launches gain nothing (30 x 100..900, 32q/8kv 218.3 / 219.8).  Packed from T = 4 num_cus on (2 num_cus at D = 256): of 60 launches
+// from there to 4 times as many rows the worst are 2 % behind at D <= 128 (d = 64, 32q/8kv T = 1536 = 36.6 / 37.3), of 24 at D = 256 4 %
+// (32q/8kv T = 768 = 64.2 / 67.0).  Below it ragged batches mostly gain as well (T = 512 ~ 20.5 / 17.2; d = 64 T = 768 ~ 17.5 / 15.1), but
+// such a launch lasts as long as its tallest tile, and equal ones can lose (16q/2kv T = 512 = 21.1 / 21.7; d = 256 T = 256 = 21.7 / 22.5).
 inline bool prefill_pack_causal(int group, int nheads, int max_seqlen_q, int total_q, int headdim, int num_cus) {
     return group > 1 && group <= kPrefillTileRows && (int64_t)max_seqlen_q * group < (1ll << 30) &&
            (int64_t)total_q * nheads >= 2ll * num_cus * (headdim <= 128 ? 2 : 1) * kPrefillTileRows;

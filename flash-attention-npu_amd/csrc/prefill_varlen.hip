@@ -282,11 +282,11 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
     };
     auto tiles_landed = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
     // Where the tiles of a paged cache are.  A page holds a multiple of 32 keys (or, a page per sequence, all of them), so each half of
-    // a tile lies in one page, and the cursor keeps the addresses of both halves.  Inside a page a step moves them on by 64 rows; where a page ends they are made from the table, whose next two entries were asked for when the page before began: by
-    // scalar loads, which nobody has to wait for behind the tiles on their way.  (All of it is scalar work of every wave: the
-    // addresses made anew for every tile cost a paged launch 8 %, 4 x 2048 tokens over 8 K keys 1136 us against 1048 dense, now 1015
-    // against 985; a page
-    // looked up per row, with 32-row pages, 8 x 51 tokens over 4481..8962 keys, d = 64, 106 us against 79 now.)
+    // a tile lies in one page, and the cursor keeps the addresses of both halves.  Inside a page a step moves them on by 64 rows;
+    // where a page ends they are made from the table, whose next two entries were asked for when the page before began: by scalar
+    // loads, which nobody has to wait for behind the tiles on their way.  All of it is scalar work of every wave: the addresses made
+    // anew for every tile cost a paged launch 8 % (4 x 2048 tokens over 8 K keys 1136 us against 1048 dense, now 1015 against 985);
+    // a page looked up per row, with 32-row pages, a third (8 x 51 tokens over 4481..8962 keys, d = 64, 106 us against 79 now).
     const int page_rows = !PAGED || p.max_blocks == 1 ? INT32_MAX : p.page_size;
     auto table = [&](int page) -> int { return constant(bt_row, min(page, p.max_blocks - 1)); };
     struct Cursor {
@@ -519,8 +519,9 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
             mloc *= scale;
             mloc = halves_max(mloc);
             // The accumulator rescale is skipped for the whole wave when no row of it saw a new maximum
-            // (most tiles once a row is a few hundred keys in).  m_run stays the exact running maximum,
-            // so the largest P of a row is exactly 1 as in the reference's golden.
+            // (most tiles once a row is a few hundred keys in).  m_run is the running maximum times the scale, rounded, and
+            // the exponent the fused s * scale - m_run: the largest P of a row is 1 but for that rounding (2^d, |d| at most
+            // half a unit in the last place of m_run), in the weights, their sum and the LSE alike.
             const bool bump = mloc > m_run;   // false for fully hidden tiles
             if (__any(bump)) {
                 const float m_new = bump ? mloc : m_run;
@@ -583,20 +584,20 @@ __device__ __forceinline__ void prefill_block(const PrefillParams &p, const unsi
                         va[step & 1][u][2 * hv + 1] = r2.y;
                     }
                 }
-        };
-        read_v(0);
+            };
+            read_v(0);
 #pragma unroll
-        for (int step = 0; step < kVSteps; ++step) {
-            const int ks = step / (Cfg::kMT / kVG), t0 = step % (Cfg::kMT / kVG) * kVG;
-            if (step + 1 < kVSteps) read_v(step + 1);
+            for (int step = 0; step < kVSteps; ++step) {
+                const int ks = step / (Cfg::kMT / kVG), t0 = step % (Cfg::kMT / kVG) * kVG;
+                if (step + 1 < kVSteps) read_v(step + 1);
 #pragma unroll
-            for (int u = 0; u < kVG; ++u) {
-                if (PART && (t0 + u) * 32 >= hd) continue;
-                o_acc[t0 + u] = mfma32<T>(va[step & 1][u], pk[ks >> 1][ks & 1], o_acc[t0 + u]);
+                for (int u = 0; u < kVG; ++u) {
+                    if (PART && (t0 + u) * 32 >= hd) continue;
+                    o_acc[t0 + u] = mfma32<T>(va[step & 1][u], pk[ks >> 1][ks & 1], o_acc[t0 + u]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        __builtin_amdgcn_s_setprio(0);
+            __builtin_amdgcn_s_setprio(0);
         };
         if (live == 2) products(std::integral_constant<int, 2>{});
         if (kHalves && live == 1) products(std::integral_constant<int, 1>{});

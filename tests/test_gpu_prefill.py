@@ -384,9 +384,8 @@ def test_varlen_paged_small_mixed_batch():
 @pytest.mark.parametrize("page", [32, 96, 160])
 @pytest.mark.parametrize("d,dtype", [(128, torch.bfloat16), (64, torch.float16), (256, torch.bfloat16)])
 def test_tall_query_block_over_pages_that_a_tile_straddles(page, d, dtype):
-    """Pages that are no multiple of the 64-key tile: a tile then lies in two or three pages and every row of it takes
-    its own page-table entry (the path of the ragged end of a sequence); pages of 64 keys and more give a whole tile
-    one base address.  Lengths that end inside a tile, on a tile and on a page."""
+    """Pages that are no multiple of the 64-key tile: a tile then lies in two pages, and the cursor gives each of
+    its 32-key halves a base address from that half's own page.  Lengths that end inside a tile, on a tile and on a page."""
     from flash_attn_npu import flash_attn_with_kvcache
     lens = [5 * page + 7, 64, page, 1000]
     case = make_paged_case(len(lens), 8, 2, d, page, lens, seqlen_q=40, seqlen_new=0, dtype=dtype, seed=60 + page)
