@@ -104,7 +104,7 @@ class HipEvents:
 
 # ----------------------------------------------------------------------------- workloads
 def decode_workload(name: str, device, seed: int = 0, kv_layout: str = "nhd"):
-    """Synthetic inputs of the decode configs (BASELINE.json configs[1..3]); returns a dict."""
+    """Synthetic inputs of the decode configs; returns a dict."""
     import torch
     g = torch.Generator(device="cpu").manual_seed(seed)
     page = 256
@@ -179,7 +179,7 @@ def decode_workload(name: str, device, seed: int = 0, kv_layout: str = "nhd"):
 
 
 def mla_workload(device, seed: int = 0):
-    """BASELINE.json configs[3]: DeepSeek-V3-shaped latent decode, int8 cache with per-token fp32 scales."""
+    """DeepSeek-V3-shaped latent decode, int8 cache with per-token fp32 scales."""
     import torch
     g = torch.Generator(device="cpu").manual_seed(seed)
     B, hq, page = 32, 128, 256
@@ -409,7 +409,7 @@ def run_decode(args, name, cpu_budget=(20.0, 10.0)):
 
 
 def prefill_workload(device, seed: int = 0):
-    """16 sequences, lengths uniform in [512, 4096] rescaled to a total of
+    """Varlen prefill: 16 sequences, lengths uniform in [512, 4096] rescaled to a total of
     32768 tokens (largest remainder), 32 q heads / 8 kv heads, d = 128, bf16, causal."""
     import torch
     g = torch.Generator(device="cpu").manual_seed(seed)
@@ -497,7 +497,7 @@ def run_prefill(args, cpu_budget_s: float = 20.0):
 
 
 def run_mixed(args):
-    """Not a BASELINE.json config: a token-major serving step over a paged cache through the varlen call, 63 decode
+    """A token-major serving step over a paged cache through the varlen call, 63 decode
     rows (contexts uniform in [1024, 8191]) and one 1024-token prompt chunk at the end of a 16384-key context,
     32 q / 8 kv heads, d = 128, bf16, causal.  The decode rows are bound by HBM, the chunk by the matrix pipe: the
     line reports the time against the sum of the two roofs."""

@@ -45,7 +45,7 @@ def test_attention_after_append_equals_fresh_cache():
 
 
 def test_config1_cpu_plumbing():
-    # BASELINE config 1: B=2, 8q/2kv heads, d=128, fp32, page 256, 8 pages, lens [300, 511], append 1, causal
+    # B=2, 8q/2kv heads, d=128, fp32, page 256, 8 pages, lens [300, 511], append 1, causal
     g = torch.Generator().manual_seed(0)
     q, kc, vc = torch.randn(2, 1, 8, 128, generator=g), torch.randn(8, 256, 2, 128, generator=g), torch.randn(8, 256, 2, 128, generator=g)
     bt = torch.randperm(8, generator=g).view(2, 4).to(torch.int32)
