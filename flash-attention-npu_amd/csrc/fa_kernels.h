@@ -209,8 +209,8 @@ inline int prefill_pack(int group, int max_seqlen_q) {
 // operand reads only two k-steps ahead.  Two / three waves at D = 128 (the former with both V buffers), three / four at D = 64,
 // TFLOP/s: 4 x 8192 tokens, 32q/8kv, bidirectional 993 / 1049 (d = 64: 864 / 882); 16 x 2048 causal 800 / 894; 4 x 4096, 32q/32kv
 // 895 / 987; us: 16 x 512..4096 causal 791.6 / 718.8, 80 x 3..350, 28q/4kv 85.9 / 78.3, 8 x 2050, 16q/16kv, d = 64, fp16 205.8 /
-// 198.8.  Random values hold the clock down (1.6-1.9 GHz; all-zero inputs run the same code 1.6 times as fast), so that half of the
-// saved cycles do not show.  `spare`: kernels that keep more beside the tile loop, a head dimension below D or a list of blocks.
+// 198.8.  Random values hold the clock down (1.7-1.95 GHz against 2.4 on all-zero inputs, which take 0.65-0.7 of the time), so that a
+// cycle saved pays by less than its share.  `spare`: kernels that keep more beside the tile loop, a head dimension below D or a list of blocks.
 // (A list kernel of three waves spills nine vector registers and 40 bytes of scratch per lane, one of four at d = 64 four and 20: 63
 // decode rows + a 1024-token chunk, 32q/8kv 531 us with two waves, 596 with three; 20 rows + 2000 tokens 1137 / 1421; d = 64, three /
 // four waves 373.7 / 375.5.)
