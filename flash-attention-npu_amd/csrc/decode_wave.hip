@@ -230,7 +230,8 @@ __device__ __forceinline__ void wave_piece(const DecodeParams &p, const int b, c
     const uint32_t v_lane_off = (uint32_t)(lq * 4) * v_row_bytes + v_lane_col;
 
     // Place of a chunk: its page in the table and its first row in the page, stepped along: a division per piece where the start of
-    // a piece and every chunk took two (1 sequence of 700 keys, 8 kv heads: 9.97 -> 9.52 us; calls of more chunks are level).
+    // a piece and every chunk took two (1 sequence of 700 keys, 8 kv heads: 9.97 -> 9.52 us; calls of more chunks are level).  A page
+    // holds whole chunks, or all the keys of its row.
     struct ChunkPlace {
         int page, row;
     };
